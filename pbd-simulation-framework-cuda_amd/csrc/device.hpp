@@ -328,6 +328,9 @@ contacts_done:
   return cnt;
 }
 
+// A NaN as the positive quiet NaN (the tile lists read the sign of a distance test).
+__device__ __forceinline__ float canonical_nan(float x) { return x == x ? x : __uint_as_float(0x7FC00000u); }
+
 // ---------------------------------------------------------------------------
 // Kernel functions, unnormalised (coefficients wc / gc applied by the caller).
 //   reference (Density.h:14-42): W ~ ((h^2 - r^2)^3)^2 on 0.001 < r < h - 0.001;
@@ -336,6 +339,14 @@ contacts_done:
 // r and 1/r come from the hardware reciprocal square root (v_rsq_f32, 1 ulp):
 // the IEEE sqrt and divide sequences cost ~16 instructions per candidate.
 __device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
+// |r|^2 with the fused operations spelled out, so that a path forms it alike whatever
+// the compiler makes of the expressions around it.  Two orders are in use (XF: x first;
+// else y first): one rounding more or less decides which side of a contact's onset a
+// pair falls on, so a path keeps the order it has.
+template <bool XF = false>
+__device__ __forceinline__ float length_sq(float x, float y, float z) {
+  return XF ? fmaf(z, z, fmaf(y, y, x * x)) : fmaf(z, z, fmaf(x, x, y * y));
+}
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // Textbook terms are branch-free: max() clamps at the supports, which gives

@@ -130,7 +130,7 @@ __global__ void k_reorder(DevParams P, const uint32_t* __restrict__ keys_s, cons
   const float cx = frame_corner(P, frame_origin(P, sc, 0), compact10(key >> 2));
   const float cy = frame_corner(P, frame_origin(P, sc, 1), compact10(key >> 1));
   const float cz = frame_corner(P, frame_origin(P, sc, 2), compact10(key));
-  Q[s] = make_float4(p.x - cx, p.y - cy, p.z - cz, p.w);
+  Q[s] = make_float4(canonical_nan(p.x - cx), canonical_nan(p.y - cy), canonical_nan(p.z - cz), p.w);
   QX[s] = make_float4(x.x - cx, x.y - cy, x.z - cz, x.w);
   VS[s] = v;
   if (!(P.gates & G_FIND_NEIGHBOURS)) CS[s] = C[j];

@@ -19,9 +19,10 @@ struct LambdaAcc {
   float A = 0.0f, B = 0.0f, gx = 0.0f, gy = 0.0f, gz = 0.0f;
 };
 
-template <int VAR>
+// XF (here and below): the order in which length_sq sums
+template <int VAR, bool XF = false>
 __device__ __forceinline__ void lambda_pair(const DevParams& P, float rx, float ry, float rz, LambdaAcc& a) {
-  const float r2 = rx * rx + ry * ry + rz * rz;
+  const float r2 = length_sq<XF>(rx, ry, rz);
   a.A += w_unnorm<VAR>(P, r2);
   float hr4;
   const float g = grad_factor<VAR>(P, r2, hr4);
@@ -78,10 +79,10 @@ __device__ __forceinline__ float scorr_pow(const DevParams& P, float x) {
   return ipow(x, P.n_scorr);
 }
 
-template <int VAR, bool DELTA, bool COLLIDE, int NS = 0>
+template <int VAR, bool DELTA, bool COLLIDE, int NS = 0, bool XF = false>
 __device__ __forceinline__ void delta_pair(const DevParams& P, float li, float lj, float rx, float ry, float rz,
                                            bool contact, DeltaAcc& a) {
-  const float r2 = rx * rx + ry * ry + rz * rz;
+  const float r2 = length_sq<XF>(rx, ry, rz);
   if (VAR == PBD_KERNEL_TEXTBOOK) {
     // one 1/r for the spiky gradient and the contact push
     const float r2c = fmaxf(r2, 1.0e-30f);
@@ -184,10 +185,10 @@ struct OmegaAcc {
   float ox = 0.0f, oy = 0.0f, oz = 0.0f;
 };
 
-template <int VAR>
+template <int VAR, bool XF = false>
 __device__ __forceinline__ void omega_pair(const DevParams& P, float rx, float ry, float rz, float vx, float vy,
                                            float vz, OmegaAcc& a) {
-  const float r2 = rx * rx + ry * ry + rz * rz;
+  const float r2 = length_sq<XF>(rx, ry, rz);
   float hr4;
   const float g = grad_factor<VAR>(P, r2, hr4);
   const float gx = g * rx, gy = g * ry, gz = g * rz;
@@ -197,11 +198,11 @@ __device__ __forceinline__ void omega_pair(const DevParams& P, float rx, float r
 }
 
 // reference omega_i = sum v_ij x grad(p_i - p_j); textbook (1/rho0) sum v_ij x grad_j W_ij
-template <int VAR>
+template <int VAR, bool XF = false>
 __device__ __forceinline__ float4 omega_finish(const DevParams& P, const OmegaAcc& a) {
   const float sc = (VAR == PBD_KERNEL_TEXTBOOK) ? -P.gc * P.vol : P.gc;
   const float ox = a.ox * sc, oy = a.oy * sc, oz = a.oz * sc;
-  return make_float4(ox, oy, oz, sqrtf(ox * ox + oy * oy + oz * oz));  // w = |omega|
+  return make_float4(ox, oy, oz, sqrtf(length_sq<XF>(ox, oy, oz)));  // w = |omega|
 }
 
 // ---------------------------------------------------------------- vorticity + XSPH + output
@@ -211,11 +212,11 @@ struct FinalAcc {
 };
 
 // Textbook vorticity: eta = sum (|w_j| - |w_i|) g r (gc applied in the finish).
-template <int VAR>
+template <int VAR, bool XF = false>
 __device__ __forceinline__ void final_pair_textbook(const DevParams& P, bool vort, bool xsph, float rx, float ry,
                                                     float rz, float4 vi, float4 vj, float oil, float ojl,
                                                     FinalAcc& a) {
-  const float r2 = rx * rx + ry * ry + rz * rz;
+  const float r2 = length_sq<XF>(rx, ry, rz);
   if (xsph) {
     const float w = w_unnorm<VAR>(P, r2);
     a.sx += (vj.x - vi.x) * w;
@@ -237,7 +238,7 @@ __device__ __forceinline__ void final_pair_textbook(const DevParams& P, bool vor
 __device__ __forceinline__ void final_pair_reference(const DevParams& P, bool vort, bool xsph, float rx, float ry,
                                                      float rz, float4 vi, float4 vj, float4 oi, float4 oj,
                                                      FinalAcc& a) {
-  const float r2 = rx * rx + ry * ry + rz * rz;
+  const float r2 = length_sq(rx, ry, rz);
   if (xsph) {
     const float w = w_unnorm<PBD_KERNEL_REFERENCE>(P, r2);
     a.sx += (vj.x - vi.x) * w;
@@ -363,7 +364,7 @@ __device__ __forceinline__ float4 delta_particle(const DevParams& P, uint32_t fl
                        if (si || sj) {
                          delta_pair<VAR, false, COLLIDE>(P, 0.0f, 0.0f, rx, ry, rz, contact, a);
                          if (fric && contact) {
-                           const float r2 = rx * rx + ry * ry + rz * rz;
+                           const float r2 = length_sq(rx, ry, rz);
                            if (r2 > 0.0f) {
                              const float il = rsq(r2), len = r2 * il;
                              if (len < P.diameter && len > 0.00001f) {
@@ -400,7 +401,7 @@ __device__ __forceinline__ void omega_particle(const DevParams& P, uint32_t s, c
                      const float4 qj = Q[j], vj = VS[j];
                      omega_pair<VAR>(P, bx - qj.x, by - qj.y, bz - qj.z, vj.x - vi.x, vj.y - vi.y, vj.z - vi.z, a);
                    });
-  OM[s] = omega_finish<VAR>(P, a);
+  OM[s] = omega_finish<VAR, true>(P, a);
 }
 
 // XSPH alone for particle s, with final_particle's neighbour order, arithmetic

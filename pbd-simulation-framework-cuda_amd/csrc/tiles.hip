@@ -65,29 +65,38 @@ struct TileShared {
   uint32_t lstart[TileGeom<BITS>::NH + 1];  // LDS start of each halo cell; lstart[NH] = total
   uint32_t gstart[TileGeom<BITS>::NH];      // sorted index of the cell's first particle
   uint32_t wsum[kTileThreads / 64];
+  float off[3][6];                          // per axis: halo cell's corner minus the block's first cell's corner
   uint32_t g0, g1;                          // the block's own particle range
   uint32_t dmax;                            // largest displacement bound in the halo (float bits)
 };
+static_assert(TileGeom<6>::HX <= 6 && TileGeom<6>::HY <= 6 && TileGeom<6>::HZ <= 6, "offset table");
 
 // Steps 1 of the tile: halo cell table, LDS offsets, own range.  Returns the
 // halo particle count.  Every thread of the team takes R halo cells; all their
 // cell-table loads are issued before the scan.
 template <int BITS, class Team>
 __device__ __forceinline__ uint32_t tile_setup(const DevParams& P, uint32_t blk, const uint32_t* __restrict__ cs,
-                                               const uint32_t* __restrict__ ce, TileShared<BITS>& sh, int& ix0,
-                                               int& iy0, int& iz0) {
+                                               const uint32_t* __restrict__ ce, TileShared<BITS>& sh) {
   using G = TileGeom<BITS>;
   constexpr uint32_t R = (G::NH + Team::kSize - 1u) / Team::kSize;
   static_assert(Team::kSize == 64u || R == 1u, "a workgroup team takes one halo cell per thread");
   const uint32_t tid = Team::tid(), lane = threadIdx.x & 63u;
   const uint32_t first = blk << BITS;
-  ix0 = (int)compact10(first >> 2);
-  iy0 = (int)compact10(first >> 1);
-  iz0 = (int)compact10(first);
+  const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
   if (tid == 0) {
     sh.g0 = 0xFFFFFFFFu;
     sh.g1 = 0u;
     sh.dmax = 0u;
+  }
+  // Offsets of the halo cells' corners from the block's first cell's.  In a batched
+  // context both cells lie in the block's scene: the occupied cells of a scene keep
+  // kernelWidthNeighbours + 1 empty cells from its slot's faces, so a halo cell
+  // outside the slot is empty and its offset is never used.
+  if (tid < 18u) {
+    const uint32_t a = tid / 6u, k = tid % 6u;
+    const uint32_t i0 = a == 0u ? (uint32_t)ix0 : (a == 1u ? (uint32_t)iy0 : (uint32_t)iz0);
+    const float o = frame_origin(P, scene_of_key(P, first), (int)a);
+    sh.off[a][k] = frame_corner(P, o, i0 + k - 1u) - frame_corner(P, o, i0);
   }
   Team::sync();
   uint32_t cnt[R];
@@ -153,6 +162,16 @@ __device__ __forceinline__ uint32_t tile_setup(const DevParams& P, uint32_t blk,
   return sh.lstart[G::NH];
 }
 
+// A halo slot as one 16-byte LDS read, also where .w is not used.  Left to itself the
+// compiler drops .w and reads 12 bytes, which takes the LDS 1.6 times as long (gfx950,
+// clocks per wave read: a scan's addresses, 8 lanes each, 7.1 against 11.1; a list's,
+// one per lane, 14.3 against 23.4).
+__device__ __forceinline__ float4 slot_read(const float4* s_q, uint32_t j) {
+  float4 v = s_q[j];
+  asm("" : "+v"(v.x) : "v"(v.w));  // x is used, so w is read
+  return v;
+}
+
 // Halo cell holding LDS slot i (largest c with lstart[c] <= i).
 template <int BITS>
 __device__ __forceinline__ int tile_cell_of(const TileShared<BITS>& sh, uint32_t i) {
@@ -165,29 +184,26 @@ __device__ __forceinline__ int tile_cell_of(const TileShared<BITS>& sh, uint32_t
   return lo;
 }
 
-// Offset of halo cell c's corner from the block's first cell's corner.
-// In a batched context both cells lie in the block's scene: the occupied cells of
-// a scene keep kernelWidthNeighbours + 1 empty cells from its slot's faces, so a
-// halo cell outside the slot is empty and its offset is never used.
+// Offset of halo cell c's corner from the block's first cell's corner (c < 216:
+// c / 6 and c / 36 by a multiplication, v_mul_hi_u32 is a quarter-rate instruction).
 template <int BITS>
-__device__ __forceinline__ float3 tile_offset(const DevParams& P, int c, int ix0, int iy0, int iz0) {
+__device__ __forceinline__ float3 tile_offset(const TileShared<BITS>& sh, uint32_t c) {
   using G = TileGeom<BITS>;
-  const int hx = c / G::SX, hy = (c / G::SY) % G::HY, hz = c % G::HZ;
-  const uint32_t sc = scene_of_key(P, morton3((uint32_t)ix0, (uint32_t)iy0, (uint32_t)iz0));
-  const float ox = frame_origin(P, sc, 0), oy = frame_origin(P, sc, 1), oz = frame_origin(P, sc, 2);
-  return make_float3(frame_corner(P, ox, (uint32_t)(ix0 - 1 + hx)) - frame_corner(P, ox, (uint32_t)ix0),
-                     frame_corner(P, oy, (uint32_t)(iy0 - 1 + hy)) - frame_corner(P, oy, (uint32_t)iy0),
-                     frame_corner(P, oz, (uint32_t)(iz0 - 1 + hz)) - frame_corner(P, oz, (uint32_t)iz0));
+  static_assert(G::HY == 6 && G::HZ == 6 && G::NH <= 216, "halo cell coordinates");
+  const uint32_t xy = __umul24(c, 171u) >> 10, hx = __umul24(xy, 43u) >> 8;
+  return make_float3(sh.off[0][hx], sh.off[1][xy - 6u * hx], sh.off[2][c - 6u * xy]);
 }
 
 // Own particle g: its halo cell and LDS slot.
 template <int BITS>
-__device__ __forceinline__ void tile_locate(const TileShared<BITS>& sh, uint32_t key, uint32_t g, int ix0, int iy0,
-                                            int iz0, int& h, uint32_t& slot) {
+__device__ __forceinline__ void tile_locate(const TileShared<BITS>& sh, uint32_t key, uint32_t g, int& h,
+                                            uint32_t& slot) {
   using G = TileGeom<BITS>;
-  const int hx = (int)compact10(key >> 2) - ix0 + 1;
-  const int hy = (int)compact10(key >> 1) - iy0 + 1;
-  const int hz = (int)compact10(key) - iz0 + 1;
+  // the key's low BITS bits are the cell's coordinates in the block, z, y, x from the LSB
+  const uint32_t l = key & ((1u << BITS) - 1u);
+  const int hx = (int)(((l >> 2) & 1u) | ((l >> 4) & 2u)) + 1;
+  const int hy = (int)(((l >> 1) & 1u) | ((l >> 3) & 2u)) + 1;
+  const int hz = (int)((l & 1u) | ((l >> 2) & 2u)) + 1;
   h = hx * G::SX + hy * G::SY + hz;
   slot = sh.lstart[h] + (g - sh.gstart[h]);
 }
@@ -204,9 +220,9 @@ template <int BITS, class Body>
 __device__ __forceinline__ uint32_t tile_stencil(const TileShared<BITS>& sh, int h, uint32_t slot, Body body) {
   using G = TileGeom<BITS>;
   uint32_t total = 0;
-#pragma unroll
+#pragma unroll 1
   for (int dx = -1; dx <= 1; ++dx) {
-#pragma unroll
+#pragma unroll 1
     for (int dy = -1; dy <= 1; ++dy) {
       const int hb = h + dx * G::SX + dy * G::SY;
       // the three z cells of a (dx, dy) column are consecutive halo cells: one range
@@ -453,55 +469,108 @@ union TileLds {
   TileRegion<BITS, TileCap<BITS>::value, GI> big;
   TileRegion<BITS, TileCap<BITS>::small, GI> small[kTileThreads / 64u];
 };
-static_assert(sizeof(TileLds<5, false>) == sizeof(TileRegion<5, TileCap<5>::value, false>), "small tiles fit");
-static_assert(sizeof(TileLds<5, true>) == sizeof(TileRegion<5, TileCap<5>::value, true>), "small tiles fit");
-static_assert(sizeof(TileLds<6, false>) == sizeof(TileRegion<6, TileCap<6>::value, false>), "small tiles fit");
-static_assert(sizeof(TileLds<6, true>) == sizeof(TileRegion<6, TileCap<6>::value, true>), "small tiles fit");
+constexpr uint32_t kLdsBytes = 160u * 1024u;  // of a CU
+static_assert(5 * sizeof(TileLds<5, false>) <= kLdsBytes && 4 * sizeof(TileLds<5, true>) <= kLdsBytes,
+              "workgroups per CU of the 2^5-cell passes");
+static_assert(3 * sizeof(TileLds<6, false>) <= kLdsBytes && 2 * sizeof(TileLds<6, true>) <= kLdsBytes,
+              "workgroups per CU of the 2^6-cell passes");
 
 // Copy the block's halo into LDS (block-local coordinates; .w = payload(i)),
 // with s_gi (when not null) the global index of every slot, and place the
 // sentinel at slot CAP (s_gi[CAP] = `any`, a valid particle whose pair terms
-// the sentinel's position zeroes).  kLoadUnroll slots per thread are in flight
-// at once; the index of a slot past the end is clamped to the last slot and its
-// result dropped.  With dk, sh.dmax receives the largest dk[i] - dm[i] (dm
-// null: dk[i]) over the halo's particles i, the bound on their displacement
-// between two delta-p passes (float bits: the bounds are >= 0, or NaN, which
-// exceeds every finite bound).
+// the sentinel's position zeroes).  With dk, sh.dmax receives the largest
+// dk[i] - dm[i] (dm null: dk[i]) over the halo's particles i, the bound on their
+// displacement between two delta-p passes (float bits: the bounds are >= 0, or
+// NaN, which exceeds every finite bound).
+//
+// A workgroup team deals the halo cells to groups of 8 lanes, so a slot's cell is
+// known without a search and its offset is looked up once per 8 slots; the first
+// 16 particles of every cell of a group are in flight at once (1M dam break, delta-p:
+// 70 -> 65 us; 32K: 13.2 -> 9.9 us, with the smaller kernels of TileRest).  A wave team's
+// tile is sparse (a few particles in a cell): there a lane takes slots, kLoadUnroll
+// in flight, and finds each slot's cell by bisection (the index of a slot past the
+// end is clamped to the last slot and its result dropped).
 template <int BITS, int CAP, class Team, class Payload>
 __device__ __forceinline__ void tile_load(const DevParams& P, TileShared<BITS>& sh, uint32_t total,
-                                          const float4* __restrict__ Q, int ix0, int iy0, int iz0, float4* s_q,
-                                          uint32_t* s_gi, uint32_t any, Payload payload,
-                                          const float* __restrict__ dk = nullptr,
+                                          const float4* __restrict__ Q, float4* s_q, uint32_t* s_gi, uint32_t any,
+                                          Payload payload, const float* __restrict__ dk = nullptr,
                                           const float* __restrict__ dm = nullptr) {
-  constexpr uint32_t U = Team::kLoadUnroll;
   const uint32_t tid = Team::tid();
   uint32_t dmax = 0u;
-  for (uint32_t i0 = tid; i0 < total; i0 += U * Team::kSize) {
-    int c[U];
-    uint32_t gi[U];
-    float4 q[U];
-    float w[U], d[U];
+  const auto bound = [&](uint32_t gi) { return dk ? __float_as_uint(dk[gi] - (dm ? dm[gi] : 0.0f)) : 0u; };
+  if constexpr (Team::kSize == 64u) {
+    constexpr uint32_t U = Team::kLoadUnroll;
+    for (uint32_t i0 = tid; i0 < total; i0 += U * Team::kSize) {
+      int c[U];
+      uint32_t gi[U], d[U];
+      float4 q[U];
+      float w[U];
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-      const uint32_t i = min(i0 + u * Team::kSize, total - 1u);
-      c[u] = tile_cell_of<BITS>(sh, i);
-      gi[u] = sh.gstart[c[u]] + (i - sh.lstart[c[u]]);
-      q[u] = Q[gi[u]];
-      w[u] = payload(gi[u]);
-      d[u] = dk ? dk[gi[u]] - (dm ? dm[gi[u]] : 0.0f) : 0.0f;
+      for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t i = min(i0 + u * Team::kSize, total - 1u);
+        c[u] = tile_cell_of<BITS>(sh, i);
+        gi[u] = sh.gstart[c[u]] + (i - sh.lstart[c[u]]);
+        q[u] = Q[gi[u]];
+        w[u] = payload(gi[u]);
+        d[u] = bound(gi[u]);
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) {
+        const uint32_t i = i0 + u * Team::kSize;
+        if (i < total) {
+          const float3 o = tile_offset<BITS>(sh, (uint32_t)c[u]);
+          s_q[i] = make_float4(q[u].x + o.x, q[u].y + o.y, q[u].z + o.z, w[u]);
+          if (s_gi) s_gi[i] = gi[u];
+        }
+      }
+      // a clamped slot repeats the last one: its bound may be taken again
+#pragma unroll
+      for (uint32_t u = 0; u < U; ++u) dmax = max(dmax, d[u]);
     }
+  } else {
+    constexpr uint32_t NG = Team::kSize / 8u, NH = TileGeom<BITS>::NH, R = (NH + NG - 1u) / NG;
+    const uint32_t l8 = tid & 7u;
+    uint32_t cell[R], ls[R], n[R], gs[R];
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) {
-      const uint32_t i = i0 + u * Team::kSize;
-      if (i < total) {
-        const float3 o = tile_offset<BITS>(P, c[u], ix0, iy0, iz0);
-        s_q[i] = make_float4(q[u].x + o.x, q[u].y + o.y, q[u].z + o.z, w[u]);
-        if (s_gi) s_gi[i] = gi[u];
+    for (uint32_t r = 0; r < R; ++r) {
+      const uint32_t c = (tid >> 3) + r * NG;
+      cell[r] = min(c, NH - 1u);
+      ls[r] = sh.lstart[cell[r]];
+      n[r] = c < NH ? sh.lstart[cell[r] + 1u] - ls[r] : 0u;
+      gs[r] = sh.gstart[cell[r]];
+    }
+    float4 q[R][2];
+    float w[R][2];
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r)
+#pragma unroll
+      for (uint32_t v = 0; v < 2u; ++v) {
+        const uint32_t j = l8 + 8u * v;
+        if (j < n[r]) {
+          q[r][v] = Q[gs[r] + j];
+          w[r][v] = payload(gs[r] + j);
+          dmax = max(dmax, bound(gs[r] + j));
+        }
+      }
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+      const float3 o = tile_offset<BITS>(sh, cell[r]);
+#pragma unroll
+      for (uint32_t v = 0; v < 2u; ++v) {
+        const uint32_t j = l8 + 8u * v;
+        if (j < n[r]) {
+          s_q[ls[r] + j] = make_float4(q[r][v].x + o.x, q[r][v].y + o.y, q[r][v].z + o.z, w[r][v]);
+          if (s_gi) s_gi[ls[r] + j] = gs[r] + j;
+        }
+      }
+      for (uint32_t j = l8 + 16u; j < n[r]; j += 8u) {
+        const uint32_t gi = gs[r] + j;
+        const float4 p = Q[gi];
+        s_q[ls[r] + j] = make_float4(p.x + o.x, p.y + o.y, p.z + o.z, payload(gi));
+        if (s_gi) s_gi[ls[r] + j] = gi;
+        dmax = max(dmax, bound(gi));
       }
     }
-    // a clamped slot repeats the last one: its bound may be taken again
-#pragma unroll
-    for (uint32_t u = 0; u < U; ++u) dmax = max(dmax, __float_as_uint(d[u]));
   }
   if (dk) {
 #pragma unroll
@@ -525,6 +594,34 @@ struct Carry {
     return p ? disp + (size_t)(p - 1u) * stride : nullptr;  // after p delta-p passes (p = 0: all zero)
   }
 };
+
+// Particles of a tile left to the per-particle global-memory path: thread `tid` of the
+// team takes the particles g, g + stride, ... < end whose bit of `bits` is set (bit k:
+// the k-th of them; all: every one, for a block whose halo exceeds the tile capacity).
+// A tile pass returns them and the kernel walks them once for both teams, so that the
+// global path is in a kernel once instead of at every place that takes it (four copies
+// made up half of the 50 to 110 KB kernels).
+struct TileRest {
+  uint32_t g = 0u, end = 0u, stride = 1u, bits = 0u;
+  bool all = false;
+  template <class Body>
+  __device__ __forceinline__ void visit(Body body) const {
+    if (!all && bits == 0u) return;
+    uint32_t k = 0u;
+    for (uint32_t i = g; i < end; i += stride, ++k)
+      if (all || ((bits >> k) & 1u)) body(i);
+  }
+};
+// A tile within the capacity has at most 12 rounds (TileCap / team size).
+template <class Team>
+__device__ __forceinline__ TileRest tile_rest(uint32_t g0, uint32_t g1, bool all) {
+  TileRest r;
+  r.g = g0 + Team::tid();
+  r.end = g1;
+  r.stride = Team::kSize;
+  r.all = all;
+  return r;
+}
 
 // Whether a tile keeps the lists it built after an earlier delta-p pass (the
 // halo bound of tile_load against P.reuse_max); read after the team barrier
@@ -564,48 +661,78 @@ __device__ __forceinline__ void nl_visit(const NeighbourList& L, uint32_t g, uin
   }
 }
 
-// In-range bits of one stencil column: bit k of (lo, hi) is set when slot a + k
-// (k < b - a <= 64) is within the list radius.  Unrolled by kScanUnroll: a group
-// may read up to kScanUnroll - 1 slots past b (still inside the LDS array); their
-// bits are masked off.
-__device__ __forceinline__ void nl_column(const float4* s_q, uint32_t a, uint32_t b, float qx, float qy, float qz,
-                                          float r2max, uint32_t& lo, uint32_t& hi) {
+// In-range bits of slots a .. a + len - 1 (len <= 32): bit k is set when slot a + k
+// is within the list radius.  The test is the sign of r^2 - r2max, shifted into the
+// mask by one v_alignbit: 7 VALU instructions a candidate (compare, select, shift and
+// or take 11).  A building lambda pass is bound by VALU issue (86 % busy) and, half as
+// much, by the LDS; 1M dam break: 152 -> 122 us, with the 16-byte reads of slot_read.  Unrolled by kScanUnroll: a group may read up to kScanUnroll - 1 slots
+// past the range (still inside the LDS array); their bits are masked off.  A position
+// that is not a number is +NaN (canonical_nan), whose sign says out of range; the
+// caller drops the mask of a particle that is itself none.
+__device__ __forceinline__ uint32_t nl_mask(const float4* s_q, uint32_t a, uint32_t len, float qx, float qy, float qz,
+                                            float r2max) {
   constexpr uint32_t U = kScanUnroll;
-  lo = 0u;
-  hi = 0u;
-  for (uint32_t k = 0; a + k < b; k += U) {
+  uint32_t m = 0u, k = 0u;
+  do {
     float4 c[U];
 #pragma unroll
-    for (uint32_t u = 0; u < U; ++u) c[u] = s_q[a + k + u];
-    uint32_t g = 0u;
+    for (uint32_t u = 0; u < U; ++u) c[u] = slot_read(s_q, a + k + u);
 #pragma unroll
     for (uint32_t u = 0; u < U; ++u) {
-      const float rx = qx - c[u].x, ry = qy - c[u].y, rz = qz - c[u].z;
-      g |= (rx * rx + ry * ry + rz * rz < r2max) ? (1u << u) : 0u;
+      const float rx = c[u].x - qx, ry = c[u].y - qy, rz = c[u].z - qz;
+      const float d = fmaf(rz, rz, fmaf(ry, ry, fmaf(rx, rx, -r2max)));
+      m = __builtin_amdgcn_alignbit(m, __float_as_uint(d), 31u);  // m << 1 | sign of d
     }
-    if (k < 32u) lo |= g << k;
-    else hi |= g << (k - 32u);
-  }
-  const uint32_t len = b - a;
-  if (len < 32u) lo &= (1u << len) - 1u;
-  if (len < 64u) hi &= len <= 32u ? 0u : (1u << (len - 32u)) - 1u;
+    k += U;
+  } while (k < len);
+  // slot a + j is bit k - 1 - j now
+  return (__brev(m) >> (32u - k)) & (0xFFFFFFFFu >> (32u - len));
 }
 
 // Appends slots to 8-entry chunks held in four registers and stores each full
 // chunk to the global list (chunk-major).
 struct ChunkWriter {
-  uint32_t w0 = 0u, w1 = 0u, w2 = 0u, w3 = 0u, k = 0u, c = 0u;
-  __device__ __forceinline__ void push(const NeighbourList& L, uint32_t g, uint32_t slot) {
+  uint32_t w0 = 0u, w1 = 0u, w2 = 0u, w3 = 0u, n = 0u;
+  uint4* p;        // the particle's next chunk
+  uint32_t stride;  // chunks from one to the next
+  __device__ __forceinline__ ChunkWriter(const NeighbourList& L, uint32_t g) : p(L.nl + g), stride(L.cap) {}
+  __device__ __forceinline__ void store() {
+    *p = make_uint4(w0, w1, w2, w3);
+    p += stride;
+  }
+  __device__ __forceinline__ void push(uint32_t slot) {
     // shift the chunk down one entry; the new slot enters at the top
     w0 = __builtin_amdgcn_alignbit(w1, w0, 16u);
     w1 = __builtin_amdgcn_alignbit(w2, w1, 16u);
     w2 = __builtin_amdgcn_alignbit(w3, w2, 16u);
     w3 = __builtin_amdgcn_alignbit(slot, w3, 16u);
-    if (++k == 8u) {
-      L.nl[(size_t)c * L.cap + g] = make_uint4(w0, w1, w2, w3);
-      ++c;
-      k = 0u;
+    if ((++n & 7u) == 0u) store();
+  }
+  // Fills the last chunk up with `pad`; returns the padded length.
+  __device__ __forceinline__ uint32_t finish(uint32_t pad) {
+    const uint32_t r = (0u - n) & 7u;  // entries to add
+    if (r) {
+      const uint32_t pp = pad | (pad << 16);
+      if (r & 4u) {
+        w0 = w2;
+        w1 = w3;
+        w2 = w3 = pp;
+      }
+      if (r & 2u) {
+        w0 = w1;
+        w1 = w2;
+        w2 = w3;
+        w3 = pp;
+      }
+      if (r & 1u) {
+        w0 = __builtin_amdgcn_alignbit(w1, w0, 16u);
+        w1 = __builtin_amdgcn_alignbit(w2, w1, 16u);
+        w2 = __builtin_amdgcn_alignbit(w3, w2, 16u);
+        w3 = __builtin_amdgcn_alignbit(pp, w3, 16u);
+      }
+      store();
     }
+    return n + r;
   }
 };
 
@@ -613,51 +740,45 @@ struct ChunkWriter {
 // neighbour (the producing pass holds the solid flag in the slot's .w).
 constexpr uint32_t kNlSolid = 0x8000u;
 
-template <bool PH>
-__device__ __forceinline__ void nl_push_bits(ChunkWriter& cw, const NeighbourList& L, uint32_t g, uint32_t base,
-                                             uint32_t m, const float4* s_q) {
-  while (m) {
-    const uint32_t k = __builtin_ctz(m);
-    m &= m - 1u;
-    uint32_t e = base + k;
-    if (PH && s_q[e].w != 0.0f) e |= kNlSolid;
-    cw.push(L, g, e);
-  }
-}
-
 // Build the list of the particle at `slot` (halo cell h), the pairs within
 // sqrt(r2) in stencil-column then slot order, into the global list, padded to a
-// multiple of 8 with the sentinel slot CAP.  Each column is scanned 64 slots at
-// a time and its in-range slots are appended at once.  Returns the padded
-// length, or kNlInvalid when more than kNlMax pairs are in range (checked before
-// a segment is appended, so no more than kNlMax entries are ever written).
+// multiple of 8 with the sentinel slot CAP.  Each column is scanned 32 slots at
+// a time and its in-range slots are appended at once; the loop over the columns
+// is not unrolled (its nine copies, in both teams, made kernels of 70 to 110 KB,
+// past the instruction cache).  Returns the padded length, or kNlInvalid when more
+// than kNlMax pairs are in range (checked before a segment is appended, so no more
+// than kNlMax entries are ever written).
 template <int BITS, int CAP, bool PH>
 __device__ __forceinline__ uint32_t nl_build(const DevParams& P, const NeighbourList& L, uint32_t g,
                                              const TileShared<BITS>& sh, const float4* s_q, int h, uint32_t slot,
                                              float4 qi, float r2) {
   using G = TileGeom<BITS>;
+  const float nan = qi.x + qi.y + qi.z;
+  const uint32_t valid = nan == nan ? 0xFFFFFFFFu : 0u;
   uint32_t n = 0;
-  ChunkWriter cw;
-#pragma unroll
-  for (int c = 0; c < 9; ++c) {
-    const int hb = h + (c / 3 - 1) * G::SX + (c % 3 - 1) * G::SY;
-    const uint32_t a = sh.lstart[hb - 1], b = sh.lstart[hb + 2];
-    for (uint32_t s = a; s < b; s += 64u) {
-      uint32_t lo, hi;
-      nl_column(s_q, s, b < s + 64u ? b : s + 64u, qi.x, qi.y, qi.z, r2, lo, hi);
-      if (c == 4) {  // the own column: drop the particle itself
-        const uint32_t k = slot - s;
-        if (k < 32u) lo &= ~(1u << k);
-        else if (k < 64u) hi &= ~(1u << (k - 32u));
+  ChunkWriter cw(L, g);
+#pragma unroll 1
+  for (int dx = -1; dx <= 1; ++dx) {
+#pragma unroll 1
+    for (int dy = -1; dy <= 1; ++dy) {
+      const int hb = h + dx * G::SX + dy * G::SY;
+      const uint32_t a = sh.lstart[hb - 1], b = sh.lstart[hb + 2];
+      for (uint32_t s = a; s < b; s += 32u) {
+        uint32_t m = nl_mask(s_q, s, min(b - s, 32u), qi.x, qi.y, qi.z, r2) & valid;
+        if (slot - s < 32u) m &= ~(1u << (slot - s));  // not the particle itself
+        n += __builtin_popcount(m);
+        if (n > kNlMax) return kNlInvalid;
+        while (m) {
+          const uint32_t k = __builtin_ctz(m);
+          m &= m - 1u;
+          uint32_t e = s + k;
+          if (PH && s_q[e].w != 0.0f) e |= kNlSolid;
+          cw.push(e);
+        }
       }
-      n += __builtin_popcount(lo) + __builtin_popcount(hi);
-      if (n > kNlMax) return kNlInvalid;
-      nl_push_bits<PH>(cw, L, g, s, lo, s_q);
-      nl_push_bits<PH>(cw, L, g, s + 32u, hi, s_q);
     }
   }
-  while (cw.k != 0u) cw.push(L, g, (uint32_t)CAP);
-  return cw.c * 8u;
+  return cw.finish((uint32_t)CAP);
 }
 
 // lambda over one tile (team: workgroup or wave, CAP: its LDS capacity),
@@ -666,7 +787,7 @@ __device__ __forceinline__ uint32_t nl_build(const DevParams& P, const Neighbour
 // tile built after an earlier delta-p pass when its halo has moved less than
 // P.reuse_max since.  A carrying tile builds with the skin (P.tile_r2).
 template <int BITS, bool FIRST, bool PH, class Team, int CAP>
-__device__ __forceinline__ void lambda_tile(const DevParams& P, uint32_t blk, const NeighbourList& L,
+__device__ __forceinline__ TileRest lambda_tile(const DevParams& P, uint32_t blk, const NeighbourList& L,
                                             const float4* __restrict__ Q, const uint32_t* __restrict__ keys,
                                             const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
                                             float* __restrict__ lam, float* __restrict__ dens,
@@ -674,16 +795,13 @@ __device__ __forceinline__ void lambda_tile(const DevParams& P, uint32_t blk, co
                                             const Carry& C, TileShared<BITS>& sh, float4* s_q) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
+  TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
-    for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
-      lambda_particle<VAR, FIRST>(P, g, Q, keys, cs, ce, lam, dens, ncnt, ccnt);
-      L.cnt[g] = kNlInvalid;
-    }
+    for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) L.cnt[g] = kNlInvalid;
     if (tid == 0) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_BLOCK], (unsigned long long)(g1 - g0));
-    return;
+    return rest;
   }
   // the first pass: whether the tile carries its lists this substep; a later
   // one: the delta-p passes before the tile's lists were built (kNoCarry: none)
@@ -691,7 +809,7 @@ __device__ __forceinline__ void lambda_tile(const DevParams& P, uint32_t blk, co
   const bool carry = !FIRST && m != kNoCarry;
   const float r2 = m != kNoCarry ? P.tile_r2 : P.list_r2;
   // .w: 1 for a solid particle (PH), else 0
-  tile_load<BITS, CAP, Team>(P, sh, total, Q, ix0, iy0, iz0, s_q, nullptr, 0u,
+  tile_load<BITS, CAP, Team>(P, sh, total, Q, s_q, nullptr, 0u,
                              [&](uint32_t gi) { return PH && P.phs[gi] ? 1.0f : 0.0f; },
                              carry ? C.bounds(C.pass) : nullptr, carry ? C.bounds(m) : nullptr);
   Team::sync();
@@ -702,23 +820,24 @@ __device__ __forceinline__ void lambda_tile(const DevParams& P, uint32_t blk, co
     if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                          (unsigned long long)(g1 - g0));
   }
-  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
+  uint32_t round = 0u;
+  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+    tile_locate<BITS>(sh, keys[g], g, h, slot);
     uint32_t cnt = 0u, n = kNlInvalid;
     if (keep) {
       // a kept list, or none: a particle over the cap takes the global path as
       // when the list was built, one with a long list scans the stencil
       n = L.cnt[g];
       if (n == kNlInvalid && tile_count<BITS>(sh, h) > P.cap) {
-        lambda_particle<VAR, FIRST>(P, g, Q, keys, cs, ce, lam, dens, ncnt, ccnt);
+        rest.bits |= 1u << round;
         continue;
       }
     } else {
       cnt = tile_count<BITS>(sh, h);
       if (cnt > P.cap) {
-        lambda_particle<VAR, FIRST>(P, g, Q, keys, cs, ce, lam, dens, ncnt, ccnt);
+        rest.bits |= 1u << round;
         L.cnt[g] = kNlInvalid;
         atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_CAP], 1ull);
         continue;
@@ -728,9 +847,9 @@ __device__ __forceinline__ void lambda_tile(const DevParams& P, uint32_t blk, co
     LambdaAcc a;
     const auto pair = [&](uint32_t j) __attribute__((always_inline)) {
       if (PH && (j & kNlSolid)) return;  // a fluid particle counts fluid neighbours only
-      const float4 qj = s_q[j];
+      const float4 qj = slot_read(s_q, j);
       if (PH && qj.w != 0.0f) return;
-      lambda_pair<VAR>(P, qi.x - qj.x, qi.y - qj.y, qi.z - qj.z, a);
+      lambda_pair<VAR, PH>(P, qi.x - qj.x, qi.y - qj.y, qi.z - qj.z, a);
     };
     if (!keep) {
       n = nl_build<BITS, CAP, PH>(P, L, g, sh, s_q, h, slot, qi, r2);
@@ -754,6 +873,7 @@ __device__ __forceinline__ void lambda_tile(const DevParams& P, uint32_t blk, co
       ccnt[g] = cnt;
     }
   }
+  return rest;
 }
 
 template <int BITS, bool FIRST, bool STRIDE, bool PH>
@@ -773,17 +893,20 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_lambda(DevParams P, TileL
     uint32_t blk;
     const int mode = tile_pick(T, it, r, blk);
     if (mode == 0) break;
+    TileRest rest;
     if (mode == 1) {
-      lambda_tile<BITS, FIRST, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, Q, keys, cs, ce, lam, dens, ncnt, ccnt,
-                                                                C, lds.big.sh, lds.big.q);
-      if (!STRIDE) break;
-      __syncthreads();  // the next rank may be small tiles in the same LDS bytes
+      rest = lambda_tile<BITS, FIRST, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
+                                                                       ccnt, C, lds.big.sh, lds.big.q);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      lambda_tile<BITS, FIRST, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, Q, keys, cs, ce, lam, dens, ncnt, ccnt, C,
-                                                               reg.sh, reg.q);
-      if (!STRIDE) break;
+      rest = lambda_tile<BITS, FIRST, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
+                                                                      ccnt, C, reg.sh, reg.q);
     }
+    rest.visit([&](uint32_t g) __attribute__((always_inline)) {
+      lambda_particle<PBD_KERNEL_TEXTBOOK, FIRST>(P, g, Q, keys, cs, ce, lam, dens, ncnt, ccnt);
+    });
+    if (!STRIDE) break;
+    if (mode == 1) __syncthreads();  // the next rank may be small tiles in the same LDS bytes
   }
 }
 
@@ -791,7 +914,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_lambda(DevParams P, TileL
 // lists (use_list) or a scan of the stencil; with a carry, each particle's
 // displacement bound after the pass is recorded.
 template <int BITS, bool COLLIDE, int NS, bool PH, class Team, int CAP>
-__device__ __forceinline__ void delta_tile(const DevParams& P, uint32_t blk, const NeighbourList& L, int use_list,
+__device__ __forceinline__ TileRest delta_tile(const DevParams& P, uint32_t blk, const NeighbourList& L, int use_list,
                                            uint32_t flags, const float4* __restrict__ Q,
                                            const float4* __restrict__ QX, const float* __restrict__ lam,
                                            const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cs,
@@ -801,31 +924,25 @@ __device__ __forceinline__ void delta_tile(const DevParams& P, uint32_t blk, con
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
-  if (total > (uint32_t)CAP) {
-    for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
-      const float4 q0 = Q[g];
-      track_move(C, g, q0, delta_particle<VAR, true, COLLIDE>(P, flags, g, Q, QX, lam, keys, cs, ce, Qo, QXo, DP, VS));
-    }
-    return;
-  }
+  TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
+  if (total > (uint32_t)CAP) return rest;
   // s_gi (friction-capable passes): the global index of every slot, for the
   // displacements of a solid contact's partner
-  tile_load<BITS, CAP, Team>(P, sh, total, Q, ix0, iy0, iz0, s_q, s_gi, g0, [&](uint32_t gi) { return lam[gi]; });
+  tile_load<BITS, CAP, Team>(P, sh, total, Q, s_q, s_gi, g0, [&](uint32_t gi) { return lam[gi]; });
   Team::sync();
-  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
+  uint32_t round = 0u;
+  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
     const uint32_t key = keys[g];
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, key, g, ix0, iy0, iz0, h, slot);
+    tile_locate<BITS>(sh, key, g, h, slot);
     const uint32_t n = use_list ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
     // with phases, a particle without a list takes the global path (the tile holds
     // no phases for a scan)
     if (n == kNlInvalid && (PH || tile_count<BITS>(sh, h) > P.cap)) {
-      const float4 q0 = Q[g];
-      track_move(C, g, q0, delta_particle<VAR, true, COLLIDE>(P, flags, g, Q, QX, lam, keys, cs, ce, Qo, QXo, DP, VS));
+      rest.bits |= 1u << round;
       continue;
     }
     const float4 qb = s_q[slot];
@@ -846,9 +963,9 @@ __device__ __forceinline__ void delta_tile(const DevParams& P, uint32_t blk, con
       const float4 qj = s_q[j];
       const float rx = qb.x - qj.x, ry = qb.y - qj.y, rz = qb.z - qj.z;
       if (PH && (si || (e & kNlSolid))) {
-        delta_pair<VAR, false, COLLIDE, NS>(P, 0.0f, 0.0f, rx, ry, rz, true, a);
+        delta_pair<VAR, false, COLLIDE, NS, PH && !COLLIDE>(P, 0.0f, 0.0f, rx, ry, rz, true, a);
         if (fric) {
-          const float r2 = rx * rx + ry * ry + rz * rz;
+          const float r2 = length_sq(rx, ry, rz);
           if (r2 > 0.0f) {
             const float il = rsq(r2), len = r2 * il;
             if (len < P.diameter && len > 0.00001f) {
@@ -859,7 +976,7 @@ __device__ __forceinline__ void delta_tile(const DevParams& P, uint32_t blk, con
           }
         }
       } else {
-        delta_pair<VAR, true, COLLIDE, NS>(P, qb.w, qj.w, rx, ry, rz, true, a);
+        delta_pair<VAR, true, COLLIDE, NS, PH && !COLLIDE>(P, qb.w, qj.w, rx, ry, rz, true, a);
       }
     };
     if (n != kNlInvalid) nl_visit(L, g, n, pair);
@@ -871,6 +988,7 @@ __device__ __forceinline__ void delta_tile(const DevParams& P, uint32_t blk, con
     const float4 q0 = Q[g];
     track_move(C, g, q0, delta_finish<VAR, true>(P, flags, g, q0, QX, a, cx, cy, cz, key, Qo, QXo, DP, VS));
   }
+  return rest;
 }
 
 template <int BITS, bool COLLIDE, int NS, bool STRIDE, bool PH>
@@ -894,19 +1012,24 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_delta(DevParams P, TileLi
     uint32_t blk;
     const int mode = tile_pick(T, it, r, blk);
     if (mode == 0) break;
+    TileRest rest;
     if (mode == 1) {
-      delta_tile<BITS, COLLIDE, NS, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, use_list, flags, Q, QX, lam, keys, cs,
-                                                                     ce, Qo, QXo, DP, VS, C, lds.big.sh, lds.big.q,
-                                                                     GI ? lds.big.gi : nullptr);
-      if (!STRIDE) break;
-      __syncthreads();  // the next rank may be small tiles in the same LDS bytes
+      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamBlock, TileCap<BITS>::value>(
+          P, blk, L, use_list, flags, Q, QX, lam, keys, cs, ce, Qo, QXo, DP, VS, C, lds.big.sh, lds.big.q,
+          GI ? lds.big.gi : nullptr);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      delta_tile<BITS, COLLIDE, NS, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, use_list, flags, Q, QX, lam, keys, cs,
-                                                                    ce, Qo, QXo, DP, VS, C, reg.sh, reg.q,
-                                                                    GI ? reg.gi : nullptr);
-      if (!STRIDE) break;
+      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, use_list, flags, Q, QX, lam,
+                                                                           keys, cs, ce, Qo, QXo, DP, VS, C, reg.sh,
+                                                                           reg.q, GI ? reg.gi : nullptr);
     }
+    rest.visit([&](uint32_t g) __attribute__((always_inline)) {
+      const float4 q0 = Q[g];
+      track_move(C, g, q0, delta_particle<PBD_KERNEL_TEXTBOOK, true, COLLIDE>(P, flags, g, Q, QX, lam, keys, cs, ce,
+                                                                            Qo, QXo, DP, VS));
+    });
+    if (!STRIDE) break;
+    if (mode == 1) __syncthreads();  // the next rank may be small tiles in the same LDS bytes
   }
 }
 
@@ -919,7 +1042,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_delta(DevParams P, TileLi
 // in the next substep: when its halo has moved less than P.reuse_max since its
 // lists were built, or, for a tile that did not carry, over the whole substep.
 template <int BITS, bool XSPH, bool PH, class Team, int CAP>
-__device__ __forceinline__ void omega_tile(const DevParams& P, uint32_t blk, const NeighbourList& L,
+__device__ __forceinline__ TileRest omega_tile(const DevParams& P, uint32_t blk, const NeighbourList& L,
                                            const float4* __restrict__ Q, const float4* __restrict__ VS,
                                            const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cs,
                                            const uint32_t* __restrict__ ce, float4* __restrict__ OM,
@@ -927,23 +1050,19 @@ __device__ __forceinline__ void omega_tile(const DevParams& P, uint32_t blk, con
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
+  TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
-    for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
-      omega_particle<VAR>(P, g, Q, VS, keys, cs, ce, OM);
-      if (XSPH) Vo[g] = xsph_particle<VAR>(P, g, Q, VS, keys, cs, ce);
-      L.cnt[g] = kNlInvalid;
-    }
+    for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) L.cnt[g] = kNlInvalid;
     if (tid == 0) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_BLOCK], (unsigned long long)(g1 - g0));
-    return;
+    return rest;
   }
   // global index of each slot: velocities are gathered from L2
   // .w: 1 for a solid particle (PH), else 0
   const uint32_t m = C.disp ? C.built[blk] : kNoCarry;
   const bool carry = m != kNoCarry;
-  tile_load<BITS, CAP, Team>(P, sh, total, Q, ix0, iy0, iz0, s_q, s_gi, g0,
+  tile_load<BITS, CAP, Team>(P, sh, total, Q, s_q, s_gi, g0,
                              [&](uint32_t gi) { return PH && P.phs[gi] ? 1.0f : 0.0f; },
                              C.disp ? C.bounds(C.pass) : nullptr, carry ? C.bounds(m) : nullptr);
   Team::sync();
@@ -954,16 +1073,16 @@ __device__ __forceinline__ void omega_tile(const DevParams& P, uint32_t blk, con
     if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                          (unsigned long long)(g1 - g0));
   }
-  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
+  uint32_t round = 0u;
+  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+    tile_locate<BITS>(sh, keys[g], g, h, slot);
     // kept lists: a particle without one is over the cap (global path, as when
     // the list was built) or has a long list (stencil scan)
     uint32_t n = keep ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
     if ((!keep || n == kNlInvalid) && tile_count<BITS>(sh, h) > P.cap) {
-      omega_particle<VAR>(P, g, Q, VS, keys, cs, ce, OM);
-      if (XSPH) Vo[g] = xsph_particle<VAR>(P, g, Q, VS, keys, cs, ce);
+      rest.bits |= 1u << round;
       if (!keep) {
         L.cnt[g] = kNlInvalid;
         atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_CAP], 1ull);
@@ -991,12 +1110,12 @@ __device__ __forceinline__ void omega_tile(const DevParams& P, uint32_t blk, con
     }
     const auto pair = [&](uint32_t j) __attribute__((always_inline)) {
       if (PH && (si || (j & kNlSolid))) return;  // fluid neighbours only
-      const float4 qj = s_q[j];
+      const float4 qj = slot_read(s_q, j);
       if (PH && qj.w != 0.0f) return;
       const float4 vj = VS[s_gi[j]];
       const float rx = qi.x - qj.x, ry = qi.y - qj.y, rz = qi.z - qj.z;
-      omega_pair<VAR>(P, rx, ry, rz, vj.x - vx, vj.y - vy, vj.z - vz, a);
-      if (XSPH) final_pair_textbook<VAR>(P, false, true, rx, ry, rz, make_float4(vx, vy, vz, vw), vj, 0.0f, 0.0f, xa);
+      omega_pair<VAR, PH>(P, rx, ry, rz, vj.x - vx, vj.y - vy, vj.z - vz, a);
+      if (XSPH) final_pair_textbook<VAR, PH>(P, false, true, rx, ry, rz, make_float4(vx, vy, vz, vw), vj, 0.0f, 0.0f, xa);
     };
     if (!keep) {
       n = nl_build<BITS, CAP, PH>(P, L, g, sh, s_q, h, slot, qi, P.list_r2);
@@ -1011,11 +1130,9 @@ __device__ __forceinline__ void omega_tile(const DevParams& P, uint32_t blk, con
       Vo[g] = make_float4(vx + c * xa.sx, vy + c * xa.sy, vz + c * xa.sz, vw + c * xa.sw);
     }
   }
+  return rest;
 }
 
-// XSPH: the same neighbour walk also applies XSPH (computeViscosity,
-// Density.h:280-310) and writes the velocities to Vo, in the order and with
-// the arithmetic of the final pass, which then leaves them alone.
 template <int BITS, bool XSPH, bool STRIDE, bool PH>
 __global__ __launch_bounds__(kTileThreads) void k_tile_omega(DevParams P, TileList T, NeighbourList L,
                                                              const float4* __restrict__ Q,
@@ -1033,22 +1150,26 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_omega(DevParams P, TileLi
     uint32_t blk;
     const int mode = tile_pick(T, it, r, blk);
     if (mode == 0) break;
+    TileRest rest;
     if (mode == 1) {
-      omega_tile<BITS, XSPH, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
-                                                              lds.big.sh, lds.big.q, lds.big.gi);
-      if (!STRIDE) break;
-      __syncthreads();  // the next rank may be small tiles in the same LDS bytes
+      rest = omega_tile<BITS, XSPH, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
+                                                                     lds.big.sh, lds.big.q, lds.big.gi);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      omega_tile<BITS, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, Q, VS, keys, cs, ce, OM, Vo, C, reg.sh,
-                                                             reg.q, reg.gi);
-      if (!STRIDE) break;
+      rest = omega_tile<BITS, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
+                                                                    reg.sh, reg.q, reg.gi);
     }
+    rest.visit([&](uint32_t g) __attribute__((always_inline)) {
+      omega_particle<PBD_KERNEL_TEXTBOOK>(P, g, Q, VS, keys, cs, ce, OM);
+      if (XSPH) Vo[g] = xsph_particle<PBD_KERNEL_TEXTBOOK>(P, g, Q, VS, keys, cs, ce);
+    });
+    if (!STRIDE) break;
+    if (mode == 1) __syncthreads();  // the next rank may be small tiles in the same LDS bytes
   }
 }
 
 template <int BITS, bool VORT, bool XSPH, bool PH, class Team, int CAP>
-__device__ __forceinline__ void final_tile(const DevParams& P, uint32_t blk, const NeighbourList& L, int use_list,
+__device__ __forceinline__ TileRest final_tile(const DevParams& P, uint32_t blk, const NeighbourList& L, int use_list,
                                            uint32_t flags, const float4* __restrict__ Q,
                                            const float4* __restrict__ QX, const float4* __restrict__ VS,
                                            const float4* __restrict__ OM, const uint32_t* __restrict__ keys,
@@ -1059,32 +1180,30 @@ __device__ __forceinline__ void final_tile(const DevParams& P, uint32_t blk, con
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   constexpr bool vort = VORT, xsph = XSPH;  // flags & FF_VORT, flags & FF_XSPH
+  TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
-    for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
-      if (PH) P.ph[g] = P.phs[g];  // phases follow the particles into the sorted order
-      final_particle<VAR>(P, flags, g, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo);
-    }
-    return;
+    for (uint32_t g = g0 + tid; PH && g < g1; g += Team::kSize) P.ph[g] = P.phs[g];  // as below
+    return rest;
   }
   // global index of each slot (XSPH only), for the velocity gathers from L2
   const auto omega_len = [&](uint32_t gi) { return vort ? OM[gi].w : 0.0f; };
-  tile_load<BITS, CAP, Team>(P, sh, total, Q, ix0, iy0, iz0, s_q, XSPH ? s_gi : nullptr, g0, omega_len);
+  tile_load<BITS, CAP, Team>(P, sh, total, Q, s_q, XSPH ? s_gi : nullptr, g0, omega_len);
   Team::sync();
-  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) {
+  uint32_t round = 0u;
+  for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
     if (PH) P.ph[g] = P.phs[g];  // phases follow the particles into the sorted order
     const uint32_t key = keys[g];
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, key, g, ix0, iy0, iz0, h, slot);
+    tile_locate<BITS>(sh, key, g, h, slot);
     const uint32_t n = use_list ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
     // with phases, a particle without a list takes the global path (the tile holds
     // no phases for a scan)
     if (n == kNlInvalid && (PH || tile_count<BITS>(sh, h) > P.cap)) {
-      final_particle<VAR>(P, flags, g, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo);
+      rest.bits |= 1u << round;
       continue;
     }
     const bool si = PH && P.phs[g] != 0u;  // a solid particle: no vorticity force, no XSPH
@@ -1098,7 +1217,7 @@ __device__ __forceinline__ void final_tile(const DevParams& P, uint32_t blk, con
     if (vort || xsph) {
       const auto pair = [&](uint32_t j) __attribute__((always_inline)) {
         if (PH && (si || (j & kNlSolid))) return;  // fluid neighbours only
-        const float4 qj = s_q[j];
+        const float4 qj = slot_read(s_q, j);
         const float4 vj = XSPH ? VS[s_gi[j]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // unused without XSPH
         final_pair_textbook<VAR>(P, vort, xsph, qb.x - qj.x, qb.y - qj.y, qb.z - qj.z, make_float4(vx, vy, vz, vw),
                                  vj, oi.w, qj.w, a);
@@ -1113,6 +1232,7 @@ __device__ __forceinline__ void final_tile(const DevParams& P, uint32_t blk, con
     final_finish<VAR>(P, flags, g, Q[g], make_float4(vx, vy, vz, vw), oi, a, cx, cy, cz, QX, CS, ncnt, Xo, Po, Vo,
                       Co, Fo);
   }
+  return rest;
 }
 
 template <int BITS, bool VORT, bool XSPH, bool STRIDE, bool PH>
@@ -1130,18 +1250,22 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_final(
     uint32_t blk;
     const int mode = tile_pick(T, it, r, blk);
     if (mode == 0) break;
+    TileRest rest;
     if (mode == 1) {
-      final_tile<BITS, VORT, XSPH, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, use_list, flags, Q, QX, VS, OM, keys, cs,
-                                                                    ce, CS, ncnt, Xo, Po, Vo, Co, Fo, lds.big.sh,
-                                                                    lds.big.q, lds.big.gi);
-      if (!STRIDE) break;
-      __syncthreads();  // the next rank may be small tiles in the same LDS bytes
+      rest = final_tile<BITS, VORT, XSPH, PH, TeamBlock, TileCap<BITS>::value>(
+          P, blk, L, use_list, flags, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo, lds.big.sh, lds.big.q,
+          lds.big.gi);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      final_tile<BITS, VORT, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, use_list, flags, Q, QX, VS, OM, keys, cs,
-                                                                   ce, CS, ncnt, Xo, Po, Vo, Co, Fo, reg.sh, reg.q, reg.gi);
-      if (!STRIDE) break;
+      rest = final_tile<BITS, VORT, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, use_list, flags, Q, QX, VS, OM,
+                                                                          keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo,
+                                                                          reg.sh, reg.q, reg.gi);
     }
+    rest.visit([&](uint32_t g) __attribute__((always_inline)) {
+      final_particle<PBD_KERNEL_TEXTBOOK>(P, flags, g, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo);
+    });
+    if (!STRIDE) break;
+    if (mode == 1) __syncthreads();  // the next rank may be small tiles in the same LDS bytes
   }
 }
 
@@ -1339,6 +1463,16 @@ __device__ __forceinline__ void tally_flush(const uint32_t* t, unsigned long lon
     atomicAdd(stats + kCounter[threadIdx.x], (unsigned long long)t[threadIdx.x]);
 }
 
+// In-range bits (lo, hi) of slots a .. b - 1 (1 <= b - a <= 64).
+__device__ __forceinline__ void nl_column(const float4* s_q, uint32_t a, uint32_t b, float4 q, float r2max,
+                                          uint32_t& lo, uint32_t& hi) {
+  const float nan = q.x + q.y + q.z;
+  const uint32_t valid = nan == nan ? 0xFFFFFFFFu : 0u;
+  const uint32_t len = b - a;
+  lo = nl_mask(s_q, a, min(len, 32u), q.x, q.y, q.z, r2max) & valid;
+  hi = len > 32u ? nl_mask(s_q, a + 32u, len - 32u, q.x, q.y, q.z, r2max) & valid : 0u;
+}
+
 // One particle's list: entries dealt to its lanes in turn, the last kAdjLanes
 // of them in a shift window w[0..7]; each full row (entries 8k .. 8k+7, one per
 // lane) is written as 32 bytes, and rows past kAdjListMax are dropped (the
@@ -1407,7 +1541,7 @@ __device__ __forceinline__ uint32_t adjlist_particle(const DevParams& P, const T
       const uint32_t oc = (uint32_t)((dx + 1) * 9 + (dy + 1) * 3);
       for (uint32_t s0 = a0; s0 < e; s0 += 64u) {
         uint32_t lo, hi;
-        nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb.x, qb.y, qb.z, P.list_r2, lo, hi);
+        nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb, P.list_r2, lo, hi);
         const uint32_t k = slot - s0;  // the particle itself (when in this segment)
         if (k < 32u) lo &= ~(1u << k);
         else if (k < 64u) hi &= ~(1u << (k - 32u));
@@ -1438,8 +1572,7 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
   constexpr uint32_t kMax = kAdjLanes * kAdjListMax;
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, TeamBlock>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, TeamBlock>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     // whole particles per pass of the loop: a particle's lanes are active together
@@ -1448,13 +1581,13 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
       adj_list_lane(P, Q, keys, cs, ce, L, flag, stats, g0 + u / kAdjLanes, u % kAdjLanes);
     return;
   }
-  tile_load<BITS, CAP, TeamBlock>(P, sh, total, Q, ix0, iy0, iz0, s_q, nullptr, 0u, adj_solid_payload(P));
+  tile_load<BITS, CAP, TeamBlock>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
   __syncthreads();
   const uint32_t n = P.n;
   for (uint32_t g = g0 + threadIdx.x; g < g1; g += kTileThreads) {
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+    tile_locate<BITS>(sh, keys[g], g, h, slot);
     const float4 qb = s_q[slot];
     // the last kAdjLanes entries in a shift window w[0..7]; each full row of
     // the list (entries 8k .. 8k+7, one per lane) is written as 32 bytes
@@ -1488,7 +1621,7 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
         const uint32_t oc = (uint32_t)((dx + 1) * 9 + (dy + 1) * 3);
         for (uint32_t s0 = a0; s0 < e; s0 += 64u) {
           uint32_t lo, hi;
-          nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb.x, qb.y, qb.z, P.list_r2, lo, hi);
+          nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb, P.list_r2, lo, hi);
           const uint32_t k = slot - s0;  // the particle itself (when in this segment)
           if (k < 32u) lo &= ~(1u << k);
           else if (k < 64u) hi &= ~(1u << (k - 32u));
@@ -1554,8 +1687,7 @@ __device__ __forceinline__ void adjlist_forward_tile(const DevParams& P, uint32_
                                                      uint32_t* __restrict__ redo, TileShared<BITS>& sh) {
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, TeamBlock>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, TeamBlock>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     if (threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
@@ -1570,7 +1702,7 @@ __device__ __forceinline__ void adjlist_forward_tile(const DevParams& P, uint32_
     }
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+    tile_locate<BITS>(sh, keys[g], g, h, slot);
     AdjRows R(L, P.n, g);
     if (fn > AdjRows::kMax) {
       R.c = AdjRows::kMax + 1u;  // more candidates than the lanes hold: scan
@@ -1640,8 +1772,7 @@ __device__ __forceinline__ void adjlist_forward_tile_wide(const DevParams& P, ui
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
   static_assert(kNlRecordChunks == kAdjLanes && kAdjListMax == kAdjLanes, "a forward chunk is a row of the lanes");
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, TeamWide>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, TeamWide>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     if (threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
@@ -1663,7 +1794,7 @@ __device__ __forceinline__ void adjlist_forward_tile_wide(const DevParams& P, ui
     int h = 0;
     if (fn <= AdjRows::kMax && k < nc) {
       uint32_t slot;
-      tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+      tile_locate<BITS>(sh, keys[g], g, h, slot);
       const uint4 v = F.nl[(size_t)k * F.cap + g];
       const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
       int col = -1;
@@ -1712,7 +1843,7 @@ __device__ __forceinline__ void adjlist_forward_tile_wide(const DevParams& P, ui
       cdst[1] = make_uint4(cl[4], cl[5], cl[6], cl[7]);
       if (fn > AdjRows::kMax || nc == 0u) {
         uint32_t slot;
-        tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+        tile_locate<BITS>(sh, keys[g], g, h, slot);
       }
       if (tile_count<BITS>(sh, h) >= P.cap) flag[0] = 1u;
     }
@@ -1743,21 +1874,20 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_adjlist_redo(DevParams P,
     __syncthreads();  // the previous block's halo is done with (and the tallies are cleared)
     TileShared<BITS>& sh = lds.big.sh;
     float4* s_q = lds.big.q;
-    int ix0, iy0, iz0;
-    const uint32_t total = tile_setup<BITS, TeamBlock>(P, redo[1u + i], cs, ce, sh, ix0, iy0, iz0);
+    const uint32_t total = tile_setup<BITS, TeamBlock>(P, redo[1u + i], cs, ce, sh);
     if (total > (uint32_t)CAP) {
       const uint32_t m = (sh.g1 - sh.g0) * kAdjLanes;
       for (uint32_t u = threadIdx.x; u < m; u += kTileThreads)
         adj_list_lane(P, Q, keys, cs, ce, L, flag, stats, sh.g0 + u / kAdjLanes, u % kAdjLanes);
       continue;
     }
-    tile_load<BITS, CAP, TeamBlock>(P, sh, total, Q, ix0, iy0, iz0, s_q, nullptr, 0u, adj_solid_payload(P));
+    tile_load<BITS, CAP, TeamBlock>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
     __syncthreads();
     for (uint32_t g = sh.g0 + threadIdx.x; g < sh.g1; g += kTileThreads) {
       if (F.cnt[g] != kNlInvalid) continue;
       int h;
       uint32_t slot;
-      tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+      tile_locate<BITS>(sh, keys[g], g, h, slot);
       const uint32_t c = adjlist_particle<BITS>(P, sh, s_q, L, g, h, slot);
       if (tile_count<BITS>(sh, h) >= P.cap) flag[0] = 1u;
       wave_tally(s_tally + 0, c <= AdjRows::kMax);
@@ -1787,8 +1917,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
   constexpr uint32_t kMax = kAdjLanes * kAdjListMax;
-  int ix0, iy0, iz0;
-  const uint32_t total = tile_setup<BITS, TeamWide>(P, blk, cs, ce, sh, ix0, iy0, iz0);
+  const uint32_t total = tile_setup<BITS, TeamWide>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     const uint32_t m = (g1 - g0) * kAdjLanes;
@@ -1796,7 +1925,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
       adj_list_lane(P, Q, keys, cs, ce, L, flag, stats, g0 + u / kAdjLanes, u % kAdjLanes);
     return;
   }
-  tile_load<BITS, CAP, TeamWide>(P, sh, total, Q, ix0, iy0, iz0, s_q, nullptr, 0u, adj_solid_payload(P));
+  tile_load<BITS, CAP, TeamWide>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
   __syncthreads();
   const uint32_t n = P.n;
   const uint32_t part = threadIdx.x / kTileThreads, pl = threadIdx.x % kTileThreads;
@@ -1810,7 +1939,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
     float4 qb = make_float4(0.f, 0.f, 0.f, 0.f);
     uint32_t lo[3] = {0u, 0u, 0u}, hi[3] = {0u, 0u, 0u}, cnt = 0;
     if (valid) {
-      tile_locate<BITS>(sh, keys[g], g, ix0, iy0, iz0, h, slot);
+      tile_locate<BITS>(sh, keys[g], g, h, slot);
       qb = s_q[slot];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
@@ -1820,7 +1949,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
         const uint32_t a0 = sh.lstart[hb - 1], e = sh.lstart[hb + 2];
         for (uint32_t s0 = a0; s0 < e; s0 += 64u) {
           uint32_t l, u;
-          nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb.x, qb.y, qb.z, P.list_r2, l, u);
+          nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb, P.list_r2, l, u);
           const uint32_t d = slot - s0;  // the particle itself (when in this segment)
           if (d < 32u) l &= ~(1u << d);
           else if (d < 64u) u &= ~(1u << (d - 32u));
@@ -1859,7 +1988,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
         for (uint32_t s0 = a0; s0 < e; s0 += 64u) {
           uint32_t l = lo[k], u = hi[k];
           if (s0 != a0) {  // a column of more than 64 slots: its later segments again
-            nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb.x, qb.y, qb.z, P.list_r2, l, u);
+            nl_column(s_q, s0, e < s0 + 64u ? e : s0 + 64u, qb, P.list_r2, l, u);
             const uint32_t d = slot - s0;
             if (d < 32u) l &= ~(1u << d);
             else if (d < 64u) u &= ~(1u << (d - 32u));
