@@ -377,6 +377,7 @@ hipError_t launch_reorder(hipStream_t st, uint32_t tpb, const DevParams& P, cons
 
 hipError_t launch_lambda(hipStream_t st, uint32_t tpb, const DevParams& P, const StepBuffers& B, const float4* Q,
                          const uint32_t* keys_s, bool first) {
+  if (wave_passes(P)) return launch_wave_lambda(st, P, B, Q, keys_s, first);
   dim3 g(blocks_for(P.n, tpb)), b(tpb);
   if (P.variant == PBD_KERNEL_TEXTBOOK) {
     if (first)
@@ -421,6 +422,8 @@ static void delta_dispatch(hipStream_t st, dim3 g, dim3 b, const DevParams& P, u
 hipError_t launch_delta(hipStream_t st, uint32_t tpb, const DevParams& P, const StepBuffers& B, uint32_t flags,
                         bool delta, bool collide, const float4* Q, const float4* QX, float4* Qo, float4* QXo,
                         const uint32_t* keys_s) {
+  if ((delta || collide) && wave_passes(P))
+    return launch_wave_delta(st, P, B, flags, delta, collide, Q, QX, Qo, QXo, keys_s);
   dim3 g(blocks_for(P.n, tpb)), b(tpb);
   if (P.variant == PBD_KERNEL_TEXTBOOK)
     delta_dispatch<PBD_KERNEL_TEXTBOOK>(st, g, b, P, flags, delta, collide, Q, QX, B.LAM, keys_s, B.cstart, B.cend, Qo,
@@ -439,6 +442,7 @@ hipError_t launch_update(hipStream_t st, uint32_t tpb, const DevParams& P, const
 
 hipError_t launch_omega(hipStream_t st, uint32_t tpb, const DevParams& P, const StepBuffers& B, const float4* Q,
                         const uint32_t* keys_s) {
+  if (wave_passes(P)) return launch_wave_omega(st, P, B, Q, keys_s);
   dim3 g(blocks_for(P.n, tpb)), b(tpb);
   if (P.variant == PBD_KERNEL_TEXTBOOK)
     hipLaunchKernelGGL(k_omega<PBD_KERNEL_TEXTBOOK>, g, b, 0, st, P, Q, B.VS, keys_s, B.cstart, B.cend, B.OM);
@@ -449,6 +453,7 @@ hipError_t launch_omega(hipStream_t st, uint32_t tpb, const DevParams& P, const 
 
 hipError_t launch_final(hipStream_t st, uint32_t tpb, const DevParams& P, const StepBuffers& B, uint32_t flags,
                         const float4* Q, const float4* QX, const uint32_t* keys_s) {
+  if (wave_passes(P)) return launch_wave_final(st, P, B, flags, Q, QX, keys_s);
   dim3 g(blocks_for(P.n, tpb)), b(tpb);
   if (P.variant == PBD_KERNEL_TEXTBOOK)
     hipLaunchKernelGGL(k_final<PBD_KERNEL_TEXTBOOK>, g, b, 0, st, P, flags, Q, QX, B.VS, B.OM, keys_s, B.cstart,

@@ -138,6 +138,22 @@ hipError_t launch_final(hipStream_t st, uint32_t tpb, const DevParams& P, const 
 hipError_t launch_collide_batches(hipStream_t st, uint32_t tpb, const DevParams& P, const StepBuffers& B,
                                   float4* Q, float4* QX, const uint32_t* keys, uint32_t batches, uint32_t* solved,
                                   uint32_t words, unsigned long long* minc, uint32_t* partner);
+// The neighbour passes with a wave per particle (wave.hip), for the particle counts and
+// stencils that wave_passes names; the launchers above take them by that rule.  The line
+// lies where a thread per particle becomes the faster one (reference parameters, whole
+// step, thread / wave, us): 1,000 particles 555 / 128, 13,824 601 / 186, 46,656 617 / 339,
+// 74,088 624 / 468, 110,592 635 / 638.
+constexpr uint32_t kWaveParticles = 3u << 15;
+bool wave_passes(const DevParams& P);
+hipError_t launch_wave_lambda(hipStream_t st, const DevParams& P, const StepBuffers& B, const float4* Q,
+                              const uint32_t* keys, bool first);
+hipError_t launch_wave_delta(hipStream_t st, const DevParams& P, const StepBuffers& B, uint32_t flags, bool delta,
+                             bool collide, const float4* Q, const float4* QX, float4* Qo, float4* QXo,
+                             const uint32_t* keys);
+hipError_t launch_wave_omega(hipStream_t st, const DevParams& P, const StepBuffers& B, const float4* Q,
+                             const uint32_t* keys);
+hipError_t launch_wave_final(hipStream_t st, const DevParams& P, const StepBuffers& B, uint32_t flags, const float4* Q,
+                             const float4* QX, const uint32_t* keys);
 hipError_t launch_check_finite(hipStream_t st, uint32_t n, const float4* X, const float4* V, uint32_t* bad);
 
 // ---- LDS cell-block tiles (tiles.hip), textbook variant, 27-cell stencil ----

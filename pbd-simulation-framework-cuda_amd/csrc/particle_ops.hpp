@@ -37,7 +37,8 @@ __device__ __forceinline__ void lambda_pair(const DevParams& P, float rx, float 
 template <int VAR>
 __device__ __forceinline__ float lambda_finish(const DevParams& P, const LambdaAcc& a, float& W, float eps) {
   W = P.wc * a.A + P.w0;
-  const float G2 = P.gc * P.gc * (a.gx * a.gx + a.gy * a.gy + a.gz * a.gz);
+  const float G2 = P.gc * P.gc * (VAR == PBD_KERNEL_TEXTBOOK ? a.gx * a.gx + a.gy * a.gy + a.gz * a.gz
+                                                             : length_sq<true>(a.gx, a.gy, a.gz));
   const float B2 = P.gc * P.gc * a.B;
   if (VAR == PBD_KERNEL_TEXTBOOK) return -(W * P.inv_rho0 - 1.0f) / ((G2 + B2) * P.inv_rho0_sq + eps);
   return -(W * P.inv_rho0 - 1.0f) / (B2 * P.inv_rho0 + G2 * P.inv_rho0 + eps);
@@ -266,7 +267,7 @@ __device__ __forceinline__ void final_finish(const DevParams& P, uint32_t flags,
     float nx, ny, nz;
     if (VAR == PBD_KERNEL_REFERENCE) {
       const float EPS = 0.00000001f;
-      const float inv = 1.0f / (sqrtf(a.ex * a.ex + a.ey * a.ey + a.ez * a.ez) + EPS);
+      const float inv = 1.0f / (sqrtf(length_sq<true>(a.ex, a.ey, a.ez)) + EPS);
       nx = inv * (a.ex + EPS);
       ny = inv * (a.ey + EPS);
       nz = inv * (a.ez + EPS);
