@@ -463,6 +463,8 @@ int Fluid::enqueue_substep() {
     // phases on tiles: 2^5-cell blocks with the direct grid only
     if (P.phased && (bits != 5 || tstride)) tiles = false;
   }
+  const uint32_t wgrid = std::min(ntiles, P.n);  // the wide passes': a workgroup per block
+  const bool wide = tiles && wide_tiles(P, bits, small_max(), wgrid);
   const TileList TL{tile_list_, tile_list_ + cap_, tile_count_};
   // Lists carried over the substep: in the tiles whose halo stayed within the
   // skin over the last substep, the first lambda pass builds them with the
@@ -547,7 +549,8 @@ int Fluid::enqueue_substep() {
     if (lambda_on) {
       if (tiles) {
         PBD_LAUNCH(carry && counted ? ST_LAMBDA_CARRY : ST_LAMBDA,
-                   launch_tile_lambda(st, bits, tgrid, tstride, P, TL, list_set(it), B_.Q[cur], keys, !counted, carry,
+                   wide ? launch_wide_lambda(st, wgrid, P, TL, list_set(it), B_.Q[cur], keys, !counted, carry, it)
+                        : launch_tile_lambda(st, bits, tgrid, tstride, P, TL, list_set(it), B_.Q[cur], keys, !counted, carry,
                                       it));
         listed = true;
       } else {
@@ -620,7 +623,9 @@ int Fluid::enqueue_substep() {
   if (g & G_OMEGA) {
     if (tiles) {
       PBD_LAUNCH(ST_OMEGA,
-                 launch_tile_omega(st, bits, tgrid, tstride, P, TL, list_set(iters), B_.Q[cur], keys, xsph_in_omega,
+                 wide ? launch_wide_omega(st, wgrid, P, TL, list_set(iters), B_.Q[cur], keys, xsph_in_omega,
+                                          carry ? iters : 0u)
+                      : launch_tile_omega(st, bits, tgrid, tstride, P, TL, list_set(iters), B_.Q[cur], keys, xsph_in_omega,
                                    carry ? iters : 0u));
     } else {
       PBD_LAUNCH(ST_OMEGA, launch_omega(st, tpb, P, B_, B_.Q[cur], keys));
@@ -632,10 +637,10 @@ int Fluid::enqueue_substep() {
   if (g & G_VORTICITY) ff |= FF_VORT;
   if (g & G_VISCOSITY) ff |= xsph_in_omega ? FF_XSPH_DONE : FF_XSPH;
   if (updated) ff |= FF_UPDATED;
-  if (tiles) {
+  if (tiles)
     PBD_LAUNCH(ST_FINAL, launch_tile_final(st, bits, tgrid, tstride, P, TL, list_set(iters), ff, omega_listed,
                                            B_.Q[cur], B_.QX[cur], keys));
-  } else
+  else
     PBD_LAUNCH(ST_FINAL, launch_final(st, tpb, P, B_, ff, B_.Q[cur], B_.QX[cur], keys));
   return PBD_OK;
 }

@@ -138,6 +138,24 @@ hipError_t launch_final(hipStream_t st, uint32_t tpb, const DevParams& P, const 
 hipError_t launch_collide_batches(hipStream_t st, uint32_t tpb, const DevParams& P, const StepBuffers& B,
                                   float4* Q, float4* QX, const uint32_t* keys, uint32_t batches, uint32_t* solved,
                                   uint32_t words, unsigned long long* minc, uint32_t* partner);
+// The wide lambda and omega passes (tiles.hip): four lanes per particle, for scenes whose
+// blocks do not fill the chip.  Measured (us a step, four lanes / one lane in these two
+// passes; columns at rest keep their lists, splashes rebuild them in every pass): 2K
+// column 230 / 254, 32K column 251 / 263, 30K splash 281 / 379, 64K column 287 / 286, 64K
+// splash 381 / 422; 125K column 405 / 328, 125K splash 455 / 462.  The other passes walk
+// kept lists, and a 32K scene's take 11.1 us (delta p) and 9.6 (final) with four lanes,
+// 9.9 and 8.9 with one.  Four lanes want a workgroup per block, so a launch shape with
+// small tiles keeps one lane, and the phased tiles have no fourfold form.
+constexpr uint32_t kWideMax = 1u << 16;
+constexpr uint32_t kWideGridMax = 8192;  // possible work items (workgroups of 16 waves, most of them empty)
+inline bool wide_tiles(const DevParams& P, int bits, uint32_t small_max, uint32_t bound) {
+  return bits == 5 && small_max == 0u && !P.phased && P.n <= kWideMax && bound <= kWideGridMax;
+}
+hipError_t launch_wide_lambda(hipStream_t st, uint32_t grid, const DevParams& P, const TileList& T,
+                              const StepBuffers& B, const float4* Q, const uint32_t* keys, bool first, bool carry,
+                              uint32_t pass);
+hipError_t launch_wide_omega(hipStream_t st, uint32_t grid, const DevParams& P, const TileList& T,
+                             const StepBuffers& B, const float4* Q, const uint32_t* keys, bool xsph, uint32_t carry);
 // The neighbour passes with a wave per particle (wave.hip), for the particle counts and
 // stencils that wave_passes names; the launchers above take them by that rule.  The line
 // lies where a thread per particle becomes the faster one (reference parameters, whole

@@ -43,6 +43,13 @@ __device__ __forceinline__ float lambda_finish(const DevParams& P, const LambdaA
   if (VAR == PBD_KERNEL_TEXTBOOK) return -(W * P.inv_rho0 - 1.0f) / ((G2 + B2) * P.inv_rho0_sq + eps);
   return -(W * P.inv_rho0 - 1.0f) / (B2 * P.inv_rho0 + G2 * P.inv_rho0 + eps);
 }
+// The same (textbook) with the fused operations spelled out as the tile pass has them.
+__device__ __forceinline__ float lambda_finish_fused(const DevParams& P, const LambdaAcc& a, float& W, float eps) {
+  W = fmaf(P.wc, a.A, P.w0);
+  const float k = P.gc * P.gc;
+  const float grads = fmaf(k, a.B, k * length_sq<true>(a.gx, a.gy, a.gz));
+  return -fmaf(W, P.inv_rho0, -1.0f) / fmaf(grads, P.inv_rho0_sq, eps);
+}
 
 // ---------------------------------------------------------------- delta p + collision
 struct DeltaAcc {

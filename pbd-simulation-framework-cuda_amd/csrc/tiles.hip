@@ -1270,6 +1270,389 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_final(
 }
 
 // ---------------------------------------------------------------------------
+// Wide tile passes, for scenes whose blocks are too few to fill the chip: four lanes
+// (a quad of the wave) per particle in 1024-thread workgroups, a workgroup per occupied
+// block (there are no small tiles).  With a thread per particle a 32K scene runs 128 to 256
+// workgroups of one wave per SIMD, and a pass lasts as long as one thread's walk over
+// its particle's candidates and pairs.  Here
+//   - the lanes of a quad scan two or three of the nine stencil columns each, and write
+//     their in-range slots to the particle's list in LDS, each from the place that the
+//     counts of the lanes before it give: the list is nl_build's;
+//   - a quad takes four list entries at a time, a lane forming each pair's terms; the
+//     terms are then added in list order, each lane adding all four (the values cross
+//     the quad by DPP), with the fused operations of the one-lane passes, so the sums
+//     are theirs bit for bit.
+// The VALU work per pair nearly doubles (13 instructions a pair and lane against 29 a
+// pair), so the one-lane passes stay the faster ones once the chip is full: wide_tiles
+// in kernels.hpp draws the line.  32K column, one lane to four: lambda with its lists
+// built 21.5 to 17.4 us, omega 24.6 to 20.2 us.
+constexpr uint32_t kQuad = 4;
+constexpr uint32_t kWideParticles = kWideThreads / kQuad;  // particles of a round
+
+struct WideLds {
+  TileShared<5> sh;
+  float4 q[TileCap<5>::value + kScanUnroll];
+  uint16_t list[kWideParticles][kNlMax];  // 16-byte chunks, as the global lists'
+};
+static_assert(2 * sizeof(WideLds) <= kLdsBytes, "two workgroups per CU");
+static_assert(sizeof(TileShared<5>) % 16 == 0 || alignof(WideLds) >= 16, "alignment of the halo");
+
+// The value that lane p of the quad holds.
+template <int p>
+__device__ __forceinline__ float quad_get(float x) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(x), p * 0x55, 0xF, 0xF, true));
+}
+template <int p>
+__device__ __forceinline__ uint32_t quad_get(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, p * 0x55, 0xF, 0xF, true);
+}
+
+// The block of work item r (every occupied block is a large one).
+__device__ __forceinline__ bool wide_pick(const TileList& T, uint32_t r, uint32_t& blk) {
+  if (r >= T.count[0]) return false;
+  blk = T.large[r];
+  return true;
+}
+
+// A thread's particles for the global path: the quad's first lane takes those of the
+// rounds in `bits`; a block beyond the capacity goes round all threads.
+__device__ __forceinline__ TileRest wide_rest(uint32_t g0, uint32_t g1, bool all) {
+  TileRest r;
+  r.g = g0 + (all ? threadIdx.x : threadIdx.x / kQuad);
+  r.end = g1;
+  r.stride = all ? kWideThreads : kWideParticles;
+  r.all = all;
+  return r;
+}
+
+// Builds the list of the quad's particle into `list` (LDS) and, chunk by chunk, the
+// global lists; as nl_build.  A column's first 64 slots are scanned once, their bits
+// kept in registers; what a longer column has more is scanned again when its slots are
+// written.
+__device__ __forceinline__ uint32_t wide_build(const NeighbourList& L, uint32_t g, const TileShared<5>& sh,
+                                               const float4* s_q, uint16_t* list, int h, uint32_t slot, float4 qi,
+                                               float r2) {
+  using G = TileGeom<5>;
+  constexpr uint32_t CAP = TileCap<5>::value;
+  const uint32_t sub = threadIdx.x % kQuad;
+  const float nan = qi.x + qi.y + qi.z;
+  const uint32_t valid = nan == nan ? 0xFFFFFFFFu : 0u;
+  const auto scan = [&](uint32_t s, uint32_t b) __attribute__((always_inline)) {
+    uint32_t m = nl_mask(s_q, s, min(b - s, 32u), qi.x, qi.y, qi.z, r2) & valid;
+    if (slot - s < 32u) m &= ~(1u << (slot - s));  // not the particle itself
+    return m;
+  };
+  // columns 2 sub and 2 sub + 1; the last lane column 8 too
+  uint32_t a[3], b[3], m0[3], m1[3], cnt = 0u;
+#pragma unroll
+  for (uint32_t k = 0; k < 3u; ++k) {
+    const uint32_t c = 2u * sub + k;
+    const int hb = h + ((int)(c / 3u) - 1) * G::SX + ((int)(c % 3u) - 1) * G::SY;
+    const bool mine = k < 2u || sub == kQuad - 1u;
+    a[k] = mine ? sh.lstart[hb - 1] : 0u;
+    b[k] = mine ? sh.lstart[hb + 2] : 0u;
+    m0[k] = m1[k] = 0u;
+    if (a[k] < b[k]) m0[k] = scan(a[k], b[k]);
+    if (a[k] + 32u < b[k]) m1[k] = scan(a[k] + 32u, b[k]);
+    cnt += __builtin_popcount(m0[k]) + __builtin_popcount(m1[k]);
+    for (uint32_t s = a[k] + 64u; s < b[k]; s += 32u) cnt += __builtin_popcount(scan(s, b[k]));
+  }
+  const uint32_t c0 = quad_get<0>(cnt), c1 = quad_get<1>(cnt), c2 = quad_get<2>(cnt), c3 = quad_get<3>(cnt);
+  const uint32_t n = c0 + c1 + c2 + c3;
+  if (n > kNlMax) return kNlInvalid;
+  uint32_t i = (sub > 0u ? c0 : 0u) + (sub > 1u ? c1 : 0u) + (sub > 2u ? c2 : 0u);
+  const auto put = [&](uint32_t s, uint32_t m) __attribute__((always_inline)) {
+    while (m) {
+      list[i++] = (uint16_t)(s + (uint32_t)__builtin_ctz(m));
+      m &= m - 1u;
+    }
+  };
+#pragma unroll
+  for (uint32_t k = 0; k < 3u; ++k) {
+    put(a[k], m0[k]);
+    put(a[k] + 32u, m1[k]);
+    for (uint32_t s = a[k] + 64u; s < b[k]; s += 32u) put(s, scan(s, b[k]));
+  }
+  const uint32_t np = (n + 7u) & ~7u;
+  for (uint32_t k = n + sub; k < np; k += kQuad) list[k] = (uint16_t)CAP;
+  TeamWave::sync();
+  for (uint32_t c = sub; c < np / 8u; c += kQuad)
+    L.nl[(size_t)c * L.cap + g] = *reinterpret_cast<const uint4*>(list + 8u * c);
+  return np;
+}
+
+// The list of particle g (n entries, a multiple of 8) from the global lists.
+__device__ __forceinline__ void wide_fetch(const NeighbourList& L, uint32_t g, uint32_t n, uint16_t* list) {
+  for (uint32_t c = threadIdx.x % kQuad; c < n / 8u; c += kQuad)
+    *reinterpret_cast<uint4*>(list + 8u * c) = L.nl[(size_t)c * L.cap + g];
+  TeamWave::sync();
+}
+
+// The quad's walk over the list: pair(j) forms a lane's terms (of slot j), add(get) adds
+// those of one lane, get(x) its value of x, lane after lane.
+template <class Pair, class Add>
+__device__ __forceinline__ void wide_visit(const uint16_t* list, uint32_t n, Pair pair, Add add) {
+  const uint32_t sub = threadIdx.x % kQuad;
+  const auto quad = [&](const auto& t) __attribute__((always_inline)) {
+    add(t, [](auto x) __attribute__((always_inline)) { return quad_get<0>(x); });
+    add(t, [](auto x) __attribute__((always_inline)) { return quad_get<1>(x); });
+    add(t, [](auto x) __attribute__((always_inline)) { return quad_get<2>(x); });
+    add(t, [](auto x) __attribute__((always_inline)) { return quad_get<3>(x); });
+  };
+  for (uint32_t k = 0; k < n; k += 2u * kQuad) {  // n is a multiple of 8
+    const auto t0 = pair((uint32_t)list[k + sub]);
+    const auto t1 = pair((uint32_t)list[k + kQuad + sub]);
+    quad(t0);
+    quad(t1);
+  }
+}
+
+template <bool FIRST>
+__global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileList T, NeighbourList L,
+                                                              const float4* __restrict__ Q,
+                                                              const uint32_t* __restrict__ keys,
+                                                              const uint32_t* __restrict__ cs,
+                                                              const uint32_t* __restrict__ ce,
+                                                              float* __restrict__ lam, float* __restrict__ dens,
+                                                              uint32_t* __restrict__ ncnt,
+                                                              uint32_t* __restrict__ ccnt, Carry C) {
+  constexpr int VAR = PBD_KERNEL_TEXTBOOK;
+  constexpr int CAP = TileCap<5>::value;
+  __shared__ WideLds lds;
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&L.stats[PBD_COUNTER_LIST_BUILDS], 1ull);
+  uint32_t blk;
+  if (!wide_pick(T, blockIdx.x, blk)) return;
+  TileShared<5>& sh = lds.sh;
+  const uint32_t tid = threadIdx.x, sub = tid % kQuad;
+  const uint32_t total = tile_setup<5, TeamWide>(P, blk, cs, ce, sh);
+  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  TileRest rest = wide_rest(g0, g1, total > (uint32_t)CAP);
+  if (total > (uint32_t)CAP) {
+    for (uint32_t g = g0 + tid; g < g1; g += kWideThreads) L.cnt[g] = kNlInvalid;
+    if (tid == 0) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_BLOCK], (unsigned long long)(g1 - g0));
+  } else {
+    // as lambda_tile
+    const uint32_t m = C.disp ? (FIRST ? (C.mode[blk] ? 0u : kNoCarry) : C.built[blk]) : kNoCarry;
+    const bool carry = !FIRST && m != kNoCarry;
+    const float r2 = m != kNoCarry ? P.tile_r2 : P.list_r2;
+    tile_load<5, CAP, TeamWide>(P, sh, total, Q, lds.q, nullptr, 0u, [](uint32_t) { return 0.0f; },
+                                carry ? C.bounds(C.pass) : nullptr, carry ? C.bounds(m) : nullptr);
+    __syncthreads();
+    const bool keep = carry && tile_keeps_lists<5>(P, sh);
+    if (tid == 0 && C.disp) {
+      if (FIRST) C.built[blk] = m;
+      else if (carry && !keep) C.built[blk] = C.pass;
+      if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
+                           (unsigned long long)(g1 - g0));
+    }
+    uint16_t* list = lds.list[tid / kQuad];
+    uint32_t round = 0u;
+    for (uint32_t g = g0 + tid / kQuad; g < g1; g += kWideParticles, ++round) {
+      int h;
+      uint32_t slot;
+      tile_locate<5>(sh, keys[g], g, h, slot);
+      uint32_t cnt = 0u, n = keep ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
+      if (!keep || n == kNlInvalid) {
+        cnt = tile_count<5>(sh, h);
+        if (cnt > P.cap) {
+          if (sub == 0u) {
+            rest.bits |= 1u << round;
+            if (!keep) {
+              L.cnt[g] = kNlInvalid;
+              atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_CAP], 1ull);
+            }
+          }
+          continue;
+        }
+      }
+      const float4 qi = lds.q[slot];
+      if (!keep) {
+        n = wide_build(L, g, sh, lds.q, list, h, slot, qi, r2);
+        if (sub == 0u) {
+          L.cnt[g] = (uint16_t)n;
+          if (n == kNlInvalid) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_LONG], 1ull);
+        }
+      } else if (n != kNlInvalid) {
+        wide_fetch(L, g, n, list);
+      }
+      LambdaAcc a;
+      if (n != kNlInvalid) {
+        struct Term {
+          float rx, ry, rz, t, t2, g, hr4;
+        };
+        wide_visit(
+            list, n,
+            [&](uint32_t j) __attribute__((always_inline)) {
+              const float4 qj = slot_read(lds.q, j);
+              Term e;
+              e.rx = qi.x - qj.x;
+              e.ry = qi.y - qj.y;
+              e.rz = qi.z - qj.z;
+              const float d2 = length_sq(e.rx, e.ry, e.rz);
+              e.t = fmaxf(P.hp2 - d2, 0.0f);
+              e.t2 = e.t * e.t;
+              e.g = grad_factor<VAR>(P, d2, e.hr4);
+              return e;
+            },
+            [&](const Term& e, auto get) __attribute__((always_inline)) {
+              const float g1_ = get(e.g);
+              a.A = fmaf(get(e.t), get(e.t2), a.A);
+              a.gx = fmaf(get(e.rx), g1_, a.gx);
+              a.gy = fmaf(get(e.ry), g1_, a.gy);
+              a.gz = fmaf(get(e.rz), g1_, a.gz);
+              a.B += get(e.hr4);
+            });
+      } else {  // more pairs than a list holds: every lane scans
+        tile_stencil<5>(sh, h, slot, [&](uint32_t j) __attribute__((always_inline)) {
+          const float4 qj = slot_read(lds.q, j);
+          lambda_pair<VAR>(P, qi.x - qj.x, qi.y - qj.y, qi.z - qj.z, a);
+        });
+      }
+      if (sub != 0u) continue;
+      float W;
+      lam[g] = lambda_finish_fused(P, a, W, scene_eps(P, keys[g]));
+      if (FIRST) {
+        dens[g] = W;
+        ncnt[g] = cnt;
+        ccnt[g] = cnt;
+      }
+    }
+  }
+  rest.visit([&](uint32_t g) __attribute__((always_inline)) {
+    lambda_particle<VAR, FIRST>(P, g, Q, keys, cs, ce, lam, dens, ncnt, ccnt);
+  });
+}
+
+template <bool XSPH>
+__global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileList T, NeighbourList L,
+                                                             const float4* __restrict__ Q,
+                                                             const float4* __restrict__ VS,
+                                                             const uint32_t* __restrict__ keys,
+                                                             const uint32_t* __restrict__ cs,
+                                                             const uint32_t* __restrict__ ce, float4* __restrict__ OM,
+                                                             float4* __restrict__ Vo, Carry C) {
+  constexpr int VAR = PBD_KERNEL_TEXTBOOK;
+  constexpr int CAP = TileCap<5>::value;
+  __shared__ WideLds lds;
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&L.stats[PBD_COUNTER_LIST_BUILDS], 1ull);
+  uint32_t blk;
+  if (!wide_pick(T, blockIdx.x, blk)) return;
+  TileShared<5>& sh = lds.sh;
+  const uint32_t tid = threadIdx.x, sub = tid % kQuad;
+  const uint32_t total = tile_setup<5, TeamWide>(P, blk, cs, ce, sh);
+  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  TileRest rest = wide_rest(g0, g1, total > (uint32_t)CAP);
+  if (total > (uint32_t)CAP) {
+    for (uint32_t g = g0 + tid; g < g1; g += kWideThreads) L.cnt[g] = kNlInvalid;
+    if (tid == 0) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_BLOCK], (unsigned long long)(g1 - g0));
+  } else {
+    // as omega_tile; .w: the slot's global index (velocities are gathered from L2), of the
+    // sentinel the block's first particle (its pair terms are zero)
+    const uint32_t m = C.disp ? C.built[blk] : kNoCarry;
+    const bool carry = m != kNoCarry;
+    tile_load<5, CAP, TeamWide>(P, sh, total, Q, lds.q, nullptr, 0u,
+                                [](uint32_t gi) { return __uint_as_float(gi); }, C.disp ? C.bounds(C.pass) : nullptr,
+                                carry ? C.bounds(m) : nullptr);
+    __syncthreads();
+    const bool calm = C.disp && tile_keeps_lists<5>(P, sh);
+    const bool keep = carry && calm;
+    if (tid == 0 && C.disp) {
+      C.mode[blk] = calm ? 1u : 0u;
+      if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
+                           (unsigned long long)(g1 - g0));
+    }
+    uint16_t* list = lds.list[tid / kQuad];
+    uint32_t round = 0u;
+    for (uint32_t g = g0 + tid / kQuad; g < g1; g += kWideParticles, ++round) {
+      int h;
+      uint32_t slot;
+      tile_locate<5>(sh, keys[g], g, h, slot);
+      uint32_t n = keep ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
+      if (n == kNlInvalid && tile_count<5>(sh, h) > P.cap) {
+        if (sub == 0u) {
+          rest.bits |= 1u << round;
+          if (!keep) {
+            L.cnt[g] = kNlInvalid;
+            atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_CAP], 1ull);
+          }
+        }
+        continue;
+      }
+      const float4 qi = lds.q[slot];
+      const float4 v4 = VS[g];
+      const float vx = v4.x, vy = v4.y, vz = v4.z, vw = v4.w;
+      if (!keep) {
+        n = wide_build(L, g, sh, lds.q, list, h, slot, qi, P.list_r2);
+        if (sub == 0u) {
+          L.cnt[g] = (uint16_t)n;
+          if (n == kNlInvalid) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_LONG], 1ull);
+        }
+      } else if (n != kNlInvalid) {
+        wide_fetch(L, g, n, list);
+      }
+      OmegaAcc a;
+      FinalAcc xa;
+      if (n != kNlInvalid) {
+        struct Term {
+          float ox, oy, oz, w, dx, dy, dz, dw;
+        };
+        wide_visit(
+            list, n,
+            [&](uint32_t j) __attribute__((always_inline)) {
+              const float4 qj = lds.q[j];
+              const float4 vj = VS[j == (uint32_t)CAP ? g0 : __float_as_uint(qj.w)];
+              const float rx = qi.x - qj.x, ry = qi.y - qj.y, rz = qi.z - qj.z;
+              const float d2 = length_sq(rx, ry, rz);
+              Term e;
+              e.dx = vj.x - vx;
+              e.dy = vj.y - vy;
+              e.dz = vj.z - vz;
+              e.dw = vj.w - vw;
+              float hr4;
+              const float gf = grad_factor<VAR>(P, d2, hr4);
+              const float gx = gf * rx, gy = gf * ry, gz = gf * rz;
+              e.ox = fmaf(e.dy, gz, -(e.dz * gy));
+              e.oy = fmaf(e.dz, gx, -(e.dx * gz));
+              e.oz = fmaf(e.dx, gy, -(e.dy * gx));
+              e.w = XSPH ? w_unnorm<VAR>(P, d2) : 0.0f;
+              return e;
+            },
+            [&](const Term& e, auto get) __attribute__((always_inline)) {
+              a.ox += get(e.ox);
+              a.oy += get(e.oy);
+              a.oz += get(e.oz);
+              if (XSPH) {
+                const float w = get(e.w);
+                xa.sx = fmaf(get(e.dx), w, xa.sx);
+                xa.sy = fmaf(get(e.dy), w, xa.sy);
+                xa.sz = fmaf(get(e.dz), w, xa.sz);
+                xa.sw = fmaf(get(e.dw), w, xa.sw);
+              }
+            });
+      } else {
+        tile_stencil<5>(sh, h, slot, [&](uint32_t j) __attribute__((always_inline)) {
+          const float4 qj = lds.q[j];
+          const float4 vj = VS[__float_as_uint(qj.w)];
+          const float rx = qi.x - qj.x, ry = qi.y - qj.y, rz = qi.z - qj.z;
+          omega_pair<VAR>(P, rx, ry, rz, vj.x - vx, vj.y - vy, vj.z - vz, a);
+          if (XSPH) final_pair_textbook<VAR>(P, false, true, rx, ry, rz, make_float4(vx, vy, vz, vw), vj, 0.0f, 0.0f, xa);
+        });
+      }
+      if (sub != 0u) continue;
+      OM[g] = omega_finish<VAR>(P, a);
+      if (XSPH) {
+        const float c = P.c_visc * P.wc * P.vol;
+        Vo[g] = make_float4(vx + c * xa.sx, vy + c * xa.sy, vz + c * xa.sz, vw + c * xa.sw);
+      }
+    }
+  }
+  rest.visit([&](uint32_t g) __attribute__((always_inline)) {
+    omega_particle<VAR>(P, g, Q, VS, keys, cs, ce, OM);
+    if (XSPH) Vo[g] = xsph_particle<VAR>(P, g, Q, VS, keys, cs, ce);
+  });
+}
+
+// ---------------------------------------------------------------------------
 // Host launchers.
 static NeighbourList nlist(const StepBuffers& B) { return NeighbourList{B.NL, B.NLC, B.nl_cap, B.STATS}; }
 // pass > 0: carried lists (lambda, omega) or recorded bounds (delta-p) of pass `pass`
@@ -1418,6 +1801,35 @@ hipError_t launch_tile_final(hipStream_t st, int bits, uint32_t grid, bool strid
   }
 #undef PBD_FINAL_S
 #undef PBD_FINAL
+  return hipGetLastError();
+}
+
+// The wide passes: `grid` workgroups, one per possible work item.
+hipError_t launch_wide_lambda(hipStream_t st, uint32_t grid, const DevParams& P, const TileList& T,
+                              const StepBuffers& B, const float4* Q, const uint32_t* keys, bool first, bool carry,
+                              uint32_t pass) {
+  if (pass > kCarryPasses || first != (pass == 0) || (carry && !(B.DISP && B.BUILT && B.MODE)) || P.phased)
+    return hipErrorInvalidValue;
+  const Carry C = carry_of(B, pass, carry);
+  if (first)
+    hipLaunchKernelGGL(k_wide_lambda<true>, dim3(grid), dim3(kWideThreads), 0, st, P, T, nlist(B), Q, keys, B.cstart,
+                       B.cend, B.LAM, B.DENS, B.NCNT, B.CCNT, C);
+  else
+    hipLaunchKernelGGL(k_wide_lambda<false>, dim3(grid), dim3(kWideThreads), 0, st, P, T, nlist(B), Q, keys, B.cstart,
+                       B.cend, B.LAM, B.DENS, B.NCNT, B.CCNT, C);
+  return hipGetLastError();
+}
+
+hipError_t launch_wide_omega(hipStream_t st, uint32_t grid, const DevParams& P, const TileList& T,
+                             const StepBuffers& B, const float4* Q, const uint32_t* keys, bool xsph, uint32_t carry) {
+  if (carry > kCarryPasses || (carry && !(B.DISP && B.BUILT)) || P.phased) return hipErrorInvalidValue;
+  const Carry C = carry_of(B, carry, carry != 0);
+  if (xsph)
+    hipLaunchKernelGGL(k_wide_omega<true>, dim3(grid), dim3(kWideThreads), 0, st, P, T, nlist(B), Q, B.VS, keys,
+                       B.cstart, B.cend, B.OM, B.V, C);
+  else
+    hipLaunchKernelGGL(k_wide_omega<false>, dim3(grid), dim3(kWideThreads), 0, st, P, T, nlist(B), Q, B.VS, keys,
+                       B.cstart, B.cend, B.OM, B.V, C);
   return hipGetLastError();
 }
 
