@@ -465,7 +465,7 @@ int Fluid::enqueue_substep() {
   }
   const uint32_t wgrid = std::min(ntiles, P.n);  // the wide passes': a workgroup per block
   const bool wide = tiles && wide_tiles(P, bits, small_max(), wgrid);
-  const TileList TL{tile_list_, tile_list_ + cap_, tile_count_};
+  const TileList TL{tile_list_, tile_list_ + cap_, tile_count_, tile_flag_, tile_end_, cap_};
   // Lists carried over the substep: in the tiles whose halo stayed within the
   // skin over the last substep, the first lambda pass builds them with the
   // skin, and the later lambda passes and the omega pass keep them while the

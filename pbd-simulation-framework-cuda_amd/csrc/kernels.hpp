@@ -64,6 +64,9 @@ struct TileList {
   const uint32_t* large;  // block ids (cell id >> bits) of the large tiles, ascending
   const uint32_t* small;  // block ids of the small tiles, ascending
   const uint32_t* count;  // count[0] large tiles, count[1] small tiles
+  const uint32_t* start;  // per occupied block: 1 + its first sorted index
+  const uint32_t* end;    // per occupied block: 1 + its last
+  uint32_t cap;           // entries of large
 };
 
 constexpr uint32_t kTileSmall = 64;           // particles of a small tile (one wave)

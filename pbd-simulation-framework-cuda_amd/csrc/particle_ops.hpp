@@ -139,11 +139,11 @@ __device__ __forceinline__ void delta_pair(const DevParams& P, float li, float l
   }
 }
 
-// Apply the pass to particle s (cell `key`, corner c): Qo/QXo <- (q, qx) + push -+ dp
+// Apply the pass to particle s (cell `key`, corner c; qi, qxi: its Q and QX): Qo/QXo <- (q, qx) + push -+ dp
 // (+ projection onto the scene's enclosure), update.  Returns the new position (cell frame).
 template <int VAR, bool DELTA>
 __device__ __forceinline__ float4 delta_finish(const DevParams& P, uint32_t flags, uint32_t s, float4 qi,
-                                             const float4* __restrict__ QX, const DeltaAcc& a, float cx, float cy,
+                                             float4 qxi, const DeltaAcc& a, float cx, float cy,
                                              float cz, uint32_t key, float4* __restrict__ Qo,
                                              float4* __restrict__ QXo, float4* __restrict__ DP,
                                              float4* __restrict__ VS) {
@@ -160,7 +160,6 @@ __device__ __forceinline__ float4 delta_finish(const DevParams& P, uint32_t flag
     dy = d.y;
     dz = d.z;
   }
-  const float4 qxi = QX[s];
   float nx = qi.x + a.px + a.fx, ny = qi.y + a.py + a.fy, nz = qi.z + a.pz + a.fz;
   float4 qx = make_float4(qxi.x + a.px, qxi.y + a.py, qxi.z + a.pz, qxi.w);
   if (flags & DF_APPLY) {
@@ -387,7 +386,7 @@ __device__ __forceinline__ float4 delta_particle(const DevParams& P, uint32_t fl
                        }
                      });
   }
-  return delta_finish<VAR, DELTA>(P, flags, s, qi, QX, a, f.cx, f.cy, f.cz, keys[s], Qo, QXo, DP, VS);
+  return delta_finish<VAR, DELTA>(P, flags, s, qi, QX[s], a, f.cx, f.cy, f.cz, keys[s], Qo, QXo, DP, VS);
 }
 
 // P.phs: phases (nullptr: all fluid); omega of a solid particle is 0, a fluid one

@@ -71,21 +71,49 @@ struct TileShared {
 };
 static_assert(TileGeom<6>::HX <= 6 && TileGeom<6>::HY <= 6 && TileGeom<6>::HZ <= 6, "offset table");
 
-// Steps 1 of the tile: halo cell table, LDS offsets, own range.  Returns the
-// halo particle count.  Every thread of the team takes R halo cells; all their
-// cell-table loads are issued before the scan.
-template <int BITS, class Team>
+// Steps 1 of the tile: halo cell table, LDS offsets and, with OWN, the own range.
+// Returns the halo particle count.  Every thread of the team takes R halo cells; all
+// their cell-table loads are issued, then those of `pre` (what the thread reads whatever
+// the halo holds), before the first is waited for: a pass over a small scene is a chain
+// of loads that miss the L2, about 0.8 us each.  With the block's own range from the
+// tile marks, the key, list length and first chunk read here and the tile's number read
+// beside the counts (us a step, before / now): 2K 230 / 220, 32K column 250 / 235, 1M
+// column 1096 / 1080, 1M splash 1725 / 1631.
+struct NoLoads {
+  __device__ __forceinline__ void operator()() const {}
+};
+template <int BITS, class Team, bool OWN = true, class Pre = NoLoads>
 __device__ __forceinline__ uint32_t tile_setup(const DevParams& P, uint32_t blk, const uint32_t* __restrict__ cs,
-                                               const uint32_t* __restrict__ ce, TileShared<BITS>& sh) {
+                                               const uint32_t* __restrict__ ce, TileShared<BITS>& sh,
+                                               Pre pre = Pre()) {
   using G = TileGeom<BITS>;
   constexpr uint32_t R = (G::NH + Team::kSize - 1u) / Team::kSize;
   static_assert(Team::kSize == 64u || R == 1u, "a workgroup team takes one halo cell per thread");
   const uint32_t tid = Team::tid(), lane = threadIdx.x & 63u;
   const uint32_t first = blk << BITS;
   const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
+  uint32_t s0[R], e0[R];
+#pragma unroll
+  for (uint32_t r = 0; r < R; ++r) {
+    const uint32_t c = r * Team::kSize + tid;
+    s0[r] = 0xFFFFFFFFu;
+    e0[r] = 0u;
+    if (c < (uint32_t)G::NH) {
+      const int hx = (int)c / G::SX, hy = ((int)c / G::SY) % G::HY, hz = (int)c % G::HZ;
+      const int cx = ix0 - 1 + hx, cy = iy0 - 1 + hy, cz = iz0 - 1 + hz;
+      if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
+        const uint32_t k = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
+        s0[r] = cs[k];
+        e0[r] = ce[k];
+      }
+    }
+  }
+  pre();
   if (tid == 0) {
-    sh.g0 = 0xFFFFFFFFu;
-    sh.g1 = 0u;
+    if (OWN) {
+      sh.g0 = 0xFFFFFFFFu;
+      sh.g1 = 0u;
+    }
     sh.dmax = 0u;
   }
   // Offsets of the halo cells' corners from the block's first cell's.  In a batched
@@ -98,30 +126,21 @@ __device__ __forceinline__ uint32_t tile_setup(const DevParams& P, uint32_t blk,
     const float o = frame_origin(P, scene_of_key(P, first), (int)a);
     sh.off[a][k] = frame_corner(P, o, i0 + k - 1u) - frame_corner(P, o, i0);
   }
-  Team::sync();
+  if (OWN) Team::sync();
   uint32_t cnt[R];
 #pragma unroll
   for (uint32_t r = 0; r < R; ++r) {
     const uint32_t c = r * Team::kSize + tid;
-    uint32_t n = 0, st = 0;
-    if (c < (uint32_t)G::NH) {
+    const bool some = s0[r] != 0xFFFFFFFFu;
+    cnt[r] = some ? e0[r] - s0[r] : 0u;
+    if (c < (uint32_t)G::NH) sh.gstart[c] = some ? s0[r] : 0u;
+    if (OWN && some) {
       const int hx = (int)c / G::SX, hy = ((int)c / G::SY) % G::HY, hz = (int)c % G::HZ;
-      const int cx = ix0 - 1 + hx, cy = iy0 - 1 + hy, cz = iz0 - 1 + hz;
-      if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
-        const uint32_t k = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
-        const uint32_t s0 = cs[k], e0 = ce[k];
-        if (s0 != 0xFFFFFFFFu) {
-          st = s0;
-          n = e0 - s0;
-          if (hx >= 1 && hx <= G::EX && hy >= 1 && hy <= G::EY && hz >= 1 && hz <= G::EZ) {
-            atomicMin(&sh.g0, st);
-            atomicMax(&sh.g1, st + n);
-          }
-        }
+      if (hx >= 1 && hx <= G::EX && hy >= 1 && hy <= G::EY && hz >= 1 && hz <= G::EZ) {
+        atomicMin(&sh.g0, s0[r]);
+        atomicMax(&sh.g1, e0[r]);
       }
-      sh.gstart[c] = st;
     }
-    cnt[r] = n;
   }
   if constexpr (Team::kSize == 64u) {
     uint32_t carry = 0;
@@ -281,12 +300,14 @@ __device__ __forceinline__ uint32_t tile_rank0() {
 // workgroup, 2 = small tile `blk` for this wave, 0 = none (for this wave, none at
 // any later rank either).
 __device__ __forceinline__ int tile_pick(const TileList& T, const TileItems& it, uint32_t r, uint32_t& blk) {
+  // loaded with the counts, not after them (the list has T.cap entries)
+  const uint32_t large = T.large[min(r, T.cap - 1u)];
   if (r < it.nl) {
-    blk = T.large[r];
+    blk = large;
     return 1;
   }
   if (r >= it.end) return 0;
-  const uint32_t i = (r - it.nl) * (kTileThreads / 64u) + (threadIdx.x >> 6);
+  const uint32_t i = (r - it.nl) * (kTileThreads / 64u) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (i < it.ns) {
     blk = T.small[i];
     return 2;
@@ -640,13 +661,12 @@ __device__ __forceinline__ void track_move(const Carry& C, uint32_t g, float4 fr
   C.bounds(C.pass)[g] = (prev ? prev[g] : 0.0f) + sqrtf(dx * dx + dy * dy + dz * dz);
 }
 
-// Visit the global list of particle g (n = padded length) in order.
+// Visit the global list of particle g (n = padded length) in order; w: its first chunk.
 template <class Body>
-__device__ __forceinline__ void nl_visit(const NeighbourList& L, uint32_t g, uint32_t n, Body body) {
+__device__ __forceinline__ void nl_visit(const NeighbourList& L, uint32_t g, uint32_t n, uint4 w, Body body) {
   const uint4* p = L.nl + g;
   const uint32_t nc = n >> 3;
   if (nc == 0) return;
-  uint4 w = p[0];
   for (uint32_t c = 1; c <= nc; ++c) {
     const uint4 nx = c < nc ? p[(size_t)c * L.cap] : w;
     body(w.x & 0xFFFFu);
@@ -787,7 +807,7 @@ __device__ __forceinline__ uint32_t nl_build(const DevParams& P, const Neighbour
 // tile built after an earlier delta-p pass when its halo has moved less than
 // P.reuse_max since.  A carrying tile builds with the skin (P.tile_r2).
 template <int BITS, bool FIRST, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest lambda_tile(const DevParams& P, uint32_t blk, const NeighbourList& L,
+__device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L,
                                             const float4* __restrict__ Q, const uint32_t* __restrict__ keys,
                                             const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
                                             float* __restrict__ lam, float* __restrict__ dens,
@@ -795,8 +815,11 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, uint32_t blk
                                             const Carry& C, TileShared<BITS>& sh, float4* s_q) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  uint32_t key = 0u;  // of the thread's next particle
+  const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
+    if (g0 + tid < g1) key = keys[g0 + tid];
+  });
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) L.cnt[g] = kNlInvalid;
@@ -822,9 +845,10 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, uint32_t blk
   }
   uint32_t round = 0u;
   for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
+    if (round) key = keys[g];
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, keys[g], g, h, slot);
+    tile_locate<BITS>(sh, key, g, h, slot);
     uint32_t cnt = 0u, n = kNlInvalid;
     if (keep) {
       // a kept list, or none: a particle over the cap takes the global path as
@@ -862,10 +886,10 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, uint32_t blk
       lam[g] = 0.0f;
       continue;
     }
-    if (n != kNlInvalid) nl_visit(L, g, n, pair);
+    if (n != kNlInvalid) nl_visit(L, g, n, L.nl[g], pair);
     else tile_stencil<BITS>(sh, h, slot, pair);
     float W;
-    const float l = lambda_finish<VAR>(P, a, W, scene_eps(P, keys[g]));
+    const float l = lambda_finish<VAR>(P, a, W, scene_eps(P, key));
     lam[g] = PH && qi.w != 0.0f ? 0.0f : l;
     if (FIRST) {
       dens[g] = W;
@@ -895,11 +919,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_lambda(DevParams P, TileL
     if (mode == 0) break;
     TileRest rest;
     if (mode == 1) {
-      rest = lambda_tile<BITS, FIRST, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
+      rest = lambda_tile<BITS, FIRST, PH, TeamBlock, TileCap<BITS>::value>(P, T, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
                                                                        ccnt, C, lds.big.sh, lds.big.q);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = lambda_tile<BITS, FIRST, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
+      rest = lambda_tile<BITS, FIRST, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
                                                                       ccnt, C, reg.sh, reg.q);
     }
     rest.visit([&](uint32_t g) __attribute__((always_inline)) {
@@ -914,7 +938,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_lambda(DevParams P, TileL
 // lists (use_list) or a scan of the stencil; with a carry, each particle's
 // displacement bound after the pass is recorded.
 template <int BITS, bool COLLIDE, int NS, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest delta_tile(const DevParams& P, uint32_t blk, const NeighbourList& L, int use_list,
+__device__ __forceinline__ TileRest delta_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L, int use_list,
                                            uint32_t flags, const float4* __restrict__ Q,
                                            const float4* __restrict__ QX, const float* __restrict__ lam,
                                            const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cs,
@@ -924,8 +948,20 @@ __device__ __forceinline__ TileRest delta_tile(const DevParams& P, uint32_t blk,
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  // the thread's next particle: its key, list length and first chunk
+  uint32_t key = 0u, n = kNlInvalid;
+  uint4 chunk = make_uint4(0u, 0u, 0u, 0u);
+  const auto next = [&](uint32_t g) __attribute__((always_inline)) {
+    key = keys[g];
+    if (use_list) {
+      n = L.cnt[g];
+      chunk = L.nl[g];
+    }
+  };
+  const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
+    if (g0 + tid < g1) next(g0 + tid);
+  });
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) return rest;
   // s_gi (friction-capable passes): the global index of every slot, for the
@@ -934,17 +970,17 @@ __device__ __forceinline__ TileRest delta_tile(const DevParams& P, uint32_t blk,
   Team::sync();
   uint32_t round = 0u;
   for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
-    const uint32_t key = keys[g];
+    if (round) next(g);
     int h;
     uint32_t slot;
     tile_locate<BITS>(sh, key, g, h, slot);
-    const uint32_t n = use_list ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
     // with phases, a particle without a list takes the global path (the tile holds
     // no phases for a scan)
     if (n == kNlInvalid && (PH || tile_count<BITS>(sh, h) > P.cap)) {
       rest.bits |= 1u << round;
       continue;
     }
+    const float4 q0 = Q[g], qx = QX[g];  // for the end, loaded beside the walk
     const float4 qb = s_q[slot];
     // phases: delta p between fluid particles only; the contact push on every pair,
     // friction on contacts with a solid (displacements p* - x from the global arrays)
@@ -952,10 +988,9 @@ __device__ __forceinline__ TileRest delta_tile(const DevParams& P, uint32_t blk,
     const bool fric = PH && COLLIDE && P.mu_s > 0.0f;
     float dix = 0.0f, diy = 0.0f, diz = 0.0f;
     if (fric) {
-      const float4 qg = Q[g], xg = QX[g];
-      dix = qg.x - xg.x;
-      diy = qg.y - xg.y;
-      diz = qg.z - xg.z;
+      dix = q0.x - qx.x;
+      diy = q0.y - qx.y;
+      diz = q0.z - qx.z;
     }
     DeltaAcc a;
     const auto pair = [&](uint32_t e) __attribute__((always_inline)) {
@@ -979,14 +1014,13 @@ __device__ __forceinline__ TileRest delta_tile(const DevParams& P, uint32_t blk,
         delta_pair<VAR, true, COLLIDE, NS, PH && !COLLIDE>(P, qb.w, qj.w, rx, ry, rz, true, a);
       }
     };
-    if (n != kNlInvalid) nl_visit(L, g, n, pair);
+    if (n != kNlInvalid) nl_visit(L, g, n, chunk, pair);
     else tile_stencil<BITS>(sh, h, slot, pair);
     const uint32_t sc = scene_of_key(P, key);
     const float cx = frame_corner(P, frame_origin(P, sc, 0), compact10(key >> 2));
     const float cy = frame_corner(P, frame_origin(P, sc, 1), compact10(key >> 1));
     const float cz = frame_corner(P, frame_origin(P, sc, 2), compact10(key));
-    const float4 q0 = Q[g];
-    track_move(C, g, q0, delta_finish<VAR, true>(P, flags, g, q0, QX, a, cx, cy, cz, key, Qo, QXo, DP, VS));
+    track_move(C, g, q0, delta_finish<VAR, true>(P, flags, g, q0, qx, a, cx, cy, cz, key, Qo, QXo, DP, VS));
   }
   return rest;
 }
@@ -1015,11 +1049,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_delta(DevParams P, TileLi
     TileRest rest;
     if (mode == 1) {
       rest = delta_tile<BITS, COLLIDE, NS, PH, TeamBlock, TileCap<BITS>::value>(
-          P, blk, L, use_list, flags, Q, QX, lam, keys, cs, ce, Qo, QXo, DP, VS, C, lds.big.sh, lds.big.q,
+          P, T, blk, L, use_list, flags, Q, QX, lam, keys, cs, ce, Qo, QXo, DP, VS, C, lds.big.sh, lds.big.q,
           GI ? lds.big.gi : nullptr);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, use_list, flags, Q, QX, lam,
+      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, use_list, flags, Q, QX, lam,
                                                                            keys, cs, ce, Qo, QXo, DP, VS, C, reg.sh,
                                                                            reg.q, GI ? reg.gi : nullptr);
     }
@@ -1042,7 +1076,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_delta(DevParams P, TileLi
 // in the next substep: when its halo has moved less than P.reuse_max since its
 // lists were built, or, for a tile that did not carry, over the whole substep.
 template <int BITS, bool XSPH, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest omega_tile(const DevParams& P, uint32_t blk, const NeighbourList& L,
+__device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L,
                                            const float4* __restrict__ Q, const float4* __restrict__ VS,
                                            const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cs,
                                            const uint32_t* __restrict__ ce, float4* __restrict__ OM,
@@ -1050,8 +1084,15 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, uint32_t blk,
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  uint32_t key = 0u;  // of the thread's next particle, and its velocity
+  float4 v4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
+    if (g0 + tid < g1) {
+      key = keys[g0 + tid];
+      v4 = VS[g0 + tid];
+    }
+  });
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) L.cnt[g] = kNlInvalid;
@@ -1075,9 +1116,13 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, uint32_t blk,
   }
   uint32_t round = 0u;
   for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
+    if (round) {
+      key = keys[g];
+      v4 = VS[g];
+    }
     int h;
     uint32_t slot;
-    tile_locate<BITS>(sh, keys[g], g, h, slot);
+    tile_locate<BITS>(sh, key, g, h, slot);
     // kept lists: a particle without one is over the cap (global path, as when
     // the list was built) or has a long list (stencil scan)
     uint32_t n = keep ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
@@ -1092,7 +1137,6 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, uint32_t blk,
     const float4 qi = s_q[slot];
     // velocity components as scalars (a float4 aggregate captured by the pair
     // lambda is not promoted to registers)
-    const float4 v4 = VS[g];
     const float vx = v4.x, vy = v4.y, vz = v4.z, vw = v4.w;
     OmegaAcc a;
     FinalAcc xa;
@@ -1122,7 +1166,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, uint32_t blk,
       L.cnt[g] = (uint16_t)n;
       if (n == kNlInvalid) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_LONG], 1ull);
     }
-    if (n != kNlInvalid) nl_visit(L, g, n, pair);
+    if (n != kNlInvalid) nl_visit(L, g, n, L.nl[g], pair);
     else tile_stencil<BITS>(sh, h, slot, pair);
     OM[g] = omega_finish<VAR>(P, a);
     if (XSPH) {
@@ -1152,11 +1196,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_omega(DevParams P, TileLi
     if (mode == 0) break;
     TileRest rest;
     if (mode == 1) {
-      rest = omega_tile<BITS, XSPH, PH, TeamBlock, TileCap<BITS>::value>(P, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
+      rest = omega_tile<BITS, XSPH, PH, TeamBlock, TileCap<BITS>::value>(P, T, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
                                                                      lds.big.sh, lds.big.q, lds.big.gi);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = omega_tile<BITS, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
+      rest = omega_tile<BITS, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
                                                                     reg.sh, reg.q, reg.gi);
     }
     rest.visit([&](uint32_t g) __attribute__((always_inline)) {
@@ -1169,7 +1213,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_omega(DevParams P, TileLi
 }
 
 template <int BITS, bool VORT, bool XSPH, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest final_tile(const DevParams& P, uint32_t blk, const NeighbourList& L, int use_list,
+__device__ __forceinline__ TileRest final_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L, int use_list,
                                            uint32_t flags, const float4* __restrict__ Q,
                                            const float4* __restrict__ QX, const float4* __restrict__ VS,
                                            const float4* __restrict__ OM, const uint32_t* __restrict__ keys,
@@ -1180,8 +1224,20 @@ __device__ __forceinline__ TileRest final_tile(const DevParams& P, uint32_t blk,
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t total = tile_setup<BITS, Team>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  // the thread's next particle: its key, list length and first chunk
+  uint32_t key = 0u, n = kNlInvalid;
+  uint4 chunk = make_uint4(0u, 0u, 0u, 0u);
+  const auto next = [&](uint32_t g) __attribute__((always_inline)) {
+    key = keys[g];
+    if (use_list) {
+      n = L.cnt[g];
+      chunk = L.nl[g];
+    }
+  };
+  const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
+    if (g0 + tid < g1) next(g0 + tid);
+  });
   constexpr bool vort = VORT, xsph = XSPH;  // flags & FF_VORT, flags & FF_XSPH
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
@@ -1195,11 +1251,10 @@ __device__ __forceinline__ TileRest final_tile(const DevParams& P, uint32_t blk,
   uint32_t round = 0u;
   for (uint32_t g = g0 + tid; g < g1; g += Team::kSize, ++round) {
     if (PH) P.ph[g] = P.phs[g];  // phases follow the particles into the sorted order
-    const uint32_t key = keys[g];
+    if (round) next(g);
     int h;
     uint32_t slot;
     tile_locate<BITS>(sh, key, g, h, slot);
-    const uint32_t n = use_list ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
     // with phases, a particle without a list takes the global path (the tile holds
     // no phases for a scan)
     if (n == kNlInvalid && (PH || tile_count<BITS>(sh, h) > P.cap)) {
@@ -1222,7 +1277,7 @@ __device__ __forceinline__ TileRest final_tile(const DevParams& P, uint32_t blk,
         final_pair_textbook<VAR>(P, vort, xsph, qb.x - qj.x, qb.y - qj.y, qb.z - qj.z, make_float4(vx, vy, vz, vw),
                                  vj, oi.w, qj.w, a);
       };
-      if (n != kNlInvalid) nl_visit(L, g, n, pair);
+      if (n != kNlInvalid) nl_visit(L, g, n, chunk, pair);
       else tile_stencil<BITS>(sh, h, slot, pair);
     }
     const uint32_t sc = scene_of_key(P, key);
@@ -1253,11 +1308,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_final(
     TileRest rest;
     if (mode == 1) {
       rest = final_tile<BITS, VORT, XSPH, PH, TeamBlock, TileCap<BITS>::value>(
-          P, blk, L, use_list, flags, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo, lds.big.sh, lds.big.q,
+          P, T, blk, L, use_list, flags, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo, lds.big.sh, lds.big.q,
           lds.big.gi);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = final_tile<BITS, VORT, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, blk, L, use_list, flags, Q, QX, VS, OM,
+      rest = final_tile<BITS, VORT, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, use_list, flags, Q, QX, VS, OM,
                                                                           keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo,
                                                                           reg.sh, reg.q, reg.gi);
     }
@@ -1309,8 +1364,9 @@ __device__ __forceinline__ uint32_t quad_get(uint32_t x) {
 
 // The block of work item r (every occupied block is a large one).
 __device__ __forceinline__ bool wide_pick(const TileList& T, uint32_t r, uint32_t& blk) {
+  const uint32_t large = T.large[min(r, T.cap - 1u)];  // with the count, not after it
   if (r >= T.count[0]) return false;
-  blk = T.large[r];
+  blk = large;
   return true;
 }
 
@@ -1424,8 +1480,11 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
   if (!wide_pick(T, blockIdx.x, blk)) return;
   TileShared<5>& sh = lds.sh;
   const uint32_t tid = threadIdx.x, sub = tid % kQuad;
-  const uint32_t total = tile_setup<5, TeamWide>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk], gf = g0 + tid / kQuad;
+  uint32_t key = 0u;  // of the quad's next particle
+  const uint32_t total = tile_setup<5, TeamWide, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
+    if (gf < g1) key = keys[gf];
+  });
   TileRest rest = wide_rest(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += kWideThreads) L.cnt[g] = kNlInvalid;
@@ -1447,10 +1506,11 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
     }
     uint16_t* list = lds.list[tid / kQuad];
     uint32_t round = 0u;
-    for (uint32_t g = g0 + tid / kQuad; g < g1; g += kWideParticles, ++round) {
+    for (uint32_t g = gf; g < g1; g += kWideParticles, ++round) {
+      if (round) key = keys[g];
       int h;
       uint32_t slot;
-      tile_locate<5>(sh, keys[g], g, h, slot);
+      tile_locate<5>(sh, key, g, h, slot);
       uint32_t cnt = 0u, n = keep ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
       if (!keep || n == kNlInvalid) {
         cnt = tile_count<5>(sh, h);
@@ -1510,7 +1570,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
       }
       if (sub != 0u) continue;
       float W;
-      lam[g] = lambda_finish_fused(P, a, W, scene_eps(P, keys[g]));
+      lam[g] = lambda_finish_fused(P, a, W, scene_eps(P, key));
       if (FIRST) {
         dens[g] = W;
         ncnt[g] = cnt;
@@ -1539,8 +1599,15 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
   if (!wide_pick(T, blockIdx.x, blk)) return;
   TileShared<5>& sh = lds.sh;
   const uint32_t tid = threadIdx.x, sub = tid % kQuad;
-  const uint32_t total = tile_setup<5, TeamWide>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
+  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk], gf = g0 + tid / kQuad;
+  uint32_t key = 0u;  // of the quad's next particle, and its velocity
+  float4 v4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const uint32_t total = tile_setup<5, TeamWide, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
+    if (gf < g1) {
+      key = keys[gf];
+      v4 = VS[gf];
+    }
+  });
   TileRest rest = wide_rest(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += kWideThreads) L.cnt[g] = kNlInvalid;
@@ -1563,10 +1630,14 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
     }
     uint16_t* list = lds.list[tid / kQuad];
     uint32_t round = 0u;
-    for (uint32_t g = g0 + tid / kQuad; g < g1; g += kWideParticles, ++round) {
+    for (uint32_t g = gf; g < g1; g += kWideParticles, ++round) {
+      if (round) {
+        key = keys[g];
+        v4 = VS[g];
+      }
       int h;
       uint32_t slot;
-      tile_locate<5>(sh, keys[g], g, h, slot);
+      tile_locate<5>(sh, key, g, h, slot);
       uint32_t n = keep ? (uint32_t)L.cnt[g] : (uint32_t)kNlInvalid;
       if (n == kNlInvalid && tile_count<5>(sh, h) > P.cap) {
         if (sub == 0u) {
@@ -1579,7 +1650,6 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
         continue;
       }
       const float4 qi = lds.q[slot];
-      const float4 v4 = VS[g];
       const float vx = v4.x, vy = v4.y, vz = v4.z, vw = v4.w;
       if (!keep) {
         n = wide_build(L, g, sh, lds.q, list, h, slot, qi, P.list_r2);

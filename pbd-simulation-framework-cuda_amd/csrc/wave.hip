@@ -265,7 +265,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_wave_delta(
     A.py = __shfl(a, (int)C + 1);
     A.pz = __shfl(a, (int)C + 2);
   }
-  if (lane == 0u) delta_finish<REF, DELTA>(P, flags, s, q, QX, A, f.cx, f.cy, f.cz, keys[s], Qo, QXo, DP, VS);
+  if (lane == 0u) delta_finish<REF, DELTA>(P, flags, s, q, QX[s], A, f.cx, f.cy, f.cz, keys[s], Qo, QXo, DP, VS);
 }
 
 __global__ __launch_bounds__(64 * kWaves) void k_wave_omega(DevParams P, const float4* __restrict__ Q,
