@@ -328,7 +328,8 @@ contacts_done:
   return cnt;
 }
 
-// A NaN as the positive quiet NaN (the tile lists read the sign of a distance test).
+// A NaN as the positive quiet NaN, for every position that a tile list may be built from
+// (the lists read the sign of a distance test, and an operation's own NaN is negative).
 __device__ __forceinline__ float canonical_nan(float x) { return x == x ? x : __uint_as_float(0x7FC00000u); }
 
 // ---------------------------------------------------------------------------

@@ -335,8 +335,9 @@ __global__ void k_batch_solve(DevParams P, float4* __restrict__ Q, float4* __res
   if (half > 0.0f && len > 0.00001f) {
     // both move half the overlap times (1 - stiffness); coll_scale = -(1 - stiffness) / 2
     const float m = -2.0f * P.coll_scale * half / len;
-    Q[s] = make_float4(qs.x - m * dx, qs.y - m * dy, qs.z - m * dz, 0.0f);  // p* is written back with w = 0
-    Q[j] = make_float4(qj.x + m * dx, qj.y + m * dy, qj.z + m * dz, 0.0f);
+    // p* is written back with w = 0
+    Q[s] = make_float4(canonical_nan(qs.x - m * dx), canonical_nan(qs.y - m * dy), canonical_nan(qs.z - m * dz), 0.0f);
+    Q[j] = make_float4(canonical_nan(qj.x + m * dx), canonical_nan(qj.y + m * dy), canonical_nan(qj.z + m * dz), 0.0f);
     const float4 xs = QX[s], xj = QX[j];
     QX[s] = make_float4(xs.x - m * dx, xs.y - m * dy, xs.z - m * dz, xs.w);
     QX[j] = make_float4(xj.x + m * dx, xj.y + m * dy, xj.z + m * dz, xj.w);

@@ -143,7 +143,7 @@ hipError_t launch_collide_batches(hipStream_t st, uint32_t tpb, const DevParams&
                                   uint32_t words, unsigned long long* minc, uint32_t* partner);
 // The wide lambda and omega passes (tiles.hip): four lanes per particle, for scenes whose
 // blocks do not fill the chip.  Measured (us a step, four lanes / one lane in these two
-// passes; columns at rest keep their lists, splashes rebuild them in every pass): 2K
+// passes; every pass builds its lists, a splash's from crowded cells): 2K
 // column 230 / 254, 32K column 251 / 263, 30K splash 281 / 379, 64K column 287 / 286, 64K
 // splash 381 / 422; 125K column 405 / 328, 125K splash 455 / 462.  The other passes walk
 // kept lists, and a 32K scene's take 11.1 us (delta p) and 9.6 (final) with four lanes,

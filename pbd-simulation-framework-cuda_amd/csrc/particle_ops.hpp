@@ -181,7 +181,7 @@ __device__ __forceinline__ float4 delta_finish(const DevParams& P, uint32_t flag
     VS[s] = make_float4((nx - qx.x) / P.dt, (ny - qx.y) / P.dt, (nz - qx.z) / P.dt, (qi.w - qx.w) / P.dt);
     qx = make_float4(nx, ny, nz, qi.w);
   }
-  const float4 q = make_float4(nx, ny, nz, qi.w);
+  const float4 q = make_float4(canonical_nan(nx), canonical_nan(ny), canonical_nan(nz), qi.w);
   Qo[s] = q;
   QXo[s] = qx;
   return q;

@@ -688,7 +688,7 @@ __device__ __forceinline__ void nl_visit(const NeighbourList& L, uint32_t g, uin
 // much, by the LDS; 1M dam break: 152 -> 122 us, with the 16-byte reads of slot_read.  Unrolled by kScanUnroll: a group may read up to kScanUnroll - 1 slots
 // past the range (still inside the LDS array); their bits are masked off.  A position
 // that is not a number is +NaN (canonical_nan), whose sign says out of range; the
-// caller drops the mask of a particle that is itself none.
+// caller drops the mask of a particle that is not finite itself (inf - inf is -NaN).
 __device__ __forceinline__ uint32_t nl_mask(const float4* s_q, uint32_t a, uint32_t len, float qx, float qy, float qz,
                                             float r2max) {
   constexpr uint32_t U = kScanUnroll;
@@ -773,8 +773,7 @@ __device__ __forceinline__ uint32_t nl_build(const DevParams& P, const Neighbour
                                              const TileShared<BITS>& sh, const float4* s_q, int h, uint32_t slot,
                                              float4 qi, float r2) {
   using G = TileGeom<BITS>;
-  const float nan = qi.x + qi.y + qi.z;
-  const uint32_t valid = nan == nan ? 0xFFFFFFFFu : 0u;
+  const uint32_t valid = fabsf(qi.x) + fabsf(qi.y) + fabsf(qi.z) < __builtin_inff() ? 0xFFFFFFFFu : 0u;
   uint32_t n = 0;
   ChunkWriter cw(L, g);
 #pragma unroll 1
@@ -1391,8 +1390,7 @@ __device__ __forceinline__ uint32_t wide_build(const NeighbourList& L, uint32_t 
   using G = TileGeom<5>;
   constexpr uint32_t CAP = TileCap<5>::value;
   const uint32_t sub = threadIdx.x % kQuad;
-  const float nan = qi.x + qi.y + qi.z;
-  const uint32_t valid = nan == nan ? 0xFFFFFFFFu : 0u;
+  const uint32_t valid = fabsf(qi.x) + fabsf(qi.y) + fabsf(qi.z) < __builtin_inff() ? 0xFFFFFFFFu : 0u;
   const auto scan = [&](uint32_t s, uint32_t b) __attribute__((always_inline)) {
     uint32_t m = nl_mask(s_q, s, min(b - s, 32u), qi.x, qi.y, qi.z, r2) & valid;
     if (slot - s < 32u) m &= ~(1u << (slot - s));  // not the particle itself
@@ -1948,8 +1946,7 @@ __device__ __forceinline__ void tally_flush(const uint32_t* t, unsigned long lon
 // In-range bits (lo, hi) of slots a .. b - 1 (1 <= b - a <= 64).
 __device__ __forceinline__ void nl_column(const float4* s_q, uint32_t a, uint32_t b, float4 q, float r2max,
                                           uint32_t& lo, uint32_t& hi) {
-  const float nan = q.x + q.y + q.z;
-  const uint32_t valid = nan == nan ? 0xFFFFFFFFu : 0u;
+  const uint32_t valid = fabsf(q.x) + fabsf(q.y) + fabsf(q.z) < __builtin_inff() ? 0xFFFFFFFFu : 0u;
   const uint32_t len = b - a;
   lo = nl_mask(s_q, a, min(len, 32u), q.x, q.y, q.z, r2max) & valid;
   hi = len > 32u ? nl_mask(s_q, a + 32u, len - 32u, q.x, q.y, q.z, r2max) & valid : 0u;

@@ -79,3 +79,28 @@ def test_gpu_tile_lists_leave_nan_neighbours_out(F):
     ref, got = step([]), step([[nan, 0.05, 0.05, 1.0], [0.05, -nan, 0.05, 1.0], [-nan, -nan, -nan, 1.0]])
     for k in ref:
         assert np.array_equal(ref[k], got[k]), k
+
+
+def test_gpu_tile_lists_leave_nan_neighbours_out_of_later_passes(F):
+    """The same for the passes that follow a delta p pass, with its moves not applied (an
+    applied one puts the particle onto the enclosure)."""
+    p, x = _crowded(F, (6, 8))
+    p.solver_iterations = 3
+    p.stabilization_iterations = 1
+    p.active_apply_delta_positions = 0
+    n = x.shape[0]
+
+    def step(extra):
+        ctx = F.Context(p, n + len(extra))
+        ctx.add_particles(np.concatenate([x, np.array(extra, np.float32).reshape(-1, 4)]))
+        ctx.compute()
+        keep = ctx.download("particle_ids") < n
+        out = {k: ctx.download(k)[keep] for k in ("densities", "lambdas", "positions", "omegas")}
+        ctx.close()
+        return out
+
+    nan = np.float32(np.nan)
+    print("NaN neighbours, later passes", flush=True)
+    ref, got = step([]), step([[nan, 0.05, 0.05, 1.0], [0.05, -nan, 0.05, 1.0], [-nan, -nan, -nan, 1.0]])
+    for k in ref:
+        assert np.array_equal(ref[k], got[k]), k
