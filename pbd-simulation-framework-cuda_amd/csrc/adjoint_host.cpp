@@ -191,8 +191,10 @@ int Fluid::adj_forward(uint32_t frames, uint32_t k_ckpt) {
   A.ids_cur = 0;
   auto save = [&](uint32_t g) {
     float4* dst = A.ckpt[g];
-    return tape_copy(dst, B_.X, n * 16) || tape_copy(dst + n, B_.V, n * 16) || tape_copy(dst + 2 * n, B_.F, n * 16) ||
-           (A.phased && tape_copy(A.ckpt_ph[g], ph_, n * 4));
+    CopySet set;
+    set.add(dst, B_.X, n * 16).add(dst + n, B_.V, n * 16).add(dst + 2 * n, B_.F, n * 16);
+    if (A.phased) set.add(A.ckpt_ph[g], ph_, n * 4);
+    return tape_copy(set);
   };
   if (save(0)) return status_;
   if (int rc = ensure_graph()) return rc;
@@ -217,10 +219,11 @@ int Fluid::adj_forward(uint32_t frames, uint32_t k_ckpt) {
   }
   A.tail_recorded = true;
   float4* fs = A.final_state;
-  if (tape_copy(fs, B_.X, n * 16) || tape_copy(fs + n, B_.P, n * 16) || tape_copy(fs + 2 * n, B_.V, n * 16) ||
-      tape_copy(fs + 3 * n, B_.C, n * 16) || tape_copy(fs + 4 * n, B_.F, n * 16) ||
-      (A.phased && tape_copy(A.final_ph, ph_, n * 4)))
-    return status_;
+  CopySet set;
+  set.add(fs, B_.X, n * 16).add(fs + n, B_.P, n * 16).add(fs + 2 * n, B_.V, n * 16);
+  set.add(fs + 3 * n, B_.C, n * 16).add(fs + 4 * n, B_.F, n * 16);
+  if (A.phased) set.add(A.final_ph, ph_, n * 4);
+  if (tape_copy(set)) return status_;
   A.valid = true;
   return PBD_OK;
 }
@@ -250,22 +253,21 @@ int Fluid::adj_backward(const float* gx, const float* gv, float* gv0, float* grh
     return hipMemcpyAsync(dst, stage, n * 16, hipMemcpyHostToDevice, stream_);
   };
   if (gx) e = upload(W.GX, gx, pin);
-  else e = hipMemsetAsync(W.GX, 0, n * 16, stream_);
-  if (e == hipSuccess) {
-    if (gv) e = upload(W.GV, gv, pin ? pin + n : nullptr);
-    else e = hipMemsetAsync(W.GV, 0, n * 16, stream_);
-  }
-  if (e == hipSuccess) e = hipMemsetAsync(W.GF, 0, n * 16, stream_);
-  if (e == hipSuccess) e = hipMemsetAsync(W.acc, 0, n * sizeof(double2), stream_);
-  if (e == hipSuccess) e = hipMemsetAsync(W.flag, 0, 4, stream_);
+  if (e == hipSuccess && gv) e = upload(W.GV, gv, pin ? pin + n : nullptr);
+  CopySet zero;
+  if (!gx) zero.add(W.GX, nullptr, n * 16);
+  if (!gv) zero.add(W.GV, nullptr, n * 16);
+  zero.add(W.GF, nullptr, n * 16).add(W.acc, nullptr, n * sizeof(double2)).add(W.flag, nullptr, 4);
+  if (e == hipSuccess) e = launch_copy_set(stream_, zero);
   if (hip_check(e, "adjoint: upload of the loss adjoints")) return status_;
   for (uint32_t g = A.nseg; g-- > 0;) {
     const uint32_t nstep = (std::min(A.frames, (g + 1) * A.k) - g * A.k) * A.sub;
     if (g + 1 < A.nseg || !A.tail_recorded) {
       const float4* c = A.ckpt[g];
-      if (tape_copy(B_.X, c, n * 16) || tape_copy(B_.V, c + n, n * 16) || tape_copy(B_.F, c + 2 * n, n * 16) ||
-          (A.phased && tape_copy(ph_, A.ckpt_ph[g], n * 4)))
-        return status_;
+      CopySet set;
+      set.add(B_.X, c, n * 16).add(B_.V, c + n, n * 16).add(B_.F, c + 2 * n, n * 16);
+      if (A.phased) set.add(ph_, A.ckpt_ph[g], n * 4);
+      if (tape_copy(set)) return status_;
       for (uint32_t t = 0; t < nstep; ++t) {
         rec_ = &A.tape[t];
         compute();
@@ -289,12 +291,11 @@ int Fluid::adj_backward(const float* gx, const float* gv, float* gv0, float* grh
     e = hipMemcpyAsync(pin ? (void*)(pin + 3 * n) : (void*)gx0, W.GX, n * 16, hipMemcpyDeviceToHost, stream_);
   // leave the context as pbd_adj_forward left it
   const float4* fs = A.final_state;
-  if (e == hipSuccess) e = hipMemcpyAsync(B_.X, fs, n * 16, hipMemcpyDeviceToDevice, stream_);
-  if (e == hipSuccess) e = hipMemcpyAsync(B_.P, fs + n, n * 16, hipMemcpyDeviceToDevice, stream_);
-  if (e == hipSuccess) e = hipMemcpyAsync(B_.V, fs + 2 * n, n * 16, hipMemcpyDeviceToDevice, stream_);
-  if (e == hipSuccess) e = hipMemcpyAsync(B_.C, fs + 3 * n, n * 16, hipMemcpyDeviceToDevice, stream_);
-  if (e == hipSuccess) e = hipMemcpyAsync(B_.F, fs + 4 * n, n * 16, hipMemcpyDeviceToDevice, stream_);
-  if (e == hipSuccess && A.phased) e = hipMemcpyAsync(ph_, A.final_ph, n * 4, hipMemcpyDeviceToDevice, stream_);
+  CopySet set;
+  set.add(B_.X, fs, n * 16).add(B_.P, fs + n, n * 16).add(B_.V, fs + 2 * n, n * 16);
+  set.add(B_.C, fs + 3 * n, n * 16).add(B_.F, fs + 4 * n, n * 16);
+  if (A.phased) set.add(ph_, A.final_ph, n * 4);
+  if (e == hipSuccess) e = launch_copy_set(stream_, set);
   if (e == hipSuccess) e = hipStreamSynchronize(stream_);
   if (hip_check(e, "adjoint: results")) return status_;
   if (pin && gv0) std::memcpy(gv0, pin + 2 * n, n * 16);

@@ -234,11 +234,10 @@ int Fluid::compute_in_place(const pbd_params& p, uint32_t n, float4* X, float4* 
   B_.C = C;
   B_.F = F;
   if (n == 0) return PBD_OK;
-  hipError_t e = launch_fill_u32(st, reinterpret_cast<uint32_t*>(B_.LAM), 0u, n);
-  if (e == hipSuccess) e = launch_fill_u32(st, reinterpret_cast<uint32_t*>(B_.DENS), 0u, n);
-  if (e == hipSuccess) e = launch_fill_u32(st, reinterpret_cast<uint32_t*>(B_.DP), 0u, 4u * n);
-  if (e == hipSuccess) e = launch_fill_u32(st, reinterpret_cast<uint32_t*>(B_.OM), 0u, 4u * n);
-  if (e == hipSuccess) e = launch_fill_u32(st, sort_.err, 0u, 1u);
+  CopySet zero;  // one launch: as five they took 9 us of a small scene's step
+  zero.add(B_.LAM, nullptr, (size_t)n * 4).add(B_.DENS, nullptr, (size_t)n * 4);
+  zero.add(B_.DP, nullptr, (size_t)n * 16).add(B_.OM, nullptr, (size_t)n * 16).add(sort_.err, nullptr, 4);
+  const hipError_t e = launch_copy_set(st, zero);
   if (hip_check(e, "clearing the region")) return status_;
   compute();
   return status_;
@@ -495,10 +494,6 @@ int Fluid::enqueue_substep() {
                      !(params_.collision_type == 1 && params_.stabilization_iterations > 0) &&
                      params_.solver_iterations > 0 && params_.solver_iterations <= kCarryPasses;
   const size_t n16 = (size_t)P.n * 16, n4 = (size_t)P.n * 4;
-  if (rec_) {  // the step's input state, for the reverse of the predict stage
-    if (tape_copy(rec_->Xin, B_.X, n16) || tape_copy(rec_->Vin, B_.V, n16) || tape_copy(rec_->Fin, B_.F, n16))
-      return status_;
-  }
   // the sort's histogram, tickets and look-back words start at zero
   PBD_LAUNCH(ST_SORT, launch_sort_prepare(st, sort_, P.n));
   // 1-2. applyForces + initializeCellIds (Fluid.cu:21-25), with the sort's digit counts
@@ -509,28 +504,40 @@ int Fluid::enqueue_substep() {
   // 3. sortIds (Fluid.cu:27)
   PBD_LAUNCH(ST_SORT, launch_sort_ranks(st, sort_, P.n, B_.keys_in, &keys_sorted_, &ids_sorted_));
   // 4-5. reorderStorage + computeCellInfo (Fluid.cu:29,33)
-  PBD_LAUNCH(ST_REORDER, launch_reorder(st, tpb, P, B_, keys_sorted_, ids_sorted_, tiles ? (uint32_t)bits : 0u,
+  // Where a recorded step's delta-p passes write whole new positions, they write them (and
+  // x, and the lambdas) to the record instead of to buffers that are copied there.
+  const uint32_t S = params_.stabilization_iterations;
+  const uint32_t iters = params_.solver_iterations;
+  const bool batched = params_.collision_type == 1 && S > 0;
+  const bool direct = rec_ && (g & G_DELTA) && !batched && iters > 0;
+  float4* Q = direct ? rec_->Q : B_.Q[0];
+  float4* QX = direct && rec_->QX ? rec_->QX : B_.QX[0];
+  StepBuffers sorted = B_;
+  sorted.Q[0] = Q;
+  sorted.QX[0] = QX;
+  PBD_LAUNCH(ST_REORDER, launch_reorder(st, tpb, P, sorted, keys_sorted_, ids_sorted_, tiles ? (uint32_t)bits : 0u,
                                         tile_flag_, tile_end_));
   if (tiles)
     PBD_LAUNCH(ST_TILES, launch_tile_compact(st, ntiles, tile_flag_, tile_end_, small_max(), tile_bcount_, tile_list_,
                                              tile_list_ + cap_, tile_count_));
   const uint32_t* keys = keys_sorted_;
   if (rec_) {
+    // the step's input state (for the reverse of the predict stage; nothing has written to
+    // it yet), its order and its cells
     const size_t tb = (size_t)B_.table_size * 4;
-    if (tape_copy(rec_->Q, B_.Q[0], n16) || tape_copy(rec_->keys, keys_sorted_, n4) ||
-        tape_copy(rec_->perm, ids_sorted_, n4) || tape_copy(rec_->cs, B_.cstart, tb) || tape_copy(rec_->ce, B_.cend, tb))
-      return status_;
-    if (rec_->PH && tape_copy(rec_->PH, phs_, n4)) return status_;  // the step's phases, sorted
+    CopySet set;
+    set.add(rec_->Xin, B_.X, n16).add(rec_->Vin, B_.V, n16).add(rec_->Fin, B_.F, n16);
+    set.add(rec_->keys, keys_sorted_, n4).add(rec_->perm, ids_sorted_, n4);
+    set.add(rec_->cs, B_.cstart, tb).add(rec_->ce, B_.cend, tb);
+    if (rec_->PH) set.add(rec_->PH, phs_, n4);  // the step's phases, sorted
+    if (!direct) set.add(rec_->Q, Q, n16);
+    if (tape_copy(set)) return status_;
   }
 
   // 6-7. solver loop (Fluid.cu:49-80); contacts/neighbours are walked inside the passes
   const bool lambda_on = g & G_LAMBDA, delta_on = g & G_DELTA, apply_on = g & G_APPLY_DELTA;
   const bool update_on = g & G_UPDATE;
-  const uint32_t S = params_.stabilization_iterations;
-  const uint32_t iters = params_.solver_iterations;
-  int cur = 0;
   bool counted = false, updated = false;
-  const bool batched = params_.collision_type == 1 && S > 0;
   if (batched) {
     // allocated ahead of any capture (ensure_graph); the eager path allocates on first use
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -543,21 +550,25 @@ int Fluid::enqueue_substep() {
   }
   for (uint32_t it = 0; it < iters; ++it) {
     const bool last_it = it + 1 == iters;
-    bool listed = false;  // the lambda pass left the neighbour lists of Q[cur]
+    bool listed = false;  // the lambda pass left the neighbour lists of Q
     // x at the iteration's start, for the reverse of the friction
-    if (rec_ && rec_->QX && tape_copy(rec_->QX + (size_t)it * P.n, B_.QX[cur], n16)) return status_;
+    if (rec_ && rec_->QX && !direct && tape_copy(CopySet().add(rec_->QX + (size_t)it * P.n, QX, n16))) return status_;
+    // the last iteration's lambdas stay in the context's buffer too
+    const bool lam_direct = direct && !last_it && lambda_on;
+    StepBuffers B = list_set(it);
+    if (lam_direct) B.LAM = rec_->LAM + (size_t)it * P.n;
     if (lambda_on) {
       if (tiles) {
         PBD_LAUNCH(carry && counted ? ST_LAMBDA_CARRY : ST_LAMBDA,
-                   wide ? launch_wide_lambda(st, wgrid, P, TL, list_set(it), B_.Q[cur], keys, !counted, carry, it)
-                        : launch_tile_lambda(st, bits, tgrid, tstride, P, TL, list_set(it), B_.Q[cur], keys, !counted, carry,
+                   wide ? launch_wide_lambda(st, wgrid, P, TL, B, Q, keys, !counted, carry, it)
+                        : launch_tile_lambda(st, bits, tgrid, tstride, P, TL, B, Q, keys, !counted, carry,
                                       it));
         listed = true;
       } else {
-        PBD_LAUNCH(ST_LAMBDA, launch_lambda(st, tpb, P, B_, B_.Q[cur], keys, !counted));
+        PBD_LAUNCH(ST_LAMBDA, launch_lambda(st, tpb, P, B, Q, keys, !counted));
       }
       counted = true;
-      if (rec_ && tape_copy(rec_->LAM + (size_t)it * P.n, B_.LAM, n4)) return status_;
+      if (rec_ && !lam_direct && tape_copy(CopySet().add(rec_->LAM + (size_t)it * P.n, B_.LAM, n4))) return status_;
     }
     // the Q-writing kernels of this iteration
     struct K {
@@ -586,7 +597,7 @@ int Fluid::enqueue_substep() {
     }
     for (uint32_t k = 0; k < nk; ++k) {
       if (ks[k].batches) {
-        PBD_LAUNCH(ST_COLLIDE, launch_collide_batches(st, tpb, P, B_, B_.Q[cur], B_.QX[cur], keys,
+        PBD_LAUNCH(ST_COLLIDE, launch_collide_batches(st, tpb, P, B_, Q, QX, keys,
                                                       params_.max_collision_batches, batch_solved_, batch_words_,
                                                       batch_min_, batch_partner_));
         continue;
@@ -597,51 +608,51 @@ int Fluid::enqueue_substep() {
         updated = true;
       }
       const int stage = ks[k].delta ? ST_DELTA : ST_COLLIDE;
+      const bool to_rec = direct && k + 1 == nk;
+      float4* Qo = to_rec ? rec_->Q + (size_t)(it + 1) * P.n : B_.Q[Q == B_.Q[0] ? 1 : 0];
+      float4* QXo = to_rec && rec_->QX && !last_it ? rec_->QX + (size_t)(it + 1) * P.n : B_.QX[QX == B_.QX[0] ? 1 : 0];
       if (tiles && ks[k].delta) {
-        PBD_LAUNCH(stage, launch_tile_delta(st, bits, tgrid, tstride, P, TL, list_set(it), fl, ks[k].collide,
-                                            listed && k == 0,
-                                            B_.Q[cur], B_.QX[cur], B_.Q[1 - cur], B_.QX[1 - cur], keys,
-                                            carry ? it + 1u : 0u));
+        PBD_LAUNCH(stage, launch_tile_delta(st, bits, tgrid, tstride, P, TL, B, fl, ks[k].collide, listed && k == 0, Q, QX,
+                                            Qo, QXo, keys, carry ? it + 1u : 0u));
       } else {
-        PBD_LAUNCH(stage, launch_delta(st, tpb, P, B_, fl, ks[k].delta, ks[k].collide, B_.Q[cur], B_.QX[cur],
-                                       B_.Q[1 - cur], B_.QX[1 - cur], keys));
+        PBD_LAUNCH(stage, launch_delta(st, tpb, P, B, fl, ks[k].delta, ks[k].collide, Q, QX, Qo, QXo, keys));
       }
-      cur = 1 - cur;
+      Q = Qo;
+      QX = QXo;
     }
-    if (rec_ && tape_copy(rec_->Q + (size_t)(it + 1) * P.n, B_.Q[cur], n16)) return status_;
+    if (rec_ && !direct && tape_copy(CopySet().add(rec_->Q + (size_t)(it + 1) * P.n, Q, n16))) return status_;
   }
   if (!counted) PBD_LAUNCH(ST_COUNT, launch_count(st, tpb, P, B_, keys));
   // 8. updatePositions (Fluid.cu:82-84) when not fused into the last solver pass
   if (update_on && !updated) {
-    PBD_LAUNCH(ST_UPDATE, launch_update(st, tpb, P, B_, B_.Q[cur], B_.QX[cur]));
+    PBD_LAUNCH(ST_UPDATE, launch_update(st, tpb, P, B_, Q, QX));
     updated = true;
   }
   // 9. computeOmega (Fluid.cu:86-88)
-  const bool omega_listed = tiles && (g & G_OMEGA);  // the omega pass leaves the lists of Q[cur]
+  const bool omega_listed = tiles && (g & G_OMEGA);  // the omega pass leaves the lists of Q
   // the tile omega pass also applies XSPH: it walks the same neighbours with their velocities
   const bool xsph_in_omega = omega_listed && (g & G_VISCOSITY);
   if (g & G_OMEGA) {
     if (tiles) {
       PBD_LAUNCH(ST_OMEGA,
-                 wide ? launch_wide_omega(st, wgrid, P, TL, list_set(iters), B_.Q[cur], keys, xsph_in_omega,
+                 wide ? launch_wide_omega(st, wgrid, P, TL, list_set(iters), Q, keys, xsph_in_omega,
                                           carry ? iters : 0u)
-                      : launch_tile_omega(st, bits, tgrid, tstride, P, TL, list_set(iters), B_.Q[cur], keys, xsph_in_omega,
+                      : launch_tile_omega(st, bits, tgrid, tstride, P, TL, list_set(iters), Q, keys, xsph_in_omega,
                                    carry ? iters : 0u));
     } else {
-      PBD_LAUNCH(ST_OMEGA, launch_omega(st, tpb, P, B_, B_.Q[cur], keys));
+      PBD_LAUNCH(ST_OMEGA, launch_omega(st, tpb, P, B_, Q, keys));
     }
   }
-  if (rec_ && (tape_copy(rec_->U, B_.VS, n16) || tape_copy(rec_->OM, B_.OM, n16))) return status_;
+  if (rec_ && tape_copy(CopySet().add(rec_->U, B_.VS, n16).add(rec_->OM, B_.OM, n16))) return status_;
   // 10-11. computeVorticity + computeViscosity (Fluid.cu:90-96) and the output
   uint32_t ff = 0;
   if (g & G_VORTICITY) ff |= FF_VORT;
   if (g & G_VISCOSITY) ff |= xsph_in_omega ? FF_XSPH_DONE : FF_XSPH;
   if (updated) ff |= FF_UPDATED;
   if (tiles)
-    PBD_LAUNCH(ST_FINAL, launch_tile_final(st, bits, tgrid, tstride, P, TL, list_set(iters), ff, omega_listed,
-                                           B_.Q[cur], B_.QX[cur], keys));
+    PBD_LAUNCH(ST_FINAL, launch_tile_final(st, bits, tgrid, tstride, P, TL, list_set(iters), ff, omega_listed, Q, QX, keys));
   else
-    PBD_LAUNCH(ST_FINAL, launch_final(st, tpb, P, B_, ff, B_.Q[cur], B_.QX[cur], keys));
+    PBD_LAUNCH(ST_FINAL, launch_final(st, tpb, P, B_, ff, Q, QX, keys));
   return PBD_OK;
 }
 
@@ -716,9 +727,7 @@ int Fluid::ensure_graph() {
   return PBD_OK;
 }
 
-int Fluid::tape_copy(void* dst, const void* src, size_t bytes) {
-  return hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, stream_), "adjoint record copy");
-}
+int Fluid::tape_copy(const CopySet& set) { return hip_check(launch_copy_set(stream_, set), "adjoint record copy"); }
 
 int Fluid::sync() {
   if (!stream_ || !sort_.err) return status_;  // not initialised: nothing queued

@@ -121,7 +121,7 @@ class Fluid : public Cuda_Computable {
   int ensure_graph();
   int adj_check();
   void adj_release();
-  int tape_copy(void* dst, const void* src, size_t bytes);
+  int tape_copy(const CopySet& set);
   void stage_begin(int stage);
   void stage_end(int stage);
   int collect_timings();

@@ -111,6 +111,21 @@ hipError_t launch_tile_compact(hipStream_t st, uint32_t nflags, const uint32_t* 
                                uint32_t* count);
 
 hipError_t launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, uint32_t n);
+// Several device arrays copied (src null: zeroed) by one launch; sizes are multiples of 4.
+struct CopySet {
+  static constexpr uint32_t kMax = 10;
+  void* dst[kMax];
+  const void* src[kMax];
+  size_t bytes[kMax];
+  uint32_t count = 0;
+  CopySet& add(void* d, const void* s, size_t b) {
+    dst[count] = d;
+    src[count] = s;
+    bytes[count++] = b;
+    return *this;
+  }
+};
+hipError_t launch_copy_set(hipStream_t st, const CopySet& c);
 // cstart[0, ts) = UINT_MAX, cend[0, ts) = n, flags[0, nflags) = 0 (flags may be null)
 hipError_t launch_cell_reset(hipStream_t st, uint32_t* cstart, uint32_t* cend, uint32_t ts, uint32_t n,
                              uint32_t* flags, uint32_t nflags);
