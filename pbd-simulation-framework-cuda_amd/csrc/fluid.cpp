@@ -21,6 +21,7 @@ Fluid::~Fluid() {
   }
   for (auto e : event_pool_) (void)hipEventDestroy(e);
   for (void* p : allocations_) (void)hipFree(p);
+  if (host_err_) (void)hipHostFree(host_err_);
   if (stream_ && owns_stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -121,7 +122,6 @@ int Fluid::init(const pbd_params& p, uint32_t capacity) {
     if (e == hipSuccess) e = hipMemsetAsync(q, 0, c * 16, stream_);
   for (void* q : {(void*)B_.LAM, (void*)B_.DENS, (void*)B_.NCNT, (void*)B_.CCNT, (void*)ph_, (void*)phs_})
     if (e == hipSuccess) e = hipMemsetAsync(q, 0, c * 4, stream_);
-  if (e == hipSuccess) e = hipMemsetAsync(sort_.err, 0, 4, stream_);
   if (e == hipSuccess) e = hipMemsetAsync(d_scratch_, 0, 16, stream_);
   if (e == hipSuccess) e = hipMemsetAsync(tile_count_, 0, 8, stream_);
   if (e == hipSuccess) e = hipMemsetAsync(B_.STATS, 0, PBD_COUNTER_COUNT * 8, stream_);
@@ -165,7 +165,15 @@ int Fluid::layout() {
   rc |= take(&sort_.hist, kSortHistWords);
   rc |= take(&sort_.tile_ctr, 4);
   rc |= take(&sort_.status, (size_t)4 * sort_.tiles_max * 256);
-  rc |= take(&sort_.err, 1);
+  if (region_) {
+    rc |= take(&sort_.err, 1);
+  } else {
+    // The sort's error flag lies in pinned host memory: kernels write it on failure only,
+    // and sync() reads it in place (a copy of 4 bytes took 10 us of every sync).
+    rc |= hipHostMalloc(reinterpret_cast<void**>(&host_err_), sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+          hipHostGetDevicePointer(reinterpret_cast<void**>(&sort_.err), host_err_, 0) != hipSuccess;
+    if (!rc) *host_err_ = 0u;
+  }
   rc |= take(&sort_.keys_alt, c);
   rc |= take(&sort_.vals_alt, c);
   rc |= take(&sort_.keys_out, c);
@@ -734,7 +742,8 @@ int Fluid::sync() {
   if (hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize")) return status_;
   if (timing_ || !pending_.empty()) collect_timings();
   uint32_t err = 0;
-  if (hip_check(hipMemcpy(&err, sort_.err, 4, hipMemcpyDeviceToHost), "read sort flag")) return status_;
+  if (host_err_) err = *static_cast<volatile uint32_t*>(host_err_);
+  else if (hip_check(hipMemcpy(&err, sort_.err, 4, hipMemcpyDeviceToHost), "read sort flag")) return status_;
   if (err) return fail(PBD_ERR_HIP, "sort look-back exceeded its spin limit");
   return status_;
 }

@@ -140,6 +140,7 @@ class Fluid : public Cuda_Computable {
   uint32_t small_max() const { return small_auto_ ? default_small_max(n_) : small_max_; }
   uint32_t stride_grid_ = kTileGridStride;  // workgroups of the capped tile grid
   uint32_t skin_pct_ = kListSkinPct;       // tile-list skin, percent of the list radius
+  uint32_t* host_err_ = nullptr;           // the sort's error flag (pinned), unless the context lies in a region
   bool tuned_ = false;                     // autotune ran (or a cached choice was applied)
   // a caller's region the buffers are carved from (init_in_place), else null
   unsigned char* region_ = nullptr;

@@ -225,7 +225,7 @@ struct SortPlan {
   uint32_t* hist;       // [4][256] exclusive digit offsets, then kSortHistCopies x [4][256] partial counts
   uint32_t* tile_ctr;   // [4] tile tickets
   uint32_t* status;     // [4][tiles_max][256] look-back words
-  uint32_t* err;        // look-back spin-limit flag
+  uint32_t* err;        // look-back spin-limit flag (device or pinned host memory)
   uint32_t* keys_alt;   // ping-pong buffers (n_max)
   uint32_t* vals_alt;
   uint32_t* keys_out;

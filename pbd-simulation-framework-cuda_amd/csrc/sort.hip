@@ -206,7 +206,8 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint32_t* __res
       t -= taken;
       if (taken == 0) {
         if (++spins > kSpinLimit) {
-          atomicOr(err, 1u);
+          // may be host memory: a plain store, the same from every wave
+          __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
           break;
         }
         __builtin_amdgcn_s_sleep(1);
