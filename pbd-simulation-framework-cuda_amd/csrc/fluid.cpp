@@ -526,7 +526,7 @@ int Fluid::enqueue_substep() {
   PBD_LAUNCH(ST_REORDER, launch_reorder(st, tpb, P, sorted, keys_sorted_, ids_sorted_, tiles ? (uint32_t)bits : 0u,
                                         tile_flag_, tile_end_));
   if (tiles)
-    PBD_LAUNCH(ST_TILES, launch_tile_compact(st, ntiles, tile_flag_, tile_end_, small_max(), tile_bcount_, tile_list_,
+    PBD_LAUNCH(ST_TILES, launch_tile_compact(st, bits, P, B_, ntiles, tile_flag_, tile_end_, small_tiles(), tile_bcount_, tile_list_,
                                              tile_list_ + cap_, tile_count_));
   const uint32_t* keys = keys_sorted_;
   if (rec_) {

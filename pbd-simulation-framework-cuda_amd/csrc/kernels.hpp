@@ -64,12 +64,14 @@ struct TileList {
   const uint32_t* large;  // block ids (cell id >> bits) of the large tiles, ascending
   const uint32_t* small;  // block ids of the small tiles, ascending
   const uint32_t* count;  // count[0] large tiles, count[1] small tiles
-  const uint32_t* start;  // per occupied block: 1 + its first sorted index
+  const uint32_t* start;  // per occupied block: 1 + its first sorted index, | kTileCrowded
   const uint32_t* end;    // per occupied block: 1 + its last
   uint32_t cap;           // entries of large
 };
 
 constexpr uint32_t kTileSmall = 64;           // particles of a small tile (one wave)
+constexpr uint32_t kTileSmallSure = 32;       // up to here small whatever its halo holds
+constexpr uint32_t kTileCrowded = 1u << 31;   // a block that is large for its halo
 // The small-tile threshold a context starts with, by particle count.  Measured
 // over 100 frames of the dam break (ms per substep at 0 / 32 / 64): up to 2^16
 // particles the occupied blocks are too few to fill the chip, and packing four
@@ -80,6 +82,11 @@ constexpr uint32_t kTileSmall = 64;           // particles of a small tile (one 
 inline uint32_t default_small_max(uint32_t n) {
   return n <= (1u << 16) ? 0u : n < (1u << 21) ? 32u : kTileSmall;
 }
+// Until a launch shape is set, blocks between that threshold (if it is not 0) and
+// kTileSmall are small as well where their halo fits a small tile: a workgroup of its own
+// leaves three of its waves idle.  us a step with small tiles up to 32 / 48 / 64: 211K
+// splash 588 / 573 / 521, 1M splash 1669 / 1544 / 1438, 64 scenes of 2K to 32K 7960 / 7530
+// / 7355, 1M column 1060 / 1065 / 1064; a 32K frame 223 without, 238 with them.
 constexpr uint32_t kNlChunks = 12;            // neighbour-list chunks of 8 slots: lists of up to 96 pairs
 constexpr uint32_t kTileCompactChunk = 4096;  // flags per block of the compaction
 #ifndef PBD_TILE_CHUNK
@@ -106,8 +113,9 @@ static_assert(kTileGridStride % kTileGridMultiple == 0 && kTileGridDirect % kTil
 // particle count end[b] - (start[b] - 1) (small: at most small_max <= kTileSmall),
 // both ascending; count[0..1] = their lengths.  bcount holds
 // ceil(nflags / kTileCompactChunk) packed block counts.
-hipError_t launch_tile_compact(hipStream_t st, uint32_t nflags, const uint32_t* start, const uint32_t* end,
-                               uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
+// A block of more than kTileSmallSure particles is small only if its halo fits a small tile.
+hipError_t launch_tile_compact(hipStream_t st, int bits, const DevParams& P, const StepBuffers& B, uint32_t nflags,
+                               uint32_t* start, const uint32_t* end, uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
                                uint32_t* count);
 
 hipError_t launch_fill_u32(hipStream_t st, uint32_t* p, uint32_t v, uint32_t n);

@@ -71,6 +71,9 @@ struct TileShared {
 };
 static_assert(TileGeom<6>::HX <= 6 && TileGeom<6>::HY <= 6 && TileGeom<6>::HZ <= 6, "offset table");
 
+// First sorted index of a block (its mark without kTileCrowded).
+__device__ __forceinline__ uint32_t tile_begin(uint32_t start) { return (start & ~kTileCrowded) - 1u; }
+
 // Steps 1 of the tile: halo cell table, LDS offsets and, with OWN, the own range.
 // Returns the halo particle count.  Every thread of the team takes R halo cells; all
 // their cell-table loads are issued, then those of `pre` (what the thread reads whatever
@@ -315,6 +318,21 @@ __device__ __forceinline__ int tile_pick(const TileList& T, const TileItems& it,
   return 0;
 }
 
+// Halo particles held in LDS; the same for the producing and the consuming pass
+// so that a slot names the same particle in both.
+template <int BITS>
+struct TileCap;
+template <>
+struct TileCap<5> {
+  static constexpr int value = 1920;  // 2x4x4 blocks: 144 halo cells, ~1150 particles at rest density
+  static constexpr int small = 420;   // a small tile's halo (one wave, a quarter of the LDS)
+};
+template <>
+struct TileCap<6> {
+  static constexpr int value = 2880;  // 4x4x4 blocks: 216 halo cells, ~1730 at rest density
+  static constexpr int small = 630;
+};
+
 // ---------------------------------------------------------------------------
 // Tile-list compaction: a two-kernel stream compaction of the occupied blocks
 // into the large and the small list.  Per-thread and per-block counts are
@@ -324,7 +342,44 @@ __device__ __forceinline__ uint32_t tile_class(uint32_t b, uint32_t nflags, cons
   if (b >= nflags) return 0u;
   const uint32_t s = start[b];
   if (s == 0u) return 0u;
-  return end[b] - (s - 1u) <= small_max ? 0x10000u : 1u;
+  return !(s & kTileCrowded) && end[b] - tile_begin(s) <= small_max ? 0x10000u : 1u;
+}
+
+// Marks the blocks of more than kTileSmallSure and at most small_max particles whose halo
+// is more than a small tile holds (kTileCrowded): they are large tiles.  As small ones
+// every pass took them particle by particle from global memory (1M splash with small
+// tiles of up to 64: 1862 us, with this 1438).  kHaloLanes lanes a block, all of a lane's
+// cells in flight at once; an empty block costs its lanes one load.  Bound by latency:
+// 6 to 9 us up to 1M particles.
+constexpr uint32_t kHaloLanes = 16;
+template <int BITS>
+__global__ __launch_bounds__(256) void k_tile_halo(DevParams P, uint32_t nflags, uint32_t* __restrict__ start,
+                                                   const uint32_t* __restrict__ end, uint32_t small_max,
+                                                   const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce) {
+  using G = TileGeom<BITS>;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, b = i / kHaloLanes, l = i % kHaloLanes;
+  if (b >= nflags) return;
+  const uint32_t s = start[b];
+  if (s == 0u) return;
+  const uint32_t own = end[b] - tile_begin(s);
+  if (own <= kTileSmallSure || own > small_max) return;
+  const uint32_t first = b << BITS;
+  const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
+  uint32_t halo = 0u;
+#pragma unroll
+  for (uint32_t r = 0; r < ((uint32_t)G::NH + kHaloLanes - 1u) / kHaloLanes; ++r) {
+    const uint32_t c = r * kHaloLanes + l;
+    if (c >= (uint32_t)G::NH) break;
+    const int cx = ix0 - 1 + (int)c / G::SX, cy = iy0 - 1 + ((int)c / G::SY) % G::HY, cz = iz0 - 1 + (int)c % G::HZ;
+    if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
+      const uint32_t k = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
+      const uint32_t a = cs[k], e = ce[k];
+      halo += a != 0xFFFFFFFFu ? e - a : 0u;
+    }
+  }
+#pragma unroll
+  for (uint32_t o = kHaloLanes / 2u; o; o >>= 1) halo += (uint32_t)__shfl_xor((int)halo, (int)o, (int)kHaloLanes);
+  if (l == 0u && halo > (uint32_t)TileCap<BITS>::small) start[b] = s | kTileCrowded;
 }
 
 __global__ __launch_bounds__(1024) void k_tile_count(uint32_t nflags, const uint32_t* __restrict__ start,
@@ -414,10 +469,17 @@ __global__ __launch_bounds__(1024) void k_tile_emit(uint32_t nflags, const uint3
   }
 }
 
-hipError_t launch_tile_compact(hipStream_t st, uint32_t nflags, const uint32_t* start, const uint32_t* end,
-                               uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
+hipError_t launch_tile_compact(hipStream_t st, int bits, const DevParams& P, const StepBuffers& B, uint32_t nflags,
+                               uint32_t* start, const uint32_t* end, uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
                                uint32_t* count) {
   if (small_max > kTileSmall) return hipErrorInvalidValue;  // a small tile is one wave, one particle per lane
+  if (small_max > kTileSmallSure) {
+    const dim3 g((uint32_t)(((size_t)nflags * kHaloLanes + 255u) / 256u)), t(256);
+    if (bits == 5)
+      hipLaunchKernelGGL(k_tile_halo<5>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend);
+    else
+      hipLaunchKernelGGL(k_tile_halo<6>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend);
+  }
   const uint32_t blocks = (nflags + kTileCompactChunk - 1u) / kTileCompactChunk;
   hipLaunchKernelGGL(k_tile_count, dim3(blocks), dim3(1024), 0, st, nflags, start, end, small_max, bcount);
   hipLaunchKernelGGL(k_tile_emit, dim3(blocks), dim3(1024), 0, st, nflags, start, end, small_max, bcount, large, small,
@@ -455,20 +517,6 @@ struct NeighbourList {
   unsigned long long* stats;  // PBD_COUNTER_LIST_*
 };
 
-// Halo particles held in LDS; the same for the producing and the consuming pass
-// so that a slot names the same particle in both.
-template <int BITS>
-struct TileCap;
-template <>
-struct TileCap<5> {
-  static constexpr int value = 1920;  // 2x4x4 blocks: 144 halo cells, ~1150 particles at rest density
-  static constexpr int small = 420;   // a small tile's halo (one wave, a quarter of the LDS)
-};
-template <>
-struct TileCap<6> {
-  static constexpr int value = 2880;  // 4x4x4 blocks: 216 halo cells, ~1730 at rest density
-  static constexpr int small = 630;
-};
 // Scan unroll: candidates tested per group in nl_column.
 #ifndef PBD_SCAN_UNROLL
 #define PBD_SCAN_UNROLL 4
@@ -814,7 +862,7 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileLi
                                             const Carry& C, TileShared<BITS>& sh, float4* s_q) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
   uint32_t key = 0u;  // of the thread's next particle
   const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
     if (g0 + tid < g1) key = keys[g0 + tid];
@@ -947,7 +995,7 @@ __device__ __forceinline__ TileRest delta_tile(const DevParams& P, const TileLis
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
   // the thread's next particle: its key, list length and first chunk
   uint32_t key = 0u, n = kNlInvalid;
   uint4 chunk = make_uint4(0u, 0u, 0u, 0u);
@@ -1083,7 +1131,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
   uint32_t key = 0u;  // of the thread's next particle, and its velocity
   float4 v4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
@@ -1223,7 +1271,7 @@ __device__ __forceinline__ TileRest final_tile(const DevParams& P, const TileLis
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk];
+  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
   // the thread's next particle: its key, list length and first chunk
   uint32_t key = 0u, n = kNlInvalid;
   uint4 chunk = make_uint4(0u, 0u, 0u, 0u);
@@ -1478,7 +1526,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
   if (!wide_pick(T, blockIdx.x, blk)) return;
   TileShared<5>& sh = lds.sh;
   const uint32_t tid = threadIdx.x, sub = tid % kQuad;
-  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk], gf = g0 + tid / kQuad;
+  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk], gf = g0 + tid / kQuad;
   uint32_t key = 0u;  // of the quad's next particle
   const uint32_t total = tile_setup<5, TeamWide, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
     if (gf < g1) key = keys[gf];
@@ -1597,7 +1645,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
   if (!wide_pick(T, blockIdx.x, blk)) return;
   TileShared<5>& sh = lds.sh;
   const uint32_t tid = threadIdx.x, sub = tid % kQuad;
-  const uint32_t g0 = T.start[blk] - 1u, g1 = T.end[blk], gf = g0 + tid / kQuad;
+  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk], gf = g0 + tid / kQuad;
   uint32_t key = 0u;  // of the quad's next particle, and its velocity
   float4 v4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const uint32_t total = tile_setup<5, TeamWide, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
