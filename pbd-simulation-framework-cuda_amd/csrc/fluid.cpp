@@ -464,14 +464,15 @@ int Fluid::enqueue_substep() {
     ntiles = ((B_.table_size - 1u) >> bits) + 1u;
     // work items (large tiles + small tiles / 4) <= occupied blocks <= min(ntiles, n);
     // a multiple of XCDs x tile chunk, so that tile_rank0 maps the grid onto [0, tgrid)
-    tgrid = (std::min(ntiles, P.n) + kTileGridMultiple - 1u) / kTileGridMultiple * kTileGridMultiple;
+    tgrid = (std::min(ntiles, P.n) + split_bound(ntiles, P.n) + kTileGridMultiple - 1u) / kTileGridMultiple *
+            kTileGridMultiple;
     tstride = tgrid > kTileGridDirect;
     if (tstride) tgrid = stride_grid_;
     // phases on tiles: 2^5-cell blocks with the direct grid only
     if (P.phased && (bits != 5 || tstride)) tiles = false;
   }
-  const uint32_t wgrid = std::min(ntiles, P.n);  // the wide passes': a workgroup per block
-  const bool wide = tiles && wide_tiles(P, bits, small_max(), wgrid);
+  const uint32_t wgrid = std::min(ntiles, P.n) + split_bound(ntiles, P.n);  // the wide passes': a workgroup per block
+  const bool wide = tiles && wide_tiles(P, bits, small_max(), std::min(ntiles, P.n));
   const TileList TL{tile_list_, tile_list_ + cap_, tile_count_, tile_flag_, tile_end_, cap_};
   // Lists carried over the substep: in the tiles whose halo stayed within the
   // skin over the last substep, the first lambda pass builds them with the
@@ -508,7 +509,7 @@ int Fluid::enqueue_substep() {
   PBD_LAUNCH(ST_PREDICT, launch_predict_keys(st, tpb, P, B_, sort_.hist, sort_.passes, kSortHistCopies));
   // resetCellInfo (Fluid.cu:31): empty = {UINT_MAX, N}
   PBD_LAUNCH(ST_CELL_RESET, launch_cell_reset(st, B_.cstart, B_.cend, B_.table_size, P.n, tiles ? tile_flag_ : nullptr,
-                                              tiles ? ntiles : 0u));
+                                              tiles ? ntiles : 0u, tile_bcount_));
   // 3. sortIds (Fluid.cu:27)
   PBD_LAUNCH(ST_SORT, launch_sort_ranks(st, sort_, P.n, B_.keys_in, &keys_sorted_, &ids_sorted_));
   // 4-5. reorderStorage + computeCellInfo (Fluid.cu:29,33)

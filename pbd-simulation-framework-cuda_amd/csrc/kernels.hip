@@ -257,7 +257,10 @@ static inline uint32_t blocks_for(uint32_t n, uint32_t tpb) { return (n + tpb - 
 // cstart = UINT_MAX, cend = n, and the occupied-block flags cleared, with 16-byte
 // stores (the arrays come from hipMalloc, 256-byte aligned).
 __global__ void k_cell_reset(uint32_t* __restrict__ cstart, uint32_t* __restrict__ cend, uint32_t ts, uint32_t n,
-                             uint32_t* __restrict__ flags, uint32_t nflags) {
+                             uint32_t* __restrict__ flags, uint32_t nflags, uint32_t* __restrict__ bcount,
+                             uint32_t nb) {
+  if (blockIdx.x == 0)
+    for (uint32_t t = threadIdx.x; t < nb; t += blockDim.x) bcount[t] = 0u;
   const uint32_t q1 = ts / 4u, q2 = nflags / 4u, total = 2u * q1 + q2;
   const uint32_t stride = gridDim.x * blockDim.x;
   const uint4 emp = make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu), cnt = make_uint4(n, n, n, n);
@@ -277,12 +280,13 @@ __global__ void k_cell_reset(uint32_t* __restrict__ cstart, uint32_t* __restrict
 }
 
 hipError_t launch_cell_reset(hipStream_t st, uint32_t* cstart, uint32_t* cend, uint32_t ts, uint32_t n,
-                             uint32_t* flags, uint32_t nflags) {
+                             uint32_t* flags, uint32_t nflags, uint32_t* bcount) {
   if (!flags) nflags = 0;
+  const uint32_t nb = (nflags + kTileCompactChunk - 1u) / kTileCompactChunk;
   const uint32_t total = 2u * (ts / 4u) + nflags / 4u + 1u;
   uint32_t b = blocks_for(total, 256);
   if (b > 4096) b = 4096;
-  hipLaunchKernelGGL(k_cell_reset, dim3(b), dim3(256), 0, st, cstart, cend, ts, n, flags, nflags);
+  hipLaunchKernelGGL(k_cell_reset, dim3(b), dim3(256), 0, st, cstart, cend, ts, n, flags, nflags, bcount, nb);
   return hipGetLastError();
 }
 

@@ -61,17 +61,20 @@ constexpr uint32_t kNoCarry = 0xFFFFFFFFu;
 // kTileSmall particles are "small": four of them share one workgroup, one wave
 // each; the others take a whole workgroup.
 struct TileList {
-  const uint32_t* large;  // block ids (cell id >> bits) of the large tiles, ascending
+  const uint32_t* large;  // block ids (cell id >> bits) of the large tiles, ascending; a split block twice, its halves' marks in bits 30, 31
   const uint32_t* small;  // block ids of the small tiles, ascending
   const uint32_t* count;  // count[0] large tiles, count[1] small tiles
-  const uint32_t* start;  // per occupied block: 1 + its first sorted index, | kTileCrowded
+  const uint32_t* start;  // per occupied block: 1 + its first sorted index, | its marks
   const uint32_t* end;    // per occupied block: 1 + its last
   uint32_t cap;           // entries of large
 };
 
 constexpr uint32_t kTileSmall = 64;           // particles of a small tile (one wave)
-constexpr uint32_t kTileSmallSure = 32;       // up to here small whatever its halo holds
+constexpr uint32_t kTileSmallSure = 8;        // up to here small whatever its halo holds
 constexpr uint32_t kTileCrowded = 1u << 31;   // a block that is large for its halo
+constexpr uint32_t kTileSplit = 1u << 30;     // a block that is two items for its halo
+// Blocks that are two items: a halo of more than 1352 particles; a particle is in at most 8 (1352 / 8 = 169).
+inline uint32_t split_bound(uint32_t ntiles, uint32_t n) { return n / 169u + 1u < ntiles ? n / 169u + 1u : ntiles; }
 // The small-tile threshold a context starts with, by particle count.  Measured
 // over 100 frames of the dam break (ms per substep at 0 / 32 / 64): up to 2^16
 // particles the occupied blocks are too few to fill the chip, and packing four
@@ -113,7 +116,8 @@ static_assert(kTileGridStride % kTileGridMultiple == 0 && kTileGridDirect % kTil
 // particle count end[b] - (start[b] - 1) (small: at most small_max <= kTileSmall),
 // both ascending; count[0..1] = their lengths.  bcount holds
 // ceil(nflags / kTileCompactChunk) packed block counts.
-// A block of more than kTileSmallSure particles is small only if its halo fits a small tile.
+// A block of more than kTileSmallSure particles is small only if its halo fits a small
+// tile, and one whose halo exceeds a tile is two items.  bcount starts at zero.
 hipError_t launch_tile_compact(hipStream_t st, int bits, const DevParams& P, const StepBuffers& B, uint32_t nflags,
                                uint32_t* start, const uint32_t* end, uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
                                uint32_t* count);
@@ -136,7 +140,7 @@ struct CopySet {
 hipError_t launch_copy_set(hipStream_t st, const CopySet& c);
 // cstart[0, ts) = UINT_MAX, cend[0, ts) = n, flags[0, nflags) = 0 (flags may be null)
 hipError_t launch_cell_reset(hipStream_t st, uint32_t* cstart, uint32_t* cend, uint32_t ts, uint32_t n,
-                             uint32_t* flags, uint32_t nflags);
+                             uint32_t* flags, uint32_t nflags, uint32_t* bcount);
 // applyForces + initializeCellIds; the keys' digits of `passes` 8-bit passes are
 // added to copy (workgroup mod copies) of the sort's histogram (SortPlan::hist).
 hipError_t launch_predict_keys(hipStream_t st, uint32_t tpb, const DevParams& P, const StepBuffers& B, uint32_t* hist,

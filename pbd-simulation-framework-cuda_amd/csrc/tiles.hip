@@ -72,7 +72,34 @@ struct TileShared {
 static_assert(TileGeom<6>::HX <= 6 && TileGeom<6>::HY <= 6 && TileGeom<6>::HZ <= 6, "offset table");
 
 // First sorted index of a block (its mark without kTileCrowded).
-__device__ __forceinline__ uint32_t tile_begin(uint32_t start) { return (start & ~kTileCrowded) - 1u; }
+__device__ __forceinline__ uint32_t tile_begin(uint32_t start) { return (start & ~(kTileCrowded | kTileSplit)) - 1u; }
+
+// A work item of the lists: a block, or one half of a block whose halo exceeds the tile
+// capacity (half 1: its cells of y 0 and 1, half 2: of y 2 and 3; the halves of a 2^5-cell
+// block are consecutive key ranges), and its own particles.
+struct TileOwn {
+  uint32_t blk, half, g0, g1;
+};
+template <int BITS>
+__device__ __forceinline__ TileOwn tile_own(const DevParams& P, const TileList& T, uint32_t item,
+                                            const uint32_t* __restrict__ cs) {
+  TileOwn o;
+  o.half = BITS == 5 ? item >> 30 : 0u;
+  o.blk = item & (kTileSplit - 1u);
+  o.g0 = tile_begin(T.start[o.blk]);
+  o.g1 = T.end[o.blk];
+  if (o.half) {
+    uint32_t mid = o.g1;  // the first particle of the second half (an empty cell starts at 2^32 - 1)
+    for (uint32_t c = 16u; c < 32u; ++c) {
+      const uint32_t k = (o.blk << 5) + c;
+      if (compact10(k >> 2) < P.dims[0] && compact10(k >> 1) < P.dims[1] && compact10(k) < P.dims[2])
+        mid = min(mid, cs[k]);
+    }
+    if (o.half == 1u) o.g1 = mid;
+    else o.g0 = mid;
+  }
+  return o;
+}
 
 // Steps 1 of the tile: halo cell table, LDS offsets and, with OWN, the own range.
 // Returns the halo particle count.  Every thread of the team takes R halo cells; all
@@ -88,13 +115,15 @@ struct NoLoads {
 template <int BITS, class Team, bool OWN = true, class Pre = NoLoads>
 __device__ __forceinline__ uint32_t tile_setup(const DevParams& P, uint32_t blk, const uint32_t* __restrict__ cs,
                                                const uint32_t* __restrict__ ce, TileShared<BITS>& sh,
-                                               Pre pre = Pre()) {
+                                               Pre pre = Pre(), uint32_t half = 0u) {
   using G = TileGeom<BITS>;
   constexpr uint32_t R = (G::NH + Team::kSize - 1u) / Team::kSize;
   static_assert(Team::kSize == 64u || R == 1u, "a workgroup team takes one halo cell per thread");
   const uint32_t tid = Team::tid(), lane = threadIdx.x & 63u;
   const uint32_t first = blk << BITS;
   const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
+  // a half's halo: the layers around its own y (the other cells count as empty)
+  const int y0 = half == 2u ? 2 : 0, y1 = half == 1u ? 4 : G::HY;
   uint32_t s0[R], e0[R];
 #pragma unroll
   for (uint32_t r = 0; r < R; ++r) {
@@ -104,7 +133,8 @@ __device__ __forceinline__ uint32_t tile_setup(const DevParams& P, uint32_t blk,
     if (c < (uint32_t)G::NH) {
       const int hx = (int)c / G::SX, hy = ((int)c / G::SY) % G::HY, hz = (int)c % G::HZ;
       const int cx = ix0 - 1 + hx, cy = iy0 - 1 + hy, cz = iz0 - 1 + hz;
-      if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
+      if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2] &&
+          hy >= y0 && hy < y1) {
         const uint32_t k = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
         s0[r] = cs[k];
         e0[r] = ce[k];
@@ -322,15 +352,23 @@ __device__ __forceinline__ int tile_pick(const TileList& T, const TileItems& it,
 // so that a slot names the same particle in both.
 template <int BITS>
 struct TileCap;
+// The capacity decides how many workgroups a CU holds: with 1352 slots (and small tiles'
+// 272) a lambda pass has 23 KB and 7 of them, as many as its 67 VGPRs allow, at 1920 slots
+// 5.  us a step at 1920 / 1352 slots: 1M column 1060 / 964, 1M splash 1438 / 1285, 16M
+// column 14700 / 13650, 64 uneven scenes 7360 / 7110.  A block with more in its halo (1152
+// at rest density) is two items, its halves, which hold as crowded cells as 1920 slots did
+// for the whole (a half's halo is 96 cells of the 144).
 template <>
 struct TileCap<5> {
-  static constexpr int value = 1920;  // 2x4x4 blocks: 144 halo cells, ~1150 particles at rest density
-  static constexpr int small = 420;   // a small tile's halo (one wave, a quarter of the LDS)
+  static constexpr int value = 1352;  // 2x4x4 blocks: 144 halo cells, ~1150 particles at rest density
+  static constexpr int small = 272;   // a small tile's halo (one wave, a quarter of the LDS)
+  static constexpr int adjoint = 1920;  // of the reverse passes' list builders
 };
 template <>
 struct TileCap<6> {
   static constexpr int value = 2880;  // 4x4x4 blocks: 216 halo cells, ~1730 at rest density
   static constexpr int small = 630;
+  static constexpr int adjoint = 2880;
 };
 
 // ---------------------------------------------------------------------------
@@ -342,63 +380,56 @@ __device__ __forceinline__ uint32_t tile_class(uint32_t b, uint32_t nflags, cons
   if (b >= nflags) return 0u;
   const uint32_t s = start[b];
   if (s == 0u) return 0u;
-  return !(s & kTileCrowded) && end[b] - tile_begin(s) <= small_max ? 0x10000u : 1u;
+  if (!(s & kTileCrowded) && end[b] - tile_begin(s) <= small_max) return 0x10000u;
+  return s & kTileSplit ? 2u : 1u;
 }
 
-// Marks the blocks of more than kTileSmallSure and at most small_max particles whose halo
-// is more than a small tile holds (kTileCrowded): they are large tiles.  As small ones
-// every pass took them particle by particle from global memory (1M splash with small
-// tiles of up to 64: 1862 us, with this 1438).  kHaloLanes lanes a block, all of a lane's
-// cells in flight at once; an empty block costs its lanes one load.  Bound by latency:
-// 6 to 9 us up to 1M particles.
+// Marks the occupied blocks by their halos and counts the items of every 4096 flags: a
+// block of at most small_max particles whose halo is more than a small tile holds is
+// large (kTileCrowded; as a small one every pass took it particle by particle from global
+// memory: 1M splash with small tiles of up to 64, 1862 us, with the marks 1438), and a
+// large one whose halo is more than a tile holds is two items (kTileSplit).  Blocks of at
+// most kTileSmallSure particles stay small.  kHaloLanes lanes a block, all of a lane's
+// cells in flight at once; an empty block costs its lanes one load.  Bound by latency: 6
+// to 9 us up to 1M particles.
 constexpr uint32_t kHaloLanes = 16;
 template <int BITS>
-__global__ __launch_bounds__(256) void k_tile_halo(DevParams P, uint32_t nflags, uint32_t* __restrict__ start,
-                                                   const uint32_t* __restrict__ end, uint32_t small_max,
-                                                   const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce) {
+__global__ __launch_bounds__(256) void k_tile_classify(DevParams P, uint32_t nflags, uint32_t* __restrict__ start,
+                                                       const uint32_t* __restrict__ end, uint32_t small_max,
+                                                       const uint32_t* __restrict__ cs,
+                                                       const uint32_t* __restrict__ ce, uint32_t* __restrict__ bcount) {
   using G = TileGeom<BITS>;
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, b = i / kHaloLanes, l = i % kHaloLanes;
-  if (b >= nflags) return;
-  const uint32_t s = start[b];
-  if (s == 0u) return;
-  const uint32_t own = end[b] - tile_begin(s);
-  if (own <= kTileSmallSure || own > small_max) return;
+  uint32_t s = b < nflags ? start[b] : 0u;
+  const uint32_t own = s ? end[b] - tile_begin(s) : 0u;
   const uint32_t first = b << BITS;
-  const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
-  uint32_t halo = 0u;
+  if (own > min(kTileSmallSure, small_max)) {
+    const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
+    uint32_t halo = 0u;
 #pragma unroll
-  for (uint32_t r = 0; r < ((uint32_t)G::NH + kHaloLanes - 1u) / kHaloLanes; ++r) {
-    const uint32_t c = r * kHaloLanes + l;
-    if (c >= (uint32_t)G::NH) break;
-    const int cx = ix0 - 1 + (int)c / G::SX, cy = iy0 - 1 + ((int)c / G::SY) % G::HY, cz = iz0 - 1 + (int)c % G::HZ;
-    if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
-      const uint32_t k = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
-      const uint32_t a = cs[k], e = ce[k];
-      halo += a != 0xFFFFFFFFu ? e - a : 0u;
+    for (uint32_t r = 0; r < ((uint32_t)G::NH + kHaloLanes - 1u) / kHaloLanes; ++r) {
+      const uint32_t c = r * kHaloLanes + l;
+      if (c >= (uint32_t)G::NH) break;
+      const int cx = ix0 - 1 + (int)c / G::SX, cy = iy0 - 1 + ((int)c / G::SY) % G::HY, cz = iz0 - 1 + (int)c % G::HZ;
+      if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
+        const uint32_t k = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
+        const uint32_t a = cs[k], e = ce[k];
+        halo += a != 0xFFFFFFFFu ? e - a : 0u;
+      }
     }
+#pragma unroll
+    for (uint32_t o = kHaloLanes / 2u; o; o >>= 1) halo += (uint32_t)__shfl_xor((int)halo, (int)o, (int)kHaloLanes);
+    uint32_t mark = 0u;
+    if (own <= small_max && halo > (uint32_t)TileCap<BITS>::small) mark = kTileCrowded;
+    if (BITS == 5 && (own > small_max || mark) && halo > (uint32_t)TileCap<BITS>::value) mark |= kTileSplit;
+    if (mark && l == 0u) start[b] = s | mark;
+    s |= mark;
   }
+  uint32_t c = 0u;
+  if (s && l == 0u) c = !(s & kTileCrowded) && own <= small_max ? 0x10000u : s & kTileSplit ? 2u : 1u;
 #pragma unroll
-  for (uint32_t o = kHaloLanes / 2u; o; o >>= 1) halo += (uint32_t)__shfl_xor((int)halo, (int)o, (int)kHaloLanes);
-  if (l == 0u && halo > (uint32_t)TileCap<BITS>::small) start[b] = s | kTileCrowded;
-}
-
-__global__ __launch_bounds__(1024) void k_tile_count(uint32_t nflags, const uint32_t* __restrict__ start,
-                                                     const uint32_t* __restrict__ end, uint32_t small_max,
-                                                     uint32_t* __restrict__ bcount) {
-  __shared__ uint32_t s_w[16];
-  const uint32_t base = blockIdx.x * kTileCompactChunk + threadIdx.x * 4u;
-  uint32_t c = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < 4; ++k) c += tile_class(base + k, nflags, start, end, small_max);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) c += __shfl_xor(c, o);
-  if ((threadIdx.x & 63u) == 0) s_w[threadIdx.x >> 6] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0;
-    for (int w = 0; w < 16; ++w) t += s_w[w];
-    bcount[blockIdx.x] = t;
-  }
+  for (int o = 32; o >= 1; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o);
+  if ((threadIdx.x & 63u) == 0u && c) atomicAdd(&bcount[b / kTileCompactChunk], c);
 }
 
 __global__ __launch_bounds__(1024) void k_tile_emit(uint32_t nflags, const uint32_t* __restrict__ start,
@@ -459,8 +490,13 @@ __global__ __launch_bounds__(1024) void k_tile_emit(uint32_t nflags, const uint3
   uint32_t pl = s_off[0] + (ex & 0xFFFFu), ps = s_off[1] + (ex >> 16);
 #pragma unroll
   for (uint32_t k = 0; k < 4; ++k) {
-    if (f[k] == 1u) large[pl++] = base + k;
-    else if (f[k]) small[ps++] = base + k;
+    if (f[k] == 1u) {
+      large[pl++] = base + k;
+    } else if (f[k] == 2u) {
+      large[pl++] = (base + k) | (1u << 30);
+      large[pl++] = (base + k) | (2u << 30);
+    }
+    if (f[k] > 2u) small[ps++] = base + k;
   }
   if (blockIdx.x == gridDim.x - 1 && tid == 1023u) {
     const uint32_t tot = pre + x;
@@ -473,15 +509,12 @@ hipError_t launch_tile_compact(hipStream_t st, int bits, const DevParams& P, con
                                uint32_t* start, const uint32_t* end, uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
                                uint32_t* count) {
   if (small_max > kTileSmall) return hipErrorInvalidValue;  // a small tile is one wave, one particle per lane
-  if (small_max > kTileSmallSure) {
-    const dim3 g((uint32_t)(((size_t)nflags * kHaloLanes + 255u) / 256u)), t(256);
-    if (bits == 5)
-      hipLaunchKernelGGL(k_tile_halo<5>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend);
-    else
-      hipLaunchKernelGGL(k_tile_halo<6>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend);
-  }
+  const dim3 g((uint32_t)(((size_t)nflags * kHaloLanes + 255u) / 256u)), t(256);
+  if (bits == 5)
+    hipLaunchKernelGGL(k_tile_classify<5>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend, bcount);
+  else
+    hipLaunchKernelGGL(k_tile_classify<6>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend, bcount);
   const uint32_t blocks = (nflags + kTileCompactChunk - 1u) / kTileCompactChunk;
-  hipLaunchKernelGGL(k_tile_count, dim3(blocks), dim3(1024), 0, st, nflags, start, end, small_max, bcount);
   hipLaunchKernelGGL(k_tile_emit, dim3(blocks), dim3(1024), 0, st, nflags, start, end, small_max, bcount, large, small,
                      count);
   return hipGetLastError();
@@ -519,7 +552,7 @@ struct NeighbourList {
 
 // Scan unroll: candidates tested per group in nl_column.
 #ifndef PBD_SCAN_UNROLL
-#define PBD_SCAN_UNROLL 4
+#define PBD_SCAN_UNROLL 8
 #endif
 constexpr uint32_t kScanUnroll = PBD_SCAN_UNROLL;
 
@@ -854,7 +887,7 @@ __device__ __forceinline__ uint32_t nl_build(const DevParams& P, const Neighbour
 // tile built after an earlier delta-p pass when its halo has moved less than
 // P.reuse_max since.  A carrying tile builds with the skin (P.tile_r2).
 template <int BITS, bool FIRST, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L,
+__device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileList& T, uint32_t item, const NeighbourList& L,
                                             const float4* __restrict__ Q, const uint32_t* __restrict__ keys,
                                             const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
                                             float* __restrict__ lam, float* __restrict__ dens,
@@ -862,11 +895,12 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileLi
                                             const Carry& C, TileShared<BITS>& sh, float4* s_q) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
+  const TileOwn own = tile_own<BITS>(P, T, item, cs);
+  const uint32_t blk = own.blk, g0 = own.g0, g1 = own.g1;
   uint32_t key = 0u;  // of the thread's next particle
   const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
     if (g0 + tid < g1) key = keys[g0 + tid];
-  });
+  }, own.half);
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) L.cnt[g] = kNlInvalid;
@@ -875,7 +909,7 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileLi
   }
   // the first pass: whether the tile carries its lists this substep; a later
   // one: the delta-p passes before the tile's lists were built (kNoCarry: none)
-  const uint32_t m = C.disp ? (FIRST ? (C.mode[blk] ? 0u : kNoCarry) : C.built[blk]) : kNoCarry;
+  const uint32_t m = C.disp && !own.half ? (FIRST ? (C.mode[blk] ? 0u : kNoCarry) : C.built[blk]) : kNoCarry;
   const bool carry = !FIRST && m != kNoCarry;
   const float r2 = m != kNoCarry ? P.tile_r2 : P.list_r2;
   // .w: 1 for a solid particle (PH), else 0
@@ -885,7 +919,7 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileLi
   Team::sync();
   const bool keep = carry && tile_keeps_lists<BITS>(P, sh);
   if (tid == 0 && C.disp) {
-    if (FIRST) C.built[blk] = m;  // 0: built now, with the skin
+    if (FIRST && !own.half) C.built[blk] = m;  // 0: built now, with the skin
     else if (carry && !keep) C.built[blk] = C.pass;  // rebuilt now
     if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                          (unsigned long long)(g1 - g0));
@@ -985,7 +1019,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_lambda(DevParams P, TileL
 // lists (use_list) or a scan of the stencil; with a carry, each particle's
 // displacement bound after the pass is recorded.
 template <int BITS, bool COLLIDE, int NS, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest delta_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L, int use_list,
+__device__ __forceinline__ TileRest delta_tile(const DevParams& P, const TileList& T, uint32_t item, const NeighbourList& L, int use_list,
                                            uint32_t flags, const float4* __restrict__ Q,
                                            const float4* __restrict__ QX, const float* __restrict__ lam,
                                            const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cs,
@@ -995,7 +1029,8 @@ __device__ __forceinline__ TileRest delta_tile(const DevParams& P, const TileLis
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
+  const TileOwn own = tile_own<BITS>(P, T, item, cs);
+  const uint32_t blk = own.blk, g0 = own.g0, g1 = own.g1;
   // the thread's next particle: its key, list length and first chunk
   uint32_t key = 0u, n = kNlInvalid;
   uint4 chunk = make_uint4(0u, 0u, 0u, 0u);
@@ -1008,7 +1043,7 @@ __device__ __forceinline__ TileRest delta_tile(const DevParams& P, const TileLis
   };
   const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
     if (g0 + tid < g1) next(g0 + tid);
-  });
+  }, own.half);
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) return rest;
   // s_gi (friction-capable passes): the global index of every slot, for the
@@ -1123,7 +1158,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_delta(DevParams P, TileLi
 // in the next substep: when its halo has moved less than P.reuse_max since its
 // lists were built, or, for a tile that did not carry, over the whole substep.
 template <int BITS, bool XSPH, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L,
+__device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileList& T, uint32_t item, const NeighbourList& L,
                                            const float4* __restrict__ Q, const float4* __restrict__ VS,
                                            const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cs,
                                            const uint32_t* __restrict__ ce, float4* __restrict__ OM,
@@ -1131,7 +1166,8 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
+  const TileOwn own = tile_own<BITS>(P, T, item, cs);
+  const uint32_t blk = own.blk, g0 = own.g0, g1 = own.g1;
   uint32_t key = 0u;  // of the thread's next particle, and its velocity
   float4 v4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
@@ -1139,7 +1175,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
       key = keys[g0 + tid];
       v4 = VS[g0 + tid];
     }
-  });
+  }, own.half);
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += Team::kSize) L.cnt[g] = kNlInvalid;
@@ -1148,7 +1184,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
   }
   // global index of each slot: velocities are gathered from L2
   // .w: 1 for a solid particle (PH), else 0
-  const uint32_t m = C.disp ? C.built[blk] : kNoCarry;
+  const uint32_t m = C.disp && !own.half ? C.built[blk] : kNoCarry;
   const bool carry = m != kNoCarry;
   tile_load<BITS, CAP, Team>(P, sh, total, Q, s_q, s_gi, g0,
                              [&](uint32_t gi) { return PH && P.phs[gi] ? 1.0f : 0.0f; },
@@ -1157,7 +1193,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
   const bool calm = C.disp && tile_keeps_lists<BITS>(P, sh);
   const bool keep = carry && calm;
   if (tid == 0 && C.disp) {
-    C.mode[blk] = calm ? 1u : 0u;
+    C.mode[blk] = calm && !own.half ? 1u : 0u;  // halves do not carry: both write 0
     if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                          (unsigned long long)(g1 - g0));
   }
@@ -1260,7 +1296,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_omega(DevParams P, TileLi
 }
 
 template <int BITS, bool VORT, bool XSPH, bool PH, class Team, int CAP>
-__device__ __forceinline__ TileRest final_tile(const DevParams& P, const TileList& T, uint32_t blk, const NeighbourList& L, int use_list,
+__device__ __forceinline__ TileRest final_tile(const DevParams& P, const TileList& T, uint32_t item, const NeighbourList& L, int use_list,
                                            uint32_t flags, const float4* __restrict__ Q,
                                            const float4* __restrict__ QX, const float4* __restrict__ VS,
                                            const float4* __restrict__ OM, const uint32_t* __restrict__ keys,
@@ -1271,7 +1307,8 @@ __device__ __forceinline__ TileRest final_tile(const DevParams& P, const TileLis
                                            float4* s_q, uint32_t* s_gi) {
   constexpr int VAR = PBD_KERNEL_TEXTBOOK;
   const uint32_t tid = Team::tid();
-  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk];
+  const TileOwn own = tile_own<BITS>(P, T, item, cs);
+  const uint32_t blk = own.blk, g0 = own.g0, g1 = own.g1;
   // the thread's next particle: its key, list length and first chunk
   uint32_t key = 0u, n = kNlInvalid;
   uint4 chunk = make_uint4(0u, 0u, 0u, 0u);
@@ -1284,7 +1321,7 @@ __device__ __forceinline__ TileRest final_tile(const DevParams& P, const TileLis
   };
   const uint32_t total = tile_setup<BITS, Team, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
     if (g0 + tid < g1) next(g0 + tid);
-  });
+  }, own.half);
   constexpr bool vort = VORT, xsph = XSPH;  // flags & FF_VORT, flags & FF_XSPH
   TileRest rest = tile_rest<Team>(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
@@ -1522,22 +1559,23 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
   constexpr int CAP = TileCap<5>::value;
   __shared__ WideLds lds;
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&L.stats[PBD_COUNTER_LIST_BUILDS], 1ull);
-  uint32_t blk;
-  if (!wide_pick(T, blockIdx.x, blk)) return;
+  uint32_t item;
+  if (!wide_pick(T, blockIdx.x, item)) return;
   TileShared<5>& sh = lds.sh;
   const uint32_t tid = threadIdx.x, sub = tid % kQuad;
-  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk], gf = g0 + tid / kQuad;
+  const TileOwn own = tile_own<5>(P, T, item, cs);
+  const uint32_t blk = own.blk, g0 = own.g0, g1 = own.g1, gf = g0 + tid / kQuad;
   uint32_t key = 0u;  // of the quad's next particle
   const uint32_t total = tile_setup<5, TeamWide, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
     if (gf < g1) key = keys[gf];
-  });
+  }, own.half);
   TileRest rest = wide_rest(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += kWideThreads) L.cnt[g] = kNlInvalid;
     if (tid == 0) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_BLOCK], (unsigned long long)(g1 - g0));
   } else {
     // as lambda_tile
-    const uint32_t m = C.disp ? (FIRST ? (C.mode[blk] ? 0u : kNoCarry) : C.built[blk]) : kNoCarry;
+    const uint32_t m = C.disp && !own.half ? (FIRST ? (C.mode[blk] ? 0u : kNoCarry) : C.built[blk]) : kNoCarry;
     const bool carry = !FIRST && m != kNoCarry;
     const float r2 = m != kNoCarry ? P.tile_r2 : P.list_r2;
     tile_load<5, CAP, TeamWide>(P, sh, total, Q, lds.q, nullptr, 0u, [](uint32_t) { return 0.0f; },
@@ -1545,7 +1583,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
     __syncthreads();
     const bool keep = carry && tile_keeps_lists<5>(P, sh);
     if (tid == 0 && C.disp) {
-      if (FIRST) C.built[blk] = m;
+      if (FIRST && !own.half) C.built[blk] = m;
       else if (carry && !keep) C.built[blk] = C.pass;
       if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                            (unsigned long long)(g1 - g0));
@@ -1641,11 +1679,12 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
   constexpr int CAP = TileCap<5>::value;
   __shared__ WideLds lds;
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&L.stats[PBD_COUNTER_LIST_BUILDS], 1ull);
-  uint32_t blk;
-  if (!wide_pick(T, blockIdx.x, blk)) return;
+  uint32_t item;
+  if (!wide_pick(T, blockIdx.x, item)) return;
   TileShared<5>& sh = lds.sh;
   const uint32_t tid = threadIdx.x, sub = tid % kQuad;
-  const uint32_t g0 = tile_begin(T.start[blk]), g1 = T.end[blk], gf = g0 + tid / kQuad;
+  const TileOwn own = tile_own<5>(P, T, item, cs);
+  const uint32_t blk = own.blk, g0 = own.g0, g1 = own.g1, gf = g0 + tid / kQuad;
   uint32_t key = 0u;  // of the quad's next particle, and its velocity
   float4 v4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const uint32_t total = tile_setup<5, TeamWide, false>(P, blk, cs, ce, sh, [&]() __attribute__((always_inline)) {
@@ -1653,7 +1692,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
       key = keys[gf];
       v4 = VS[gf];
     }
-  });
+  }, own.half);
   TileRest rest = wide_rest(g0, g1, total > (uint32_t)CAP);
   if (total > (uint32_t)CAP) {
     for (uint32_t g = g0 + tid; g < g1; g += kWideThreads) L.cnt[g] = kNlInvalid;
@@ -1661,7 +1700,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
   } else {
     // as omega_tile; .w: the slot's global index (velocities are gathered from L2), of the
     // sentinel the block's first particle (its pair terms are zero)
-    const uint32_t m = C.disp ? C.built[blk] : kNoCarry;
+    const uint32_t m = C.disp && !own.half ? C.built[blk] : kNoCarry;
     const bool carry = m != kNoCarry;
     tile_load<5, CAP, TeamWide>(P, sh, total, Q, lds.q, nullptr, 0u,
                                 [](uint32_t gi) { return __uint_as_float(gi); }, C.disp ? C.bounds(C.pass) : nullptr,
@@ -1670,7 +1709,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
     const bool calm = C.disp && tile_keeps_lists<5>(P, sh);
     const bool keep = carry && calm;
     if (tid == 0 && C.disp) {
-      C.mode[blk] = calm ? 1u : 0u;
+      C.mode[blk] = calm && !own.half ? 1u : 0u;  // halves do not carry: both write 0
       if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                            (unsigned long long)(g1 - g0));
     }
@@ -2097,7 +2136,7 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
                                              uint32_t* __restrict__ flag, unsigned long long* __restrict__ stats,
                                              uint32_t* tally, TileShared<BITS>& sh, float4* s_q) {
   using G = TileGeom<BITS>;
-  constexpr int CAP = TileCap<BITS>::value;
+  constexpr int CAP = TileCap<BITS>::adjoint;
   constexpr uint32_t kMax = kAdjLanes * kAdjListMax;
   const uint32_t total = tile_setup<BITS, TeamBlock>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
@@ -2200,8 +2239,8 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
 // halo cell; slots at or past the halo size are the forward's padding, and the
 // forward's solid bit becomes kAdjSolid.  A particle without a forward list
 // (over the neighbour cap, more pairs than a forward list holds, or in a block
-// beyond a small tile's capacity) and a block beyond the tile capacity are left
-// to k_tile_adjlist_redo: the block is appended to redo (redo[0]: the count).
+// beyond a small tile's capacity) and a block beyond the tile capacity (whose halves'
+// slots are not the block's) are left to k_tile_adjlist_redo: the block is appended to redo (redo[0]: the count).
 //
 // adjlist_forward_tile: a thread per particle, which deals the entries as
 // adjlist_particle does.
@@ -2392,15 +2431,15 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_adjlist_redo(DevParams P,
                                                                     AdjList L, uint32_t* __restrict__ flag,
                                                                     unsigned long long* __restrict__ stats,
                                                                     const uint32_t* __restrict__ redo) {
-  constexpr int CAP = TileCap<BITS>::value;
-  __shared__ TileLds<BITS, false> lds;
+  constexpr int CAP = TileCap<BITS>::adjoint;
+  __shared__ TileRegion<BITS, TileCap<BITS>::adjoint, false> lds;
   __shared__ uint32_t s_tally[kAdjTallies];
   tally_begin(s_tally);
   const uint32_t count = redo[0];
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
     __syncthreads();  // the previous block's halo is done with (and the tallies are cleared)
-    TileShared<BITS>& sh = lds.big.sh;
-    float4* s_q = lds.big.q;
+    TileShared<BITS>& sh = lds.sh;
+    float4* s_q = lds.q;
     const uint32_t total = tile_setup<BITS, TeamBlock>(P, redo[1u + i], cs, ce, sh);
     if (total > (uint32_t)CAP) {
       const uint32_t m = (sh.g1 - sh.g0) * kAdjLanes;
@@ -2411,7 +2450,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_adjlist_redo(DevParams P,
     tile_load<BITS, CAP, TeamBlock>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
     __syncthreads();
     for (uint32_t g = sh.g0 + threadIdx.x; g < sh.g1; g += kTileThreads) {
-      if (F.cnt[g] != kNlInvalid) continue;
+      if (F.cnt[g] != kNlInvalid && total <= (uint32_t)TileCap<BITS>::value) continue;  // converted
       int h;
       uint32_t slot;
       tile_locate<BITS>(sh, keys[g], g, h, slot);
@@ -2442,7 +2481,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
                                                   uint32_t* tally, TileShared<BITS>& sh, float4* s_q,
                                                   uint32_t (*s_part)[kTileThreads]) {
   using G = TileGeom<BITS>;
-  constexpr int CAP = TileCap<BITS>::value;
+  constexpr int CAP = TileCap<BITS>::adjoint;
   constexpr uint32_t kMax = kAdjLanes * kAdjListMax;
   const uint32_t total = tile_setup<BITS, TeamWide>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
@@ -2560,7 +2599,7 @@ __global__ __launch_bounds__(kWideThreads) void k_tile_adjlist_wide(DevParams P,
                                                                     const uint32_t* __restrict__ ce, AdjList L,
                                                                     uint32_t* __restrict__ flag,
                                                                     unsigned long long* __restrict__ stats) {
-  __shared__ TileRegion<BITS, TileCap<BITS>::value, false> lds;
+  __shared__ TileRegion<BITS, TileCap<BITS>::adjoint, false> lds;
   __shared__ uint32_t s_part[kWideParts][kTileThreads];
   __shared__ uint32_t s_occ;
   __shared__ uint32_t s_tally[kAdjTallies];
@@ -2601,7 +2640,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_adjlist(DevParams P, uint
                                                                const uint32_t* __restrict__ ce, AdjList L,
                                                                uint32_t* __restrict__ flag,
                                                                unsigned long long* __restrict__ stats) {
-  __shared__ TileLds<BITS, false> lds;
+  __shared__ TileRegion<BITS, TileCap<BITS>::adjoint, false> lds;
   __shared__ uint32_t s_occ;
   __shared__ uint32_t s_tally[kAdjTallies];
   constexpr uint32_t kCells = 1u << BITS;
@@ -2620,7 +2659,7 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_adjlist(DevParams P, uint
     for (uint32_t i = 0; i < kPer; ++i) {
       if (!((occ >> i) & 1u)) continue;
       adjlist_tile<BITS>(P, blockIdx.x + (i0 + i) * gridDim.x, Q, keys, cs, ce, L, flag, stats, s_tally,
-                         lds.big.sh, lds.big.q);
+                         lds.sh, lds.q);
       __syncthreads();
     }
     __syncthreads();
