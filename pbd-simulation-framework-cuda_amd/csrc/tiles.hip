@@ -1823,7 +1823,8 @@ hipError_t launch_tile_lambda(hipStream_t st, int bits, uint32_t grid, bool stri
   dim3 g(grid), b(kTileThreads);
   const NeighbourList L = nlist(B);
   // the first pass (pass 0) builds every list; the later ones follow `pass` delta-p passes
-  if (pass > kCarryPasses || first != (pass == 0) || (carry && !(B.DISP && B.BUILT && B.MODE)))
+  // (carried lists hold the bounds of kCarryPasses passes, any other step has any number)
+  if (first != (pass == 0) || (carry && (pass > kCarryPasses || !(B.DISP && B.BUILT && B.MODE))))
     return hipErrorInvalidValue;
   const Carry C = carry_of(B, pass, carry);
 #define PBD_LAMBDA(BITS_, F_, S_, PH_)                                                                           \
@@ -1963,7 +1964,7 @@ hipError_t launch_tile_final(hipStream_t st, int bits, uint32_t grid, bool strid
 hipError_t launch_wide_lambda(hipStream_t st, uint32_t grid, const DevParams& P, const TileList& T,
                               const StepBuffers& B, const float4* Q, const uint32_t* keys, bool first, bool carry,
                               uint32_t pass) {
-  if (pass > kCarryPasses || first != (pass == 0) || (carry && !(B.DISP && B.BUILT && B.MODE)) || P.phased)
+  if (first != (pass == 0) || (carry && (pass > kCarryPasses || !(B.DISP && B.BUILT && B.MODE))) || P.phased)
     return hipErrorInvalidValue;
   const Carry C = carry_of(B, pass, carry);
   if (first)
