@@ -7,13 +7,14 @@
 //   1. the lanes look up a cell each, in the stencil's order; a scan of the counts
 //      gives every neighbour its place in the particle's list, which is the order
 //      the walk visits (27 contact cells, then the shells, cut off at
-//      maxNeighboursPerParticle);
+//      maxNeighboursPerParticle); 256 places of it are in LDS at a time;
 //   2. the lanes form the terms of 64 pairs at a time;
 //   3. one lane per component of the sums adds the terms one by one, in list order
 //      and with the walk's fused operations, so the sums are the walk's bit for bit.
 // The 13,824-particle scene: lambda 116 -> 20 us, delta-p 123 -> 21, omega 116 -> 17,
 // final 142 -> 23 us, bound by the latency of the dependent loads (keys, cells, positions)
-// over three rounds of resident waves.  A wave issues about ten times the instructions of
+// over three rounds of resident waves.  Compressed to 3.5 particles a cell (lists of 430):
+// 321 us a step, 59,319 particles 974 us; with a thread per particle 1936 and 1952 us.  A wave issues about ten times the instructions of
 // a particle's thread, so the passes go to kernels.hip above kWaveParticles.
 #include <hip/hip_runtime.h>
 
@@ -27,7 +28,7 @@ namespace {
 constexpr uint32_t kWaves = 4;          // of a workgroup, a particle each
 constexpr int kWaveStencil = 2;         // stencils of up to 5 x 5 x 5 cells
 constexpr uint32_t kWaveCells = 125;
-constexpr uint32_t kWaveList = 256;     // neighbours a wave's list holds; more are walked by one lane
+constexpr uint32_t kWaveList = 256;     // neighbours a wave's list holds at a time
 constexpr uint32_t kMaxTerms = 8;       // components of a pass's sums
 
 // The stencil's cells in the walk's order: the 27 contact cells, then shell 2.
@@ -68,25 +69,31 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// The neighbour list of particle s; returns its length (at most P.cap; only the first
-// kWaveList entries are stored), nc: how many of them are contacts.
-__device__ __forceinline__ uint32_t wave_list(const DevParams& P, uint32_t s, const CellFrame& f,
-                                              const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
-                                              WaveLds& L, uint32_t& nc) {
+// The neighbour list of particle s as the lanes hold it: of cell (chunk k, lane) its
+// particles st .. en - 1, from list place `at` on (s itself left out).
+struct WaveCells {
+  static constexpr uint32_t kChunks = (kWaveCells + 63u) / 64u;
+  uint32_t st[kChunks], en[kChunks], at[kChunks], first;
+};
+
+// Looks the cells up; returns the list's length (at most P.cap), nc: how many are contacts.
+__device__ __forceinline__ uint32_t wave_cells(const DevParams& P, uint32_t s, const CellFrame& f,
+                                               const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
+                                               WaveCells& W, uint32_t& nc) {
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t first = (P.gates & G_FIND_CONTACTS) ? 0u : 27u;
+  W.first = (P.gates & G_FIND_CONTACTS) ? 0u : 27u;
   const uint32_t last = (P.gates & G_FIND_NEIGHBOURS) && P.kw > 1 ? kWaveCells : 27u;
-  const uint32_t keep = min(P.cap, kWaveList);
   uint32_t base = 0u, contacts = 0u;
-  for (uint32_t c0 = first; c0 < last; c0 += 64u) {
-    const uint32_t c = c0 + lane;
+#pragma unroll
+  for (uint32_t k = 0; k < WaveCells::kChunks; ++k) {
+    const uint32_t c = W.first + 64u * k + lane;
     uint32_t st = 0u, en = 0u, cnt = 0u;
     if (c < last) {
       const int dx = kStencil.d[c][0], dy = kStencil.d[c][1], dz = kStencil.d[c][2];
       const uint32_t nx = f.ix + (uint32_t)dx, ny = f.iy + (uint32_t)dy, nz = f.iz + (uint32_t)dz;
       if (nx < P.dims[0] && ny < P.dims[1] && nz < P.dims[2]) {
-        const uint32_t k = morton3(nx, ny, nz);
-        const uint32_t s0 = cs[k], e0 = ce[k];
+        const uint32_t key = morton3(nx, ny, nz);
+        const uint32_t s0 = cs[key], e0 = ce[key];
         if (s0 != 0xFFFFFFFFu) {
           st = s0;
           en = e0;
@@ -100,19 +107,31 @@ __device__ __forceinline__ uint32_t wave_list(const DevParams& P, uint32_t s, co
       const uint32_t y = __shfl_up(x, o);
       if (lane >= o) x += y;
     }
-    uint32_t i = base + x - cnt;
-    for (uint32_t j = st; j < en && i < keep; ++j) {
-      if (j == s) continue;
-      L.j[i] = j;
-      L.cell[i] = (uint8_t)c;
-      ++i;
-    }
-    if (c0 == 0u) contacts = __shfl(x, 26);
+    W.st[k] = st;
+    W.en[k] = en;
+    W.at[k] = base + x - cnt;
+    if (k == 0u && W.first == 0u) contacts = __shfl(x, 26);
     base += __shfl(x, 63);
   }
-  wave_fence();
   nc = min(contacts, P.cap);
   return min(base, P.cap);
+}
+
+// Entries w0 .. min(w0 + kWaveList, n) - 1 of the list to L.
+__device__ __forceinline__ void wave_list(const WaveCells& W, uint32_t s, uint32_t w0, uint32_t n, WaveLds& L) {
+  const uint32_t lane = threadIdx.x & 63u, end = min(n, w0 + kWaveList);
+#pragma unroll
+  for (uint32_t k = 0; k < WaveCells::kChunks; ++k) {
+    uint32_t i = max(W.at[k], w0), j = W.st[k] + (i - W.at[k]);
+    if (s >= W.st[k] && s < j) ++j;  // s is among the entries before
+    for (; j < W.en[k] && i < end; ++j) {
+      if (j == s) continue;
+      L.j[i - w0] = j;
+      L.cell[i - w0] = (uint8_t)(W.first + 64u * k + lane);
+      ++i;
+    }
+  }
+  wave_fence();
 }
 
 // Base vector of neighbour list entry i: p_s - p_j = b - q_j.
@@ -123,38 +142,45 @@ __device__ __forceinline__ float3 wave_base(const DevParams& P, const CellFrame&
                      q.z + (f.cz - frame_corner(P, f.oz, nz)));
 }
 
-// The sums of N components over the list: terms(i, j, r, put) forms pair i's terms,
-// put(c, u, v) the addition of u v to component c (v = 1: of u, exactly); a component
-// that it does not put gets nothing.  Returns component (lane) of the sums.
+// The sums of N components over the first n entries of the list, kWaveList of them at a
+// time: terms(i, j, r, put) forms pair i's terms, put(c, u, v) the addition of u v to
+// component c (v = 1: of u, exactly); a component that it does not put gets nothing.
+// Returns component (lane) of the sums.
 template <uint32_t N, class Terms>
-__device__ __forceinline__ float wave_sums(const DevParams& P, const CellFrame& f, const float4* __restrict__ Q,
-                                           float4 q, uint32_t n, WaveLds& L, Terms terms) {
+__device__ __forceinline__ float wave_sums(const DevParams& P, uint32_t s, const CellFrame& f, const WaveCells& W,
+                                           const float4* __restrict__ Q, float4 q, uint32_t n, WaveLds& L,
+                                           Terms terms) {
   static_assert(N <= kMaxTerms, "components");
   const uint32_t lane = threadIdx.x & 63u;
   float acc = 0.0f;
-  for (uint32_t k = 0; k < n; k += 64u) {
-    const uint32_t m = min(n - k, 64u);
-    if (lane < m) {
-      const uint32_t j = L.j[k + lane];
-      const float4 qj = Q[j];
-      const float3 b = wave_base(P, f, q, L.cell[k + lane]);
-      terms(k + lane, j, b.x - qj.x, b.y - qj.y, b.z - qj.z,
-            [&](uint32_t c, float u, float v) { L.term[c][lane] = make_float2(u, v); });
-    }
-    wave_fence();
-    if (lane < N) {
-      const float2* t = L.term[lane];
-      uint32_t i = 0;
-      for (; i + 8u <= m; i += 8u) {
-        float2 w[8];
-#pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u) w[u] = t[i + u];
-#pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u) acc = fmaf(w[u].x, w[u].y, acc);
+#pragma unroll 1
+  for (uint32_t w0 = 0; w0 < n; w0 += kWaveList) {
+    wave_list(W, s, w0, n, L);
+    const uint32_t held = min(n - w0, kWaveList);
+    for (uint32_t k = 0; k < held; k += 64u) {
+      const uint32_t m = min(held - k, 64u);
+      if (lane < m) {
+        const uint32_t j = L.j[k + lane];
+        const float4 qj = Q[j];
+        const float3 b = wave_base(P, f, q, L.cell[k + lane]);
+        terms(w0 + k + lane, j, b.x - qj.x, b.y - qj.y, b.z - qj.z,
+              [&](uint32_t c, float u, float v) { L.term[c][lane] = make_float2(u, v); });
       }
-      for (; i < m; ++i) acc = fmaf(t[i].x, t[i].y, acc);
+      wave_fence();
+      if (lane < N) {
+        const float2* t = L.term[lane];
+        uint32_t i = 0;
+        for (; i + 8u <= m; i += 8u) {
+          float2 w[8];
+#pragma unroll
+          for (uint32_t u = 0; u < 8u; ++u) w[u] = t[i + u];
+#pragma unroll
+          for (uint32_t u = 0; u < 8u; ++u) acc = fmaf(w[u].x, w[u].y, acc);
+        }
+        for (; i < m; ++i) acc = fmaf(t[i].x, t[i].y, acc);
+      }
+      wave_fence();
     }
-    wave_fence();
   }
   return acc;
 }
@@ -174,13 +200,10 @@ __global__ __launch_bounds__(64 * kWaves) void k_wave_lambda(DevParams P, const 
   WaveLds& L = lds[threadIdx.x >> 6];
   const CellFrame f = make_frame(P, keys[s]);
   const float4 q = Q[s];
+  WaveCells W;
   uint32_t nc;
-  const uint32_t n = wave_list(P, s, f, cs, ce, L, nc);
-  if (n > kWaveList) {
-    if (lane == 0u) lambda_particle<REF, FIRST>(P, s, Q, keys, cs, ce, lam, dens, ncnt, ccnt);
-    return;
-  }
-  const float a = wave_sums<5>(P, f, Q, q, n, L, [&](uint32_t, uint32_t, float rx, float ry, float rz, auto put) {
+  const uint32_t n = wave_cells(P, s, f, cs, ce, W, nc);
+  const float a = wave_sums<5>(P, s, f, W, Q, q, n, L, [&](uint32_t, uint32_t, float rx, float ry, float rz, auto put) {
     const float r2 = length_sq(rx, ry, rz);
     float hr4;
     const float g = grad_factor<REF>(P, r2, hr4);
@@ -197,10 +220,10 @@ __global__ __launch_bounds__(64 * kWaves) void k_wave_lambda(DevParams P, const 
   A.gz = __shfl(a, 3);
   A.B = __shfl(a, 4);
   if (lane != 0u) return;
-  float W;
-  lam[s] = lambda_finish<REF>(P, A, W, scene_eps(P, keys[s]));
+  float rho;
+  lam[s] = lambda_finish<REF>(P, A, rho, scene_eps(P, keys[s]));
   if (FIRST) {
-    dens[s] = W;
+    dens[s] = rho;
     ncnt[s] = n;
     ccnt[s] = nc;
   }
@@ -218,17 +241,14 @@ __global__ __launch_bounds__(64 * kWaves) void k_wave_delta(
   WaveLds& L = lds[threadIdx.x >> 6];
   const CellFrame f = make_frame(P, keys[s]);
   const float4 q = Q[s];
+  WaveCells W;
   uint32_t nc;
-  const uint32_t all = wave_list(P, s, f, cs, ce, L, nc);
-  if (all > kWaveList) {
-    if (lane == 0u) delta_particle<REF, DELTA, COLLIDE>(P, flags, s, Q, QX, lam, keys, cs, ce, Qo, QXo, DP, VS);
-    return;
-  }
+  const uint32_t all = wave_cells(P, s, f, cs, ce, W, nc);
   // without DELTA only the contacts count
   const uint32_t n = DELTA ? all : nc;
   const float li = DELTA ? lam[s] : 0.0f;
   constexpr uint32_t N = (DELTA ? 3u : 0u) + (COLLIDE ? 3u : 0u), C = DELTA ? 3u : 0u;
-  const float a = wave_sums<N>(P, f, Q, q, n, L, [&](uint32_t i, uint32_t j, float rx, float ry, float rz, auto put) {
+  const float a = wave_sums<N>(P, s, f, W, Q, q, n, L, [&](uint32_t i, uint32_t j, float rx, float ry, float rz, auto put) {
     const float r2 = length_sq(rx, ry, rz);
     if (DELTA) {
       const float w = P.wc * w_unnorm<REF>(P, r2);
@@ -280,13 +300,10 @@ __global__ __launch_bounds__(64 * kWaves) void k_wave_omega(DevParams P, const f
   WaveLds& L = lds[threadIdx.x >> 6];
   const CellFrame f = make_frame(P, keys[s]);
   const float4 q = Q[s], vi = VS[s];
+  WaveCells W;
   uint32_t nc;
-  const uint32_t n = wave_list(P, s, f, cs, ce, L, nc);
-  if (n > kWaveList) {
-    if (lane == 0u) omega_particle<REF>(P, s, Q, VS, keys, cs, ce, OM);
-    return;
-  }
-  const float a = wave_sums<3>(P, f, Q, q, n, L, [&](uint32_t, uint32_t j, float rx, float ry, float rz, auto put) {
+  const uint32_t n = wave_cells(P, s, f, cs, ce, W, nc);
+  const float a = wave_sums<3>(P, s, f, W, Q, q, n, L, [&](uint32_t, uint32_t j, float rx, float ry, float rz, auto put) {
     const float4 vj = VS[j];
     const float vx = vj.x - vi.x, vy = vj.y - vi.y, vz = vj.z - vi.z;
     float hr4;
@@ -317,14 +334,10 @@ __global__ __launch_bounds__(64 * kWaves) void k_wave_final(
   const CellFrame f = make_frame(P, keys[s]);
   const float4 q = Q[s], vi = VS[s];
   const float4 oi = vort ? OM[s] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  WaveCells W;
   uint32_t nc, n = 0u;
-  if (vort || xsph) n = wave_list(P, s, f, cs, ce, L, nc);
-  if (n > kWaveList) {
-    if (lane == 0u)
-      final_particle<REF>(P, flags, s, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo);
-    return;
-  }
-  const float a = wave_sums<7>(P, f, Q, q, n, L, [&](uint32_t, uint32_t j, float rx, float ry, float rz, auto put) {
+  if (vort || xsph) n = wave_cells(P, s, f, cs, ce, W, nc);
+  const float a = wave_sums<7>(P, s, f, W, Q, q, n, L, [&](uint32_t, uint32_t j, float rx, float ry, float rz, auto put) {
     float w = 0.0f;
     float4 dv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (xsph) {
