@@ -389,47 +389,73 @@ __device__ __forceinline__ uint32_t tile_class(uint32_t b, uint32_t nflags, cons
 // large (kTileCrowded; as a small one every pass took it particle by particle from global
 // memory: 1M splash with small tiles of up to 64, 1862 us, with the marks 1438), and a
 // large one whose halo is more than a tile holds is two items (kTileSplit).  Blocks of at
-// most kTileSmallSure particles stay small.  kHaloLanes lanes a block, all of a lane's
-// cells in flight at once; an empty block costs its lanes one load.  Bound by latency: 6
-// to 9 us up to 1M particles.
+// most kTileSmallSure particles stay small.  A wave takes F flags, a lane each, and counts
+// the halos of those that need it four at a time, kHaloLanes lanes a block, all of a
+// lane's cells in flight at once.
 constexpr uint32_t kHaloLanes = 16;
-template <int BITS>
+// Flags of a wave.  Where the blocks fill few waves, four blocks a wave are one chain of two
+// loads (6 to 9 us up to 1M particles in a box that they fill); with more flags the chain
+// repeats, but the waves that only sweep empty blocks, of a box far larger than its fluid,
+// are fewer.  us a step at 4 / 16 / 64 flags: 2K 167 / 173 / 173, 211K splash (45K flags) 472
+// / 485 / 509, 1M column (41K) 949 / 951 / 988, 16M column (0.3M) 13557 / 13370 / 13368, 1.2M
+// in a 300-cell box (2.2M) 1818 / 1759 / 1795, 5K in a 1024^3-cell box (34M) 3222 / 2502 / 2318.
+static uint32_t classify_flags(uint32_t nflags) {
+  return nflags <= (1u << 17) ? 4u : nflags <= (1u << 22) ? 16u : 64u;
+}
+template <int BITS, uint32_t F>
 __global__ __launch_bounds__(256) void k_tile_classify(DevParams P, uint32_t nflags, uint32_t* __restrict__ start,
                                                        const uint32_t* __restrict__ end, uint32_t small_max,
                                                        const uint32_t* __restrict__ cs,
                                                        const uint32_t* __restrict__ ce, uint32_t* __restrict__ bcount) {
   using G = TileGeom<BITS>;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, b = i / kHaloLanes, l = i % kHaloLanes;
-  uint32_t s = b < nflags ? start[b] : 0u;
-  const uint32_t own = s ? end[b] - tile_begin(s) : 0u;
-  const uint32_t first = b << BITS;
-  if (own > min(kTileSmallSure, small_max)) {
-    const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
-    uint32_t halo = 0u;
+  static_assert(F <= 64u && kTileCompactChunk % F == 0u, "a wave's flags lie in one chunk of the compaction");
+  const uint32_t lane = threadIdx.x & 63u, l = lane % kHaloLanes;
+  const uint32_t base = (blockIdx.x * (blockDim.x / 64u) + (threadIdx.x >> 6)) * F;
+  const uint32_t s = lane < F && base + lane < nflags ? start[base + lane] : 0u;
+  const uint32_t own = s ? end[base + lane] - tile_begin(s) : 0u;
+  uint32_t mark = 0u;
+  for (uint64_t todo = __ballot(own > min(kTileSmallSure, small_max)); todo;) {
+    // the next four blocks, one for each group of lanes
+    uint32_t k = 64u;
 #pragma unroll
-    for (uint32_t r = 0; r < ((uint32_t)G::NH + kHaloLanes - 1u) / kHaloLanes; ++r) {
-      const uint32_t c = r * kHaloLanes + l;
-      if (c >= (uint32_t)G::NH) break;
-      const int cx = ix0 - 1 + (int)c / G::SX, cy = iy0 - 1 + ((int)c / G::SY) % G::HY, cz = iz0 - 1 + (int)c % G::HZ;
-      if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
-        const uint32_t k = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
-        const uint32_t a = cs[k], e = ce[k];
-        halo += a != 0xFFFFFFFFu ? e - a : 0u;
+    for (uint32_t i = 0; i < 64u / kHaloLanes; ++i)
+      if (todo) {
+        if (lane / kHaloLanes == i) k = (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1u;
+      }
+    const uint32_t first = (base + k) << BITS;
+    uint32_t halo = 0u;
+    if (k < 64u) {
+      const int ix0 = (int)compact10(first >> 2), iy0 = (int)compact10(first >> 1), iz0 = (int)compact10(first);
+#pragma unroll
+      for (uint32_t r = 0; r < ((uint32_t)G::NH + kHaloLanes - 1u) / kHaloLanes; ++r) {
+        const uint32_t c = r * kHaloLanes + l;
+        if (c >= (uint32_t)G::NH) break;
+        const int cx = ix0 - 1 + (int)c / G::SX, cy = iy0 - 1 + ((int)c / G::SY) % G::HY, cz = iz0 - 1 + (int)c % G::HZ;
+        if (cx >= 0 && cy >= 0 && cz >= 0 && cx < (int)P.dims[0] && cy < (int)P.dims[1] && cz < (int)P.dims[2]) {
+          const uint32_t m = morton3((uint32_t)cx, (uint32_t)cy, (uint32_t)cz);
+          const uint32_t a = cs[m], e = ce[m];
+          halo += a != 0xFFFFFFFFu ? e - a : 0u;
+        }
       }
     }
 #pragma unroll
     for (uint32_t o = kHaloLanes / 2u; o; o >>= 1) halo += (uint32_t)__shfl_xor((int)halo, (int)o, (int)kHaloLanes);
-    uint32_t mark = 0u;
-    if (own <= small_max && halo > (uint32_t)TileCap<BITS>::small) mark = kTileCrowded;
-    if (BITS == 5 && (own > small_max || mark) && halo > (uint32_t)TileCap<BITS>::value) mark |= kTileSplit;
-    if (mark && l == 0u) start[b] = s | mark;
-    s |= mark;
+    // to the block's own lane
+#pragma unroll
+    for (uint32_t i = 0; i < 64u / kHaloLanes; ++i) {
+      const uint32_t h = (uint32_t)__shfl((int)halo, (int)(i * kHaloLanes)), at = (uint32_t)__shfl((int)k, (int)(i * kHaloLanes));
+      if (at != lane) continue;
+      if (own <= small_max && h > (uint32_t)TileCap<BITS>::small) mark = kTileCrowded;
+      if (BITS == 5 && (own > small_max || mark) && h > (uint32_t)TileCap<BITS>::value) mark |= kTileSplit;
+    }
   }
+  if (mark) start[base + lane] = s | mark;
   uint32_t c = 0u;
-  if (s && l == 0u) c = !(s & kTileCrowded) && own <= small_max ? 0x10000u : s & kTileSplit ? 2u : 1u;
+  if (s) c = !(mark & kTileCrowded) && own <= small_max ? 0x10000u : mark & kTileSplit ? 2u : 1u;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o);
-  if ((threadIdx.x & 63u) == 0u && c) atomicAdd(&bcount[b / kTileCompactChunk], c);
+  if (lane == 0u && c) atomicAdd(&bcount[base / kTileCompactChunk], c);
 }
 
 __global__ __launch_bounds__(1024) void k_tile_emit(uint32_t nflags, const uint32_t* __restrict__ start,
@@ -509,11 +535,23 @@ hipError_t launch_tile_compact(hipStream_t st, int bits, const DevParams& P, con
                                uint32_t* start, const uint32_t* end, uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
                                uint32_t* count) {
   if (small_max > kTileSmall) return hipErrorInvalidValue;  // a small tile is one wave, one particle per lane
-  const dim3 g((uint32_t)(((size_t)nflags * kHaloLanes + 255u) / 256u)), t(256);
-  if (bits == 5)
-    hipLaunchKernelGGL(k_tile_classify<5>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend, bcount);
-  else
-    hipLaunchKernelGGL(k_tile_classify<6>, g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend, bcount);
+  const uint32_t F = classify_flags(nflags);
+  const dim3 g((nflags + 4u * F - 1u) / (4u * F)), t(256);
+#define PBD_CLASSIFY(F_)                                                                                          \
+  if (bits == 5)                                                                                                  \
+    hipLaunchKernelGGL((k_tile_classify<5, F_>), g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend, \
+                       bcount);                                                                                   \
+  else                                                                                                            \
+    hipLaunchKernelGGL((k_tile_classify<6, F_>), g, t, 0, st, P, nflags, start, end, small_max, B.cstart, B.cend, \
+                       bcount)
+  if (F == 4u) {
+    PBD_CLASSIFY(4u);
+  } else if (F == 16u) {
+    PBD_CLASSIFY(16u);
+  } else {
+    PBD_CLASSIFY(64u);
+  }
+#undef PBD_CLASSIFY
   const uint32_t blocks = (nflags + kTileCompactChunk - 1u) / kTileCompactChunk;
   hipLaunchKernelGGL(k_tile_emit, dim3(blocks), dim3(1024), 0, st, nflags, start, end, small_max, bcount, large, small,
                      count);
