@@ -787,7 +787,10 @@ __device__ __forceinline__ void nl_visit(const NeighbourList& L, uint32_t g, uin
   const uint32_t nc = n >> 3;
   if (nc == 0) return;
   for (uint32_t c = 1; c <= nc; ++c) {
-    const uint4 nx = c < nc ? p[(size_t)c * L.cap] : w;
+    // (as a conditional expression this is a flat load from a selected address, with w in
+    // scratch, and the next read of the LDS waits for it)
+    uint4 nx = w;
+    if (c < nc) nx = p[(size_t)c * L.cap];
     body(w.x & 0xFFFFu);
     body(w.x >> 16);
     body(w.y & 0xFFFFu);
@@ -2333,7 +2336,8 @@ __device__ __forceinline__ void adjlist_forward_tile(const DevParams& P, uint32_
       bool done = nc == 0u;
       uint4 v = nc ? p[0] : make_uint4(0u, 0u, 0u, 0u);
       for (uint32_t k = 0; k < nc && !done; ++k) {
-        const uint4 nx = k + 1u < nc ? p[(size_t)(k + 1u) * F.cap] : v;
+        uint4 nx = v;  // as nl_visit
+        if (k + 1u < nc) nx = p[(size_t)(k + 1u) * F.cap];
         const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
         v = nx;
 #pragma unroll
