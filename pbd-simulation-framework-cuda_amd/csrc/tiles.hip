@@ -36,29 +36,43 @@ struct TileGeom {
 
 constexpr uint32_t kTileThreads = 256;
 
+// The thread's index.  LOOP, for a kernel whose workgroups take tile after tile: as a value
+// that the compiler cannot trace to the hardware's.  What a tile derives from the index
+// (halo cells, cell groups, addresses) is otherwise kept in registers over the whole loop:
+// 143 to 172 VGPRs in the 2^5-cell passes of a capped grid, 110 to 127 so (with a bound of
+// four waves for omega and final).  us, before / now: four steps of 256 scenes of 2K to 64K
+// 54940 / 45790, a step of 1.2M particles in a 300-cell box 1818 / 1360, its splash 2650 / 2018.
+template <bool LOOP>
+__device__ __forceinline__ uint32_t thread_index() {
+  uint32_t t = threadIdx.x;
+  if (LOOP) asm volatile("" : "+v"(t));
+  return t;
+}
+
 // A team walks one tile: the whole workgroup for a large tile, one wave for a
 // small one.  A wave's LDS accesses complete in order, so a wave team needs no
 // hardware barrier, only one the compiler does not move memory accesses across.
-template <uint32_t N>
+template <uint32_t N, bool LOOP = false>
 struct TeamBlockN {
   static constexpr uint32_t kSize = N;
-  static constexpr uint32_t kLoadUnroll = 2;  // halo loads in flight per thread
-  static __device__ __forceinline__ uint32_t tid() { return threadIdx.x; }
+  static __device__ __forceinline__ uint32_t tid() { return thread_index<LOOP>(); }
   static __device__ __forceinline__ void sync() { __syncthreads(); }
 };
 using TeamBlock = TeamBlockN<kTileThreads>;
 // The reverse-mode list builder for small scenes: four threads per particle.
 constexpr uint32_t kWideThreads = 1024;
 using TeamWide = TeamBlockN<kWideThreads>;
-struct TeamWave {
+template <bool LOOP = false>
+struct TeamWaveT {
   static constexpr uint32_t kSize = 64;
-  static constexpr uint32_t kLoadUnroll = 4;
-  static __device__ __forceinline__ uint32_t tid() { return threadIdx.x & 63u; }
+  static constexpr uint32_t kLoadUnroll = 4;  // halo loads in flight per lane
+  static __device__ __forceinline__ uint32_t tid() { return thread_index<LOOP>() & 63u; }
   static __device__ __forceinline__ void sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
 };
+using TeamWave = TeamWaveT<>;
 
 template <int BITS>
 struct TileShared {
@@ -1041,11 +1055,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_lambda(DevParams P, TileL
     if (mode == 0) break;
     TileRest rest;
     if (mode == 1) {
-      rest = lambda_tile<BITS, FIRST, PH, TeamBlock, TileCap<BITS>::value>(P, T, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
+      rest = lambda_tile<BITS, FIRST, PH, TeamBlockN<kTileThreads, STRIDE>, TileCap<BITS>::value>(P, T, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
                                                                        ccnt, C, lds.big.sh, lds.big.q);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = lambda_tile<BITS, FIRST, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
+      rest = lambda_tile<BITS, FIRST, PH, TeamWaveT<STRIDE>, TileCap<BITS>::small>(P, T, blk, L, Q, keys, cs, ce, lam, dens, ncnt,
                                                                       ccnt, C, reg.sh, reg.q);
     }
     rest.visit([&](uint32_t g) __attribute__((always_inline)) {
@@ -1171,12 +1185,12 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_delta(DevParams P, TileLi
     if (mode == 0) break;
     TileRest rest;
     if (mode == 1) {
-      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamBlock, TileCap<BITS>::value>(
+      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamBlockN<kTileThreads, STRIDE>, TileCap<BITS>::value>(
           P, T, blk, L, use_list, flags, Q, QX, lam, keys, cs, ce, Qo, QXo, DP, VS, C, lds.big.sh, lds.big.q,
           GI ? lds.big.gi : nullptr);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, use_list, flags, Q, QX, lam,
+      rest = delta_tile<BITS, COLLIDE, NS, PH, TeamWaveT<STRIDE>, TileCap<BITS>::small>(P, T, blk, L, use_list, flags, Q, QX, lam,
                                                                            keys, cs, ce, Qo, QXo, DP, VS, C, reg.sh,
                                                                            reg.q, GI ? reg.gi : nullptr);
     }
@@ -1302,7 +1316,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
 }
 
 template <int BITS, bool XSPH, bool STRIDE, bool PH>
-__global__ __launch_bounds__(kTileThreads) void k_tile_omega(DevParams P, TileList T, NeighbourList L,
+__global__ __launch_bounds__(kTileThreads, STRIDE && BITS == 5 ? 4 : 1) void k_tile_omega(DevParams P, TileList T, NeighbourList L,
                                                              const float4* __restrict__ Q,
                                                              const float4* __restrict__ VS,
                                                              const uint32_t* __restrict__ keys,
@@ -1320,11 +1334,11 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_omega(DevParams P, TileLi
     if (mode == 0) break;
     TileRest rest;
     if (mode == 1) {
-      rest = omega_tile<BITS, XSPH, PH, TeamBlock, TileCap<BITS>::value>(P, T, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
+      rest = omega_tile<BITS, XSPH, PH, TeamBlockN<kTileThreads, STRIDE>, TileCap<BITS>::value>(P, T, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
                                                                      lds.big.sh, lds.big.q, lds.big.gi);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = omega_tile<BITS, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
+      rest = omega_tile<BITS, XSPH, PH, TeamWaveT<STRIDE>, TileCap<BITS>::small>(P, T, blk, L, Q, VS, keys, cs, ce, OM, Vo, C,
                                                                     reg.sh, reg.q, reg.gi);
     }
     rest.visit([&](uint32_t g) __attribute__((always_inline)) {
@@ -1416,7 +1430,7 @@ __device__ __forceinline__ TileRest final_tile(const DevParams& P, const TileLis
 }
 
 template <int BITS, bool VORT, bool XSPH, bool STRIDE, bool PH>
-__global__ __launch_bounds__(kTileThreads) void k_tile_final(
+__global__ __launch_bounds__(kTileThreads, STRIDE && BITS == 5 ? 4 : 1) void k_tile_final(
     DevParams P, TileList T, NeighbourList L, int use_list, uint32_t flags, const float4* __restrict__ Q,
     const float4* __restrict__ QX, const float4* __restrict__ VS, const float4* __restrict__ OM,
     const uint32_t* __restrict__ keys, const uint32_t* __restrict__ cs, const uint32_t* __restrict__ ce,
@@ -1432,12 +1446,12 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_final(
     if (mode == 0) break;
     TileRest rest;
     if (mode == 1) {
-      rest = final_tile<BITS, VORT, XSPH, PH, TeamBlock, TileCap<BITS>::value>(
+      rest = final_tile<BITS, VORT, XSPH, PH, TeamBlockN<kTileThreads, STRIDE>, TileCap<BITS>::value>(
           P, T, blk, L, use_list, flags, Q, QX, VS, OM, keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo, lds.big.sh, lds.big.q,
           lds.big.gi);
     } else {
       auto& reg = lds.small[threadIdx.x >> 6];
-      rest = final_tile<BITS, VORT, XSPH, PH, TeamWave, TileCap<BITS>::small>(P, T, blk, L, use_list, flags, Q, QX, VS, OM,
+      rest = final_tile<BITS, VORT, XSPH, PH, TeamWaveT<STRIDE>, TileCap<BITS>::small>(P, T, blk, L, use_list, flags, Q, QX, VS, OM,
                                                                           keys, cs, ce, CS, ncnt, Xo, Po, Vo, Co, Fo,
                                                                           reg.sh, reg.q, reg.gi);
     }

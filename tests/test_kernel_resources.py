@@ -49,3 +49,14 @@ def test_tile_passes_use_no_scratch(kernels):
     assert len(passes) > 50
     bad = {k: v[1] for k, v in passes.items() if v[1]}
     assert not bad, bad
+
+
+def test_capped_grid_passes_keep_four_waves(kernels):
+    """The passes whose workgroups take tile after tile (batches, large boxes) hold at most
+    128 registers a lane: four waves on a SIMD."""
+    stride = {"k_tile_lambda": r"<5, \w+, true, ", "k_tile_delta": r"<5, \w+, \d, true, ",
+              "k_tile_omega": r"<5, \w+, true, ", "k_tile_final": r"<5, \w+, \w+, true, "}
+    vgprs = {k: v[0] for k, v in kernels.items() for n, args in stride.items() if re.match(n + args, k)}
+    assert len(vgprs) == 12, sorted(vgprs)
+    bad = {k: v for k, v in vgprs.items() if v > 128}
+    assert not bad, bad
