@@ -825,9 +825,12 @@ __device__ __forceinline__ void nl_visit(const NeighbourList& L, uint32_t g, uin
 // past the range (still inside the LDS array); their bits are masked off.  A position
 // that is not a number is +NaN (canonical_nan), whose sign says out of range; the
 // caller drops the mask of a particle that is not finite itself (inf - inf is -NaN).
+// (The language leaves a NaN's sign open: that the hardware's instructions keep it through
+// the subtraction and the fused additions is what the tests of NaN neighbours hold.)
+template <uint32_t U = kScanUnroll>
 __device__ __forceinline__ uint32_t nl_mask(const float4* s_q, uint32_t a, uint32_t len, float qx, float qy, float qz,
                                             float r2max) {
-  constexpr uint32_t U = kScanUnroll;
+  static_assert(U <= kScanUnroll && 32u % U == 0u, "whole groups fill a mask");
   uint32_t m = 0u, k = 0u;
   do {
     float4 c[U];
@@ -2086,13 +2089,16 @@ __device__ __forceinline__ void tally_flush(const uint32_t* t, unsigned long lon
     atomicAdd(stats + kCounter[threadIdx.x], (unsigned long long)t[threadIdx.x]);
 }
 
-// In-range bits (lo, hi) of slots a .. b - 1 (1 <= b - a <= 64).
+// In-range bits (lo, hi) of slots a .. b - 1 (1 <= b - a <= 64).  Four candidates a group:
+// these builders keep a window of entries and two masks beside them, and eight take them
+// from four waves a SIMD to three (165 VGPRs; the reverse of two substeps of 729K particles
+// with its lists built here 4520 us, 4410 so with the team's opaque index).
 __device__ __forceinline__ void nl_column(const float4* s_q, uint32_t a, uint32_t b, float4 q, float r2max,
                                           uint32_t& lo, uint32_t& hi) {
   const uint32_t valid = fabsf(q.x) + fabsf(q.y) + fabsf(q.z) < __builtin_inff() ? 0xFFFFFFFFu : 0u;
   const uint32_t len = b - a;
-  lo = nl_mask(s_q, a, min(len, 32u), q.x, q.y, q.z, r2max) & valid;
-  hi = len > 32u ? nl_mask(s_q, a + 32u, len - 32u, q.x, q.y, q.z, r2max) & valid : 0u;
+  lo = nl_mask<4u>(s_q, a, min(len, 32u), q.x, q.y, q.z, r2max) & valid;
+  hi = len > 32u ? nl_mask<4u>(s_q, a + 32u, len - 32u, q.x, q.y, q.z, r2max) & valid : 0u;
 }
 
 // One particle's list: entries dealt to its lanes in turn, the last kAdjLanes
@@ -2194,7 +2200,7 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::adjoint;
   constexpr uint32_t kMax = kAdjLanes * kAdjListMax;
-  const uint32_t total = tile_setup<BITS, TeamBlock>(P, blk, cs, ce, sh);
+  const uint32_t total = tile_setup<BITS, TeamBlockN<kTileThreads, true>>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     // whole particles per pass of the loop: a particle's lanes are active together
@@ -2203,7 +2209,7 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
       adj_list_lane(P, Q, keys, cs, ce, L, flag, stats, g0 + u / kAdjLanes, u % kAdjLanes);
     return;
   }
-  tile_load<BITS, CAP, TeamBlock>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
+  tile_load<BITS, CAP, TeamBlockN<kTileThreads, true>>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
   __syncthreads();
   const uint32_t n = P.n;
   for (uint32_t g = g0 + threadIdx.x; g < g1; g += kTileThreads) {
@@ -2309,7 +2315,7 @@ __device__ __forceinline__ void adjlist_forward_tile(const DevParams& P, uint32_
                                                      uint32_t* __restrict__ redo, TileShared<BITS>& sh) {
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
-  const uint32_t total = tile_setup<BITS, TeamBlock>(P, blk, cs, ce, sh);
+  const uint32_t total = tile_setup<BITS, TeamBlockN<kTileThreads, true>>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     if (threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
@@ -2395,7 +2401,7 @@ __device__ __forceinline__ void adjlist_forward_tile_wide(const DevParams& P, ui
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
   static_assert(kNlRecordChunks == kAdjLanes && kAdjListMax == kAdjLanes, "a forward chunk is a row of the lanes");
-  const uint32_t total = tile_setup<BITS, TeamWide>(P, blk, cs, ce, sh);
+  const uint32_t total = tile_setup<BITS, TeamBlockN<kWideThreads, true>>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     if (threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
@@ -2481,7 +2487,7 @@ __device__ __forceinline__ void adjlist_forward_tile_wide(const DevParams& P, ui
 // forward list built by adjlist_particle on the block's halo, or, in a block
 // beyond the tile capacity, every particle by adj_list_lane.
 template <int BITS>
-__global__ __launch_bounds__(kTileThreads) void k_tile_adjlist_redo(DevParams P, const float4* __restrict__ Q,
+__global__ __launch_bounds__(kTileThreads, 4) void k_tile_adjlist_redo(DevParams P, const float4* __restrict__ Q,
                                                                     const uint32_t* __restrict__ keys,
                                                                     const uint32_t* __restrict__ cs,
                                                                     const uint32_t* __restrict__ ce, NeighbourList F,
@@ -2497,14 +2503,14 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_adjlist_redo(DevParams P,
     __syncthreads();  // the previous block's halo is done with (and the tallies are cleared)
     TileShared<BITS>& sh = lds.sh;
     float4* s_q = lds.q;
-    const uint32_t total = tile_setup<BITS, TeamBlock>(P, redo[1u + i], cs, ce, sh);
+    const uint32_t total = tile_setup<BITS, TeamBlockN<kTileThreads, true>>(P, redo[1u + i], cs, ce, sh);
     if (total > (uint32_t)CAP) {
       const uint32_t m = (sh.g1 - sh.g0) * kAdjLanes;
       for (uint32_t u = threadIdx.x; u < m; u += kTileThreads)
         adj_list_lane(P, Q, keys, cs, ce, L, flag, stats, sh.g0 + u / kAdjLanes, u % kAdjLanes);
       continue;
     }
-    tile_load<BITS, CAP, TeamBlock>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
+    tile_load<BITS, CAP, TeamBlockN<kTileThreads, true>>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
     __syncthreads();
     for (uint32_t g = sh.g0 + threadIdx.x; g < sh.g1; g += kTileThreads) {
       if (F.cnt[g] != kNlInvalid && total <= (uint32_t)TileCap<BITS>::value) continue;  // converted
@@ -2540,7 +2546,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::adjoint;
   constexpr uint32_t kMax = kAdjLanes * kAdjListMax;
-  const uint32_t total = tile_setup<BITS, TeamWide>(P, blk, cs, ce, sh);
+  const uint32_t total = tile_setup<BITS, TeamBlockN<kWideThreads, true>>(P, blk, cs, ce, sh);
   const uint32_t g0 = sh.g0, g1 = sh.g1;
   if (total > (uint32_t)CAP) {
     const uint32_t m = (g1 - g0) * kAdjLanes;
@@ -2548,7 +2554,7 @@ __device__ __forceinline__ void adjlist_tile_wide(const DevParams& P, uint32_t b
       adj_list_lane(P, Q, keys, cs, ce, L, flag, stats, g0 + u / kAdjLanes, u % kAdjLanes);
     return;
   }
-  tile_load<BITS, CAP, TeamWide>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
+  tile_load<BITS, CAP, TeamBlockN<kWideThreads, true>>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
   __syncthreads();
   const uint32_t n = P.n;
   const uint32_t part = threadIdx.x / kTileThreads, pl = threadIdx.x % kTileThreads;
@@ -2690,7 +2696,7 @@ __global__ __launch_bounds__(kWideThreads) void k_tile_adjlist_wide(DevParams P,
 // those one by one; interleaved so that the occupied blocks, which lie in a
 // few Morton ranges, spread over all workgroups.
 template <int BITS>
-__global__ __launch_bounds__(kTileThreads) void k_tile_adjlist(DevParams P, uint32_t nblocks, uint32_t table,
+__global__ __launch_bounds__(kTileThreads, 4) void k_tile_adjlist(DevParams P, uint32_t nblocks, uint32_t table,
                                                                const float4* __restrict__ Q,
                                                                const uint32_t* __restrict__ keys,
                                                                const uint32_t* __restrict__ cs,

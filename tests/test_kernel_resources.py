@@ -60,3 +60,10 @@ def test_capped_grid_passes_keep_four_waves(kernels):
     assert len(vgprs) == 12, sorted(vgprs)
     bad = {k: v for k, v in vgprs.items() if v > 128}
     assert not bad, bad
+
+
+def test_reverse_list_builders_keep_four_waves(kernels):
+    built = _of(kernels, "k_tile_adjlist", "k_tile_adjlist_redo", "k_tile_adjlist_wide")
+    assert len(built) == 3, sorted(built)
+    bad = {k: v for k, v in built.items() if v[0] > 128 or v[1]}
+    assert not bad, bad
