@@ -183,7 +183,7 @@ __device__ __forceinline__ uint32_t tile_setup(const DevParams& P, uint32_t blk,
     if (c < (uint32_t)G::NH) sh.gstart[c] = some ? s0[r] : 0u;
     if (OWN && some) {
       const int hx = (int)c / G::SX, hy = ((int)c / G::SY) % G::HY, hz = (int)c % G::HZ;
-      if (hx >= 1 && hx <= G::EX && hy >= 1 && hy <= G::EY && hz >= 1 && hz <= G::EZ) {
+      if (hx >= 1 && hx <= G::EX && hy >= max(1, y0 + 1) && hy <= min((int)G::EY, y1 - 2) && hz >= 1 && hz <= G::EZ) {
         atomicMin(&sh.g0, s0[r]);
         atomicMax(&sh.g1, e0[r]);
       }
@@ -2300,9 +2300,12 @@ __device__ __forceinline__ void adjlist_tile(const DevParams& P, uint32_t blk, c
 // slots of a list increase, so a walk over the nine columns gives each slot's
 // halo cell; slots at or past the halo size are the forward's padding, and the
 // forward's solid bit becomes kAdjSolid.  A particle without a forward list
-// (over the neighbour cap, more pairs than a forward list holds, or in a block
-// beyond a small tile's capacity) and a block beyond the tile capacity (whose halves'
-// slots are not the block's) are left to k_tile_adjlist_redo: the block is appended to redo (redo[0]: the count).
+// (over the neighbour cap, more pairs than a forward list holds, or in a tile or half
+// beyond its capacity) is left to k_tile_adjlist_redo, and so is a block beyond the
+// builders' capacity: the block is appended to redo (redo[0]: the count).  A block beyond
+// the tile capacity is taken as its two halves, whose cell tables the forward's slots
+// count in (all of it left to the redo pass, the reverse of two substeps of 729K particles
+// at 1.6 times their rest density took 18.8 ms, as halves 14.2).
 //
 // adjlist_forward_tile: a thread per particle, which deals the entries as
 // adjlist_particle does.
@@ -2315,71 +2318,80 @@ __device__ __forceinline__ void adjlist_forward_tile(const DevParams& P, uint32_
                                                      uint32_t* __restrict__ redo, TileShared<BITS>& sh) {
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
-  const uint32_t total = tile_setup<BITS, TeamBlockN<kTileThreads, true>>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
-  if (total > (uint32_t)CAP) {
+  uint32_t total = tile_setup<BITS, TeamBlockN<kTileThreads, true>>(P, blk, cs, ce, sh);
+  if (total > (uint32_t)TileCap<BITS>::adjoint) {
     if (threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
     return;
   }
+  const uint32_t last = total > (uint32_t)CAP ? 2u : 0u;
   int missing = 0;
-  for (uint32_t g = g0 + threadIdx.x; g < g1; g += kTileThreads) {
-    const uint32_t fn = F.cnt[g];
-    if (fn == kNlInvalid) {
-      missing = 1;
-      continue;
+#pragma unroll 1
+  for (uint32_t half = last ? 1u : 0u; half <= last; ++half) {
+    if (half) {
+      __syncthreads();
+      total = tile_setup<BITS, TeamBlockN<kTileThreads, true>>(P, blk, cs, ce, sh, NoLoads(), half);
     }
-    int h;
-    uint32_t slot;
-    tile_locate<BITS>(sh, keys[g], g, h, slot);
-    AdjRows R(L, P.n, g);
-    if (fn > AdjRows::kMax) {
-      R.c = AdjRows::kMax + 1u;  // more candidates than the lanes hold: scan
-    } else {
-      // column `col` (dx = col / 3 - 1, dy = col % 3 - 1): slots [a0, e), z cells from a1, a2
-      int col = 0;
-      uint32_t a1 = 0, a2 = 0, e = 0, b0 = 0, b1 = 0, b2 = 0, oc = 0;
-      const auto column = [&](int c3) __attribute__((always_inline)) {
-        const int hb = h + (c3 / 3 - 1) * G::SX + (c3 % 3 - 1) * G::SY;
-        const uint32_t a0 = sh.lstart[hb - 1];
-        a1 = sh.lstart[hb];
-        a2 = sh.lstart[hb + 1];
-        e = sh.lstart[hb + 2];
-        b0 = sh.gstart[hb - 1] - a0;
-        b1 = sh.gstart[hb] - a1;
-        b2 = sh.gstart[hb + 1] - a2;
-        oc = (uint32_t)((c3 / 3) * 9 + (c3 % 3) * 3);
-      };
-      column(0);
-      // chunk k + 1 is loaded while chunk k is taken apart
-      const uint4* p = F.nl + g;
-      const uint32_t nc = fn / 8u;
-      bool done = nc == 0u;
-      uint4 v = nc ? p[0] : make_uint4(0u, 0u, 0u, 0u);
-      for (uint32_t k = 0; k < nc && !done; ++k) {
-        uint4 nx = v;  // as nl_visit
-        if (k + 1u < nc) nx = p[(size_t)(k + 1u) * F.cap];
-        const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
-        v = nx;
+    const uint32_t g0 = sh.g0, g1 = sh.g1;
+    if (g0 >= g1) continue;  // an empty half
+    for (uint32_t g = g0 + threadIdx.x; g < g1; g += kTileThreads) {
+      const uint32_t fn = F.cnt[g];
+      if (fn == kNlInvalid) {
+        missing = 1;
+        continue;
+      }
+      int h;
+      uint32_t slot;
+      tile_locate<BITS>(sh, keys[g], g, h, slot);
+      AdjRows R(L, P.n, g);
+      if (fn > AdjRows::kMax) {
+        R.c = AdjRows::kMax + 1u;  // more candidates than the lanes hold: scan
+      } else {
+        // column `col` (dx = col / 3 - 1, dy = col % 3 - 1): slots [a0, e), z cells from a1, a2
+        int col = 0;
+        uint32_t a1 = 0, a2 = 0, e = 0, b0 = 0, b1 = 0, b2 = 0, oc = 0;
+        const auto column = [&](int c3) __attribute__((always_inline)) {
+          const int hb = h + (c3 / 3 - 1) * G::SX + (c3 % 3 - 1) * G::SY;
+          const uint32_t a0 = sh.lstart[hb - 1];
+          a1 = sh.lstart[hb];
+          a2 = sh.lstart[hb + 1];
+          e = sh.lstart[hb + 2];
+          b0 = sh.gstart[hb - 1] - a0;
+          b1 = sh.gstart[hb] - a1;
+          b2 = sh.gstart[hb + 1] - a2;
+          oc = (uint32_t)((c3 / 3) * 9 + (c3 % 3) * 3);
+        };
+        column(0);
+        // chunk k + 1 is loaded while chunk k is taken apart
+        const uint4* p = F.nl + g;
+        const uint32_t nc = fn / 8u;
+        bool done = nc == 0u;
+        uint4 v = nc ? p[0] : make_uint4(0u, 0u, 0u, 0u);
+        for (uint32_t k = 0; k < nc && !done; ++k) {
+          uint4 nx = v;  // as nl_visit
+          if (k + 1u < nc) nx = p[(size_t)(k + 1u) * F.cap];
+          const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
+          v = nx;
 #pragma unroll
-        for (uint32_t i = 0; i < 8u; ++i) {
-          const uint32_t raw = (wd[i / 2u] >> (16u * (i & 1u))) & 0xFFFFu;
-          const uint32_t j = raw & (kNlSolid - 1u);
-          if (done || j >= total) {  // the padding, after the last entry
-            done = true;
-            continue;
+          for (uint32_t i = 0; i < 8u; ++i) {
+            const uint32_t raw = (wd[i / 2u] >> (16u * (i & 1u))) & 0xFFFFu;
+            const uint32_t j = raw & (kNlSolid - 1u);
+            if (done || j >= total) {  // the padding, after the last entry
+              done = true;
+              continue;
+            }
+            while (j >= e && col < 8) column(++col);
+            const uint32_t z = j < a1 ? 0u : (j < a2 ? 1u : 2u);
+            const uint32_t base = z == 0u ? b0 : (z == 1u ? b1 : b2);
+            R.push((base + j) | ((oc + z) << 27) | ((raw & kNlSolid) ? kAdjSolid : 0u));
           }
-          while (j >= e && col < 8) column(++col);
-          const uint32_t z = j < a1 ? 0u : (j < a2 ? 1u : 2u);
-          const uint32_t base = z == 0u ? b0 : (z == 1u ? b1 : b2);
-          R.push((base + j) | ((oc + z) << 27) | ((raw & kNlSolid) ? kAdjSolid : 0u));
         }
       }
+      R.finish(L, g);
+      if (tile_count<BITS>(sh, h) >= P.cap) flag[0] = 1u;
+      wave_tally(tally + 0, R.c <= AdjRows::kMax);
+      wave_tally(tally + 1, R.c > AdjRows::kMax);
+      wave_tally(tally + 2, true);
     }
-    R.finish(L, g);
-    if (tile_count<BITS>(sh, h) >= P.cap) flag[0] = 1u;
-    wave_tally(tally + 0, R.c <= AdjRows::kMax);
-    wave_tally(tally + 1, R.c > AdjRows::kMax);
-    wave_tally(tally + 2, true);
   }
   if (__syncthreads_or(missing) && threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
 }
@@ -2401,84 +2413,92 @@ __device__ __forceinline__ void adjlist_forward_tile_wide(const DevParams& P, ui
   using G = TileGeom<BITS>;
   constexpr int CAP = TileCap<BITS>::value;
   static_assert(kNlRecordChunks == kAdjLanes && kAdjListMax == kAdjLanes, "a forward chunk is a row of the lanes");
-  const uint32_t total = tile_setup<BITS, TeamBlockN<kWideThreads, true>>(P, blk, cs, ce, sh);
-  const uint32_t g0 = sh.g0, g1 = sh.g1;
-  if (total > (uint32_t)CAP) {
+  uint32_t total = tile_setup<BITS, TeamBlockN<kWideThreads, true>>(P, blk, cs, ce, sh);
+  if (total > (uint32_t)TileCap<BITS>::adjoint) {
     if (threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
     return;
   }
-  const uint32_t n = P.n;
+  const uint32_t n = P.n, last = total > (uint32_t)CAP ? 2u : 0u;
   int missing = 0;
-  for (uint32_t u = threadIdx.x; u < (g1 - g0) * kAdjLanes; u += kWideThreads) {
-    const uint32_t g = g0 + u / kAdjLanes, k = u % kAdjLanes;
-    const uint32_t fn = F.cnt[g];
-    if (fn == kNlInvalid) {
-      missing = 1;
-      continue;
+#pragma unroll 1
+  for (uint32_t half = last ? 1u : 0u; half <= last; ++half) {
+    if (half) {
+      __syncthreads();
+      total = tile_setup<BITS, TeamBlockN<kWideThreads, true>>(P, blk, cs, ce, sh, NoLoads(), half);
     }
-    const uint32_t nc = fn / 8u;
-    // the thread that writes the counts: the last chunk's, or chunk 0's without a row
-    const bool counter = fn > AdjRows::kMax || nc == 0u ? k == 0u : k + 1u == nc;
-    uint32_t c = 0;
-    int h = 0;
-    if (fn <= AdjRows::kMax && k < nc) {
-      uint32_t slot;
-      tile_locate<BITS>(sh, keys[g], g, h, slot);
-      const uint4 v = F.nl[(size_t)k * F.cap + g];
-      const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
-      int col = -1;
-      uint32_t a1 = 0, a2 = 0, e = 0, b0 = 0, b1 = 0, b2 = 0, oc = 0;
-      const auto column = [&](int c3) __attribute__((always_inline)) {
-        const int hb = h + (c3 / 3 - 1) * G::SX + (c3 % 3 - 1) * G::SY;
-        const uint32_t a0 = sh.lstart[hb - 1];
-        a1 = sh.lstart[hb];
-        a2 = sh.lstart[hb + 1];
-        e = sh.lstart[hb + 2];
-        b0 = sh.gstart[hb - 1] - a0;
-        b1 = sh.gstart[hb] - a1;
-        b2 = sh.gstart[hb + 1] - a2;
-        oc = (uint32_t)((c3 / 3) * 9 + (c3 % 3) * 3);
-      };
-      column(++col);
-      uint32_t w[kAdjLanes];
-#pragma unroll
-      for (uint32_t i = 0; i < kAdjLanes; ++i) {
-        const uint32_t raw = (wd[i / 2u] >> (16u * (i & 1u))) & 0xFFFFu;
-        const uint32_t j = raw & (kNlSolid - 1u);
-        w[i] = 0u;
-        if (j >= total) continue;  // the padding, after the last entry
-        ++c;
-        while (j >= e && col < 8) column(++col);
-        const uint32_t z = j < a1 ? 0u : (j < a2 ? 1u : 2u);
-        const uint32_t base = z == 0u ? b0 : (z == 1u ? b1 : b2);
-        w[i] = (base + j) | ((oc + z) << 27) | ((raw & kNlSolid) ? kAdjSolid : 0u);
+    const uint32_t g0 = sh.g0, g1 = sh.g1;
+    if (g0 >= g1) continue;  // an empty half
+    for (uint32_t u = threadIdx.x; u < (g1 - g0) * kAdjLanes; u += kWideThreads) {
+      const uint32_t g = g0 + u / kAdjLanes, k = u % kAdjLanes;
+      const uint32_t fn = F.cnt[g];
+      if (fn == kNlInvalid) {
+        missing = 1;
+        continue;
       }
-      uint4* dst = reinterpret_cast<uint4*>(L.e + ((size_t)k * n + g) * kAdjLanes);
-      dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
-      dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
-    }
-    if (counter) {
-      if (fn > AdjRows::kMax) {
-        c = AdjRows::kMax + 1u;  // more candidates than the lanes hold: scan
-      } else if (nc) {
-        c += 8u * (nc - 1u);
-      }
-      uint32_t cl[kAdjLanes];
-#pragma unroll
-      for (uint32_t lane = 0; lane < kAdjLanes; ++lane)
-        cl[lane] = c > AdjRows::kMax ? kAdjScan : (c + kAdjLanes - 1u - lane) / kAdjLanes;
-      uint4* cdst = reinterpret_cast<uint4*>(L.cnt + (size_t)g * kAdjLanes);
-      cdst[0] = make_uint4(cl[0], cl[1], cl[2], cl[3]);
-      cdst[1] = make_uint4(cl[4], cl[5], cl[6], cl[7]);
-      if (fn > AdjRows::kMax || nc == 0u) {
+      const uint32_t nc = fn / 8u;
+      // the thread that writes the counts: the last chunk's, or chunk 0's without a row
+      const bool counter = fn > AdjRows::kMax || nc == 0u ? k == 0u : k + 1u == nc;
+      uint32_t c = 0;
+      int h = 0;
+      if (fn <= AdjRows::kMax && k < nc) {
         uint32_t slot;
         tile_locate<BITS>(sh, keys[g], g, h, slot);
+        const uint4 v = F.nl[(size_t)k * F.cap + g];
+        const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
+        int col = -1;
+        uint32_t a1 = 0, a2 = 0, e = 0, b0 = 0, b1 = 0, b2 = 0, oc = 0;
+        const auto column = [&](int c3) __attribute__((always_inline)) {
+          const int hb = h + (c3 / 3 - 1) * G::SX + (c3 % 3 - 1) * G::SY;
+          const uint32_t a0 = sh.lstart[hb - 1];
+          a1 = sh.lstart[hb];
+          a2 = sh.lstart[hb + 1];
+          e = sh.lstart[hb + 2];
+          b0 = sh.gstart[hb - 1] - a0;
+          b1 = sh.gstart[hb] - a1;
+          b2 = sh.gstart[hb + 1] - a2;
+          oc = (uint32_t)((c3 / 3) * 9 + (c3 % 3) * 3);
+        };
+        column(++col);
+        uint32_t w[kAdjLanes];
+#pragma unroll
+        for (uint32_t i = 0; i < kAdjLanes; ++i) {
+          const uint32_t raw = (wd[i / 2u] >> (16u * (i & 1u))) & 0xFFFFu;
+          const uint32_t j = raw & (kNlSolid - 1u);
+          w[i] = 0u;
+          if (j >= total) continue;  // the padding, after the last entry
+          ++c;
+          while (j >= e && col < 8) column(++col);
+          const uint32_t z = j < a1 ? 0u : (j < a2 ? 1u : 2u);
+          const uint32_t base = z == 0u ? b0 : (z == 1u ? b1 : b2);
+          w[i] = (base + j) | ((oc + z) << 27) | ((raw & kNlSolid) ? kAdjSolid : 0u);
+        }
+        uint4* dst = reinterpret_cast<uint4*>(L.e + ((size_t)k * n + g) * kAdjLanes);
+        dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
       }
-      if (tile_count<BITS>(sh, h) >= P.cap) flag[0] = 1u;
+      if (counter) {
+        if (fn > AdjRows::kMax) {
+          c = AdjRows::kMax + 1u;  // more candidates than the lanes hold: scan
+        } else if (nc) {
+          c += 8u * (nc - 1u);
+        }
+        uint32_t cl[kAdjLanes];
+#pragma unroll
+        for (uint32_t lane = 0; lane < kAdjLanes; ++lane)
+          cl[lane] = c > AdjRows::kMax ? kAdjScan : (c + kAdjLanes - 1u - lane) / kAdjLanes;
+        uint4* cdst = reinterpret_cast<uint4*>(L.cnt + (size_t)g * kAdjLanes);
+        cdst[0] = make_uint4(cl[0], cl[1], cl[2], cl[3]);
+        cdst[1] = make_uint4(cl[4], cl[5], cl[6], cl[7]);
+        if (fn > AdjRows::kMax || nc == 0u) {
+          uint32_t slot;
+          tile_locate<BITS>(sh, keys[g], g, h, slot);
+        }
+        if (tile_count<BITS>(sh, h) >= P.cap) flag[0] = 1u;
+      }
+      wave_tally(tally + 0, counter && c <= AdjRows::kMax);
+      wave_tally(tally + 1, counter && c > AdjRows::kMax);
+      wave_tally(tally + 2, counter);
     }
-    wave_tally(tally + 0, counter && c <= AdjRows::kMax);
-    wave_tally(tally + 1, counter && c > AdjRows::kMax);
-    wave_tally(tally + 2, counter);
   }
   if (__syncthreads_or(missing) && threadIdx.x == 0) redo[1u + atomicAdd(redo, 1u)] = blk;
 }
@@ -2513,7 +2533,7 @@ __global__ __launch_bounds__(kTileThreads, 4) void k_tile_adjlist_redo(DevParams
     tile_load<BITS, CAP, TeamBlockN<kTileThreads, true>>(P, sh, total, Q, s_q, nullptr, 0u, adj_solid_payload(P));
     __syncthreads();
     for (uint32_t g = sh.g0 + threadIdx.x; g < sh.g1; g += kTileThreads) {
-      if (F.cnt[g] != kNlInvalid && total <= (uint32_t)TileCap<BITS>::value) continue;  // converted
+      if (F.cnt[g] != kNlInvalid) continue;  // converted
       int h;
       uint32_t slot;
       tile_locate<BITS>(sh, keys[g], g, h, slot);
