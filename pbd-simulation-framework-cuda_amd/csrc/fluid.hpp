@@ -138,8 +138,7 @@ class Fluid : public Cuda_Computable {
   uint32_t small_max_ = kTileSmall;       // blocks of at most this many particles take one wave
   bool small_auto_ = true;                 // until a launch shape is set: default_small_max(n_)
   uint32_t small_max() const { return small_auto_ ? default_small_max(n_) : small_max_; }
-  // the largest small tile the compaction makes
-  uint32_t small_tiles() const { return small_auto_ && default_small_max(n_) ? kTileSmall : small_max(); }
+  uint32_t small_tiles() const { return small_tile_limit(small_max()); }  // as the compaction makes them
   uint32_t stride_grid_ = kTileGridStride;  // workgroups of the capped tile grid
   uint32_t skin_pct_ = kListSkinPct;       // tile-list skin, percent of the list radius
   uint32_t* host_err_ = nullptr;           // the sort's error flag (pinned), unless the context lies in a region

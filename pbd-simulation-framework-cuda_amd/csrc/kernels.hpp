@@ -85,11 +85,13 @@ inline uint32_t split_bound(uint32_t ntiles, uint32_t n) { return n / 169u + 1u 
 inline uint32_t default_small_max(uint32_t n) {
   return n <= (1u << 16) ? 0u : n < (1u << 21) ? 32u : kTileSmall;
 }
-// Until a launch shape is set, blocks between that threshold (if it is not 0) and
-// kTileSmall are small as well where their halo fits a small tile: a workgroup of its own
-// leaves three of its waves idle.  us a step with small tiles up to 32 / 48 / 64: 211K
-// splash 588 / 573 / 521, 1M splash 1669 / 1544 / 1438, 64 scenes of 2K to 32K 7960 / 7530
-// / 7355, 1M column 1060 / 1065 / 1064; a 32K frame 223 without, 238 with them.
+// The largest block that is small under a threshold: from 32 on, blocks of up to kTileSmall
+// are, where their halo fits a small tile: a workgroup of its own leaves three of its waves
+// idle.  us a step with small tiles up to 32 / 48 / 64: 211K splash 588 / 573 / 521, 1M
+// splash 1669 / 1544 / 1438, 64 scenes of 2K to 32K 7960 / 7530 / 7355, 1M column 1060 /
+// 1065 / 1064; a 32K frame 223 without, 238 with them.  A rule of the threshold alone, so
+// that a shape read and set again launches the same step.
+inline uint32_t small_tile_limit(uint32_t small_max) { return small_max < 32u ? small_max : kTileSmall; }
 constexpr uint32_t kNlChunks = 12;            // neighbour-list chunks of 8 slots: lists of up to 96 pairs
 constexpr uint32_t kTileCompactChunk = 4096;  // flags per block of the compaction
 #ifndef PBD_TILE_CHUNK

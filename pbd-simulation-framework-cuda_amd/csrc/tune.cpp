@@ -229,11 +229,9 @@ int Fluid::autotune(uint32_t trial_steps, LaunchShape* chosen, double* ms_chosen
     // not 0 (small tiles off): they pay once the flow has spread into sparse
     // blocks, which trial steps from an earlier state may not see (off was 3 %
     // faster over steps 21-28 of the 1M dam break and 14 % slower over 21-220)
-    for (uint32_t v : {32u, 64u}) {
-      LaunchShape s = best;
-      s.small_max = v;
-      if (v != best.small_max) trial(s);
-    }
+    LaunchShape s = best;
+    s.small_max = kTileSmall;
+    if (small_tile_limit(best.small_max) != kTileSmall) trial(s);
   }
   for (uint32_t v : {128u, 256u, 512u}) {
     LaunchShape s = best;
