@@ -462,12 +462,8 @@ int Fluid::enqueue_substep() {
   bool tstride = false;
   if (tiles) {
     ntiles = ((B_.table_size - 1u) >> bits) + 1u;
-    // work items (large tiles + small tiles / 4) <= occupied blocks <= min(ntiles, n);
-    // a multiple of XCDs x tile chunk, so that tile_rank0 maps the grid onto [0, tgrid)
-    tgrid = (std::min(ntiles, P.n) + split_bound(ntiles, P.n) + kTileGridMultiple - 1u) / kTileGridMultiple *
-            kTileGridMultiple;
-    tstride = tgrid > kTileGridDirect;
-    if (tstride) tgrid = stride_grid_;
+    tstride = capped_grid(ntiles, P.n);
+    tgrid = tstride ? stride_grid_ : direct_grid(ntiles, P.n);
     // phases on tiles: 2^5-cell blocks with the direct grid only
     if (P.phased && (bits != 5 || tstride)) tiles = false;
   }

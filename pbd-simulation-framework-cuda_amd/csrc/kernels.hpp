@@ -114,6 +114,20 @@ constexpr uint32_t kListSkinPct = 10;
 constexpr uint32_t kListSkinPctMax = 50;
 constexpr uint32_t kCarryPasses = 8;  // solver iterations up to which lists are carried
 static_assert(kTileGridStride % kTileGridMultiple == 0 && kTileGridDirect % kTileGridMultiple == 0, "tile grids");
+// Work items (large tiles + small tiles / 4) <= occupied blocks <= min(ntiles, n), and the
+// second halves of split blocks.  Whether a step takes the capped grid is decided by the
+// blocks alone: phased scenes have no capped form, and the halves of those just below the
+// line lie past it.  A direct grid is a multiple of XCDs x tile chunk, so that tile_rank0
+// maps it onto [0, grid).
+inline uint32_t tile_grid_round(uint32_t items) {
+  return (items + kTileGridMultiple - 1u) / kTileGridMultiple * kTileGridMultiple;
+}
+inline bool capped_grid(uint32_t ntiles, uint32_t n) {
+  return tile_grid_round(ntiles < n ? ntiles : n) > kTileGridDirect;
+}
+inline uint32_t direct_grid(uint32_t ntiles, uint32_t n) {
+  return tile_grid_round((ntiles < n ? ntiles : n) + split_bound(ntiles, n));
+}
 // Splits the occupied blocks (start[b] != 0) into large[] and small[] by their
 // particle count end[b] - (start[b] - 1) (small: at most small_max <= kTileSmall),
 // both ascending; count[0..1] = their lengths.  bcount holds

@@ -185,8 +185,7 @@ int Fluid::autotune(uint32_t trial_steps, LaunchShape* chosen, double* ms_chosen
   const bool tiles = params_.tile_bits != 0 && params_.kernel_variant == PBD_KERNEL_TEXTBOOK &&
                      params_.kernel_width_neighbours == 1 && params_.active_find_contacts;
   const uint32_t ntiles = ((B_.table_size - 1u) >> 5) + 1u;
-  const bool stride = tiles && ((std::min(ntiles, n_) + kTileGridMultiple - 1u) / kTileGridMultiple *
-                                    kTileGridMultiple > kTileGridDirect);
+  const bool stride = tiles && capped_grid(ntiles, n_);
   LaunchShape best = start;
   double best_ms = 0.0, first_ms = 0.0;
   int rc = time_shape(best, trial_steps, &best_ms);

@@ -26,6 +26,8 @@ int main(int, char** v) {
     s.skin_pct = 5;
     rc |= f.set_launch_shape(s);
     std::printf("%d %u %u %u %u %u\n", rc, reported, f.launch_shape().small_max, before, same, f.small_tiles());
+  } else {  // grid: blocks, particles
+    std::printf("%d %u\n", capped_grid(arg(v, 2), arg(v, 3)) ? 1 : 0, direct_grid(arg(v, 2), arg(v, 3)));
   }
   return 0;
 }
@@ -54,3 +56,17 @@ def test_a_shape_read_and_set_again_launches_the_same_step(ask, n, small, tiles)
     rc, reported, after, default, same, skin = ask("shape", n)
     assert rc == 0 and reported == small and after == small
     assert default == tiles and same == tiles and skin == tiles
+
+
+# around 2^20 items, where a step leaves the direct grid (and a phased one its tiles), by
+# blocks and by particles; few blocks; one
+@pytest.mark.parametrize("blocks,n,capped", [(1 << 22, 1 << 20, 0), (1 << 22, (1 << 20) + 1, 1), (1 << 20, 1 << 24, 0),
+                                             ((1 << 20) + 1, 1 << 24, 1), (1 << 22, 1042411, 0), (1 << 22, 1047000, 0),
+                                             (40960, 1 << 20, 0), (1, 5000, 0), (16, 1, 0)])
+def test_split_blocks_do_not_decide_the_grid(ask, blocks, n, capped):
+    is_capped, grid = ask("grid", blocks, n)
+    assert is_capped == capped
+    # every block, and as many halves more as there can be: a halo of more than 1352
+    # particles, each particle in at most 8 halos
+    items = min(blocks, n) + min(blocks, n // 169)
+    assert grid >= items and grid % 32 == 0 and grid < items + 64
