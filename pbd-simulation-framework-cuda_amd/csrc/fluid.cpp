@@ -90,8 +90,8 @@ int Fluid::alloc_table() {
   const uint32_t tt = region_ ? region_table_ : ts;
   const uint32_t nt = ((tt - 1u) >> 5) + 1u;
   if (take(&B_.cstart, tt) || take(&B_.cend, tt) || take(&tile_flag_, nt) || take(&tile_end_, nt) ||
-      take(&tile_bcount_, (nt + kTileCompactChunk - 1u) / kTileCompactChunk) || take(&B_.BUILT, nt) ||
-      take(&B_.MODE, nt))
+      take(&tile_bcount_, (nt + kTileCompactChunk - 1u) / kTileCompactChunk) || take(&B_.BUILT, 2 * (size_t)nt) ||
+      take(&B_.MODE, 2 * (size_t)nt))
     return fail(PBD_ERR_NOMEM, "cell table allocation failed");
   // no tile carries its lists before its halo has been seen to stay within the skin
   // (a region is zeroed whole by init_in_place)

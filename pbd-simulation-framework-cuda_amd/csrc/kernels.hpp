@@ -46,15 +46,16 @@ struct StepBuffers {
   // Tile lists carried from pass to pass: DISP[(p - 1) nl_cap + i] bounds the
   // displacement of particle i over the substep's first p delta-p passes (the
   // sum of the lengths of its moves; p = 1 .. kCarryPasses, and 0 for p = 0),
-  // BUILT[b] is the number of delta-p passes before tile b last built its lists
-  // (kNoCarry: the tile rebuilds them every pass this substep), MODE[b] whether
+  // BUILT[2 b] is the number of delta-p passes before tile b last built its lists
+  // (kNoCarry: the tile rebuilds them every pass this substep), MODE[2 b] whether
   // tile b carries its lists in the next substep (its halo stayed within the
-  // skin in the last one).
+  // skin in the last one).  Of a block of two items, 2 b is the first's place and
+  // 2 b + 1 the second's.
   float* DISP;
-  uint32_t* BUILT;
-  uint32_t* MODE;
+  uint16_t* BUILT;
+  uint16_t* MODE;
 };
-constexpr uint32_t kNoCarry = 0xFFFFFFFFu;
+constexpr uint32_t kNoCarry = 0xFFFFu;
 
 // Occupied Morton blocks of the current step in Morton order (the reorder
 // kernel marks them, launch_tile_compact lists them).  Blocks of at most

@@ -93,6 +93,8 @@ __device__ __forceinline__ uint32_t tile_begin(uint32_t start) { return (start &
 // block are consecutive key ranges), and its own particles.
 struct TileOwn {
   uint32_t blk, half, g0, g1;
+  // its place in StepBuffers::BUILT and MODE
+  __device__ __forceinline__ uint32_t carried() const { return 2u * blk + (half == 2u ? 1u : 0u); }
 };
 template <int BITS>
 __device__ __forceinline__ TileOwn tile_own(const DevParams& P, const TileList& T, uint32_t item,
@@ -740,8 +742,8 @@ __device__ __forceinline__ void tile_load(const DevParams& P, TileShared<BITS>& 
 // delta-p pass `pass` (1-based); disp null: no carry.
 struct Carry {
   float* disp;
-  uint32_t* built;
-  uint32_t* mode;
+  uint16_t* built;
+  uint16_t* mode;
   uint32_t stride;
   uint32_t pass;
   __device__ __forceinline__ float* bounds(uint32_t p) const {
@@ -967,7 +969,7 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileLi
   }
   // the first pass: whether the tile carries its lists this substep; a later
   // one: the delta-p passes before the tile's lists were built (kNoCarry: none)
-  const uint32_t m = C.disp && !own.half ? (FIRST ? (C.mode[blk] ? 0u : kNoCarry) : C.built[blk]) : kNoCarry;
+  const uint32_t m = C.disp ? (FIRST ? (C.mode[own.carried()] ? 0u : kNoCarry) : C.built[own.carried()]) : kNoCarry;
   const bool carry = !FIRST && m != kNoCarry;
   const float r2 = m != kNoCarry ? P.tile_r2 : P.list_r2;
   // .w: 1 for a solid particle (PH), else 0
@@ -977,8 +979,8 @@ __device__ __forceinline__ TileRest lambda_tile(const DevParams& P, const TileLi
   Team::sync();
   const bool keep = carry && tile_keeps_lists<BITS>(P, sh);
   if (tid == 0 && C.disp) {
-    if (FIRST && !own.half) C.built[blk] = m;  // 0: built now, with the skin
-    else if (carry && !keep) C.built[blk] = C.pass;  // rebuilt now
+    if (FIRST) C.built[own.carried()] = (uint16_t)m;  // 0: built now, with the skin
+    else if (carry && !keep) C.built[own.carried()] = (uint16_t)C.pass;  // rebuilt now
     if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                          (unsigned long long)(g1 - g0));
   }
@@ -1242,7 +1244,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
   }
   // global index of each slot: velocities are gathered from L2
   // .w: 1 for a solid particle (PH), else 0
-  const uint32_t m = C.disp && !own.half ? C.built[blk] : kNoCarry;
+  const uint32_t m = C.disp ? C.built[own.carried()] : kNoCarry;
   const bool carry = m != kNoCarry;
   tile_load<BITS, CAP, Team>(P, sh, total, Q, s_q, s_gi, g0,
                              [&](uint32_t gi) { return PH && P.phs[gi] ? 1.0f : 0.0f; },
@@ -1251,7 +1253,7 @@ __device__ __forceinline__ TileRest omega_tile(const DevParams& P, const TileLis
   const bool calm = C.disp && tile_keeps_lists<BITS>(P, sh);
   const bool keep = carry && calm;
   if (tid == 0 && C.disp) {
-    C.mode[blk] = calm && !own.half ? 1u : 0u;  // halves do not carry: both write 0
+    C.mode[own.carried()] = calm ? 1u : 0u;
     if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                          (unsigned long long)(g1 - g0));
   }
@@ -1633,7 +1635,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
     if (tid == 0) atomicAdd(&L.stats[PBD_COUNTER_UNLISTED_BLOCK], (unsigned long long)(g1 - g0));
   } else {
     // as lambda_tile
-    const uint32_t m = C.disp && !own.half ? (FIRST ? (C.mode[blk] ? 0u : kNoCarry) : C.built[blk]) : kNoCarry;
+    const uint32_t m = C.disp ? (FIRST ? (C.mode[own.carried()] ? 0u : kNoCarry) : C.built[own.carried()]) : kNoCarry;
     const bool carry = !FIRST && m != kNoCarry;
     const float r2 = m != kNoCarry ? P.tile_r2 : P.list_r2;
     tile_load<5, CAP, TeamWide>(P, sh, total, Q, lds.q, nullptr, 0u, [](uint32_t) { return 0.0f; },
@@ -1641,8 +1643,8 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_lambda(DevParams P, TileL
     __syncthreads();
     const bool keep = carry && tile_keeps_lists<5>(P, sh);
     if (tid == 0 && C.disp) {
-      if (FIRST && !own.half) C.built[blk] = m;
-      else if (carry && !keep) C.built[blk] = C.pass;
+      if (FIRST) C.built[own.carried()] = (uint16_t)m;
+      else if (carry && !keep) C.built[own.carried()] = (uint16_t)C.pass;
       if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                            (unsigned long long)(g1 - g0));
     }
@@ -1758,7 +1760,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
   } else {
     // as omega_tile; .w: the slot's global index (velocities are gathered from L2), of the
     // sentinel the block's first particle (its pair terms are zero)
-    const uint32_t m = C.disp && !own.half ? C.built[blk] : kNoCarry;
+    const uint32_t m = C.disp ? C.built[own.carried()] : kNoCarry;
     const bool carry = m != kNoCarry;
     tile_load<5, CAP, TeamWide>(P, sh, total, Q, lds.q, nullptr, 0u,
                                 [](uint32_t gi) { return __uint_as_float(gi); }, C.disp ? C.bounds(C.pass) : nullptr,
@@ -1767,7 +1769,7 @@ __global__ __launch_bounds__(kWideThreads) void k_wide_omega(DevParams P, TileLi
     const bool calm = C.disp && tile_keeps_lists<5>(P, sh);
     const bool keep = carry && calm;
     if (tid == 0 && C.disp) {
-      C.mode[blk] = calm && !own.half ? 1u : 0u;  // halves do not carry: both write 0
+      C.mode[own.carried()] = calm ? 1u : 0u;
       if (carry) atomicAdd(&L.stats[keep ? PBD_COUNTER_LIST_CARRIES : PBD_COUNTER_LIST_RESCANS],
                            (unsigned long long)(g1 - g0));
     }
