@@ -74,8 +74,8 @@ constexpr uint32_t kTileSmall = 64;           // particles of a small tile (one 
 constexpr uint32_t kTileSmallSure = 8;        // up to here small whatever its halo holds
 constexpr uint32_t kTileCrowded = 1u << 31;   // a block that is large for its halo
 constexpr uint32_t kTileSplit = 1u << 30;     // a block that is two items for its halo
-// Blocks that are two items: a halo of more than 1352 particles; a particle is in at most 8 (1352 / 8 = 169).
-inline uint32_t split_bound(uint32_t ntiles, uint32_t n) { return n / 169u + 1u < ntiles ? n / 169u + 1u : ntiles; }
+// Blocks that are two items: a halo of more than 1528 particles; a particle is in at most 8 (1528 / 8 = 191).
+inline uint32_t split_bound(uint32_t ntiles, uint32_t n) { return n / 191u + 1u < ntiles ? n / 191u + 1u : ntiles; }
 // The small-tile threshold a context starts with, by particle count.  Measured
 // over 100 frames of the dam break (ms per substep at 0 / 32 / 64): up to 2^16
 // particles the occupied blocks are too few to fill the chip, and packing four

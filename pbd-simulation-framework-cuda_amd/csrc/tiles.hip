@@ -368,15 +368,20 @@ __device__ __forceinline__ int tile_pick(const TileList& T, const TileItems& it,
 // so that a slot names the same particle in both.
 template <int BITS>
 struct TileCap;
-// The capacity decides how many workgroups a CU holds: with 1352 slots (and small tiles'
-// 272) a lambda pass has 23 KB and 7 of them, as many as its 67 VGPRs allow, at 1920 slots
-// 5.  us a step at 1920 / 1352 slots: 1M column 1060 / 964, 1M splash 1438 / 1285, 16M
-// column 14700 / 13650, 64 uneven scenes 7360 / 7110.  A block with more in its halo (1152
-// at rest density) is two items, its halves, which hold as crowded cells as 1920 slots did
-// for the whole (a half's halo is 96 cells of the 144).
+// The capacity decides how many workgroups a CU holds: with 1528 slots (and small tiles'
+// 272) a lambda pass has 26 KB and 6 of them, as many as its 73 to 79 VGPRs allow, an omega
+// pass (a slot's global index beside it) 32 KB and 5, at 1920 slots 5 and 4.  us a step at
+// 1920 / 1352 slots, when it was lowered: 1M column 1060 / 964, 1M splash 1438 / 1285, 16M
+// column 14700 / 13650, 64 uneven scenes 7360 / 7110; at 1352 / 1528 / 1560: 1M column 912 /
+// 912 / 927, 1M splash 1177 / 1190 / 1225, 16M column 12395 / 12392 / 12650, 64 uneven
+// scenes 6930 / 7030 / 7110.  A block with more in its halo (1152 at rest density) is two
+// items, its halves.  1528 slots hold a half (96 cells of the 144) of nearly every halo of up
+// to 1920 within the neighbour cap; with 1352, layers of 9, 20, 20 and 9 a cell went particle
+// by particle from global memory (401K of them 2830 us a step, as halves in the LDS 2193, as
+// whole blocks of 1920 slots 2331).
 template <>
 struct TileCap<5> {
-  static constexpr int value = 1352;  // 2x4x4 blocks: 144 halo cells, ~1150 particles at rest density
+  static constexpr int value = 1528;  // 2x4x4 blocks: 144 halo cells, ~1150 particles at rest density
   static constexpr int small = 272;   // a small tile's halo (one wave, a quarter of the LDS)
   static constexpr int adjoint = 1920;  // of the reverse passes' list builders
 };
@@ -626,7 +631,7 @@ union TileLds {
   TileRegion<BITS, TileCap<BITS>::small, GI> small[kTileThreads / 64u];
 };
 constexpr uint32_t kLdsBytes = 160u * 1024u;  // of a CU
-static_assert(5 * sizeof(TileLds<5, false>) <= kLdsBytes && 4 * sizeof(TileLds<5, true>) <= kLdsBytes,
+static_assert(6 * sizeof(TileLds<5, false>) <= kLdsBytes && 5 * sizeof(TileLds<5, true>) <= kLdsBytes,
               "workgroups per CU of the 2^5-cell passes");
 static_assert(3 * sizeof(TileLds<6, false>) <= kLdsBytes && 2 * sizeof(TileLds<6, true>) <= kLdsBytes,
               "workgroups per CU of the 2^6-cell passes");

@@ -1,4 +1,4 @@
-"""Lists carried from substep to substep where blocks are two items (halos of more than 1352
+"""Lists carried from substep to substep where blocks are two items (halos of more than 1528
 particles): the halves of calm blocks keep theirs, and a block that becomes one item or two
 between substeps, or holds more than the halves do, steps as with lists rebuilt in every
 pass, bit for bit, in every output."""
@@ -33,9 +33,9 @@ def _same(a, b):
             assert np.array_equal(u[k], w[k]), (s, k)
 
 
-# blocks past a tile's capacity (halos of 1440 to 1700) everywhere but at the walls
+# blocks past a tile's capacity (halos of 1700 to 1800) everywhere but at the walls
 @pytest.mark.parametrize("small", [0, 64])
-@pytest.mark.parametrize("counts", [(10, 10, 11), (9, 12, 13)])
+@pytest.mark.parametrize("counts", [(12, 12, 13), (11, 12, 13)])
 def test_gpu_split_blocks_carry_their_lists(F, small, counts):
     p, x, v = _scene(F, (8, 12, 12), counts, 0.98)
     p.active_apply_delta_positions = 0  # calm: nothing moves but by its velocity
@@ -51,14 +51,14 @@ def test_gpu_split_blocks_carry_their_lists(F, small, counts):
     assert c["list_carries"] + c["unlisted_cap"] >= 0.99 * 12 * len(x)
 
 
-# halos around 1352 and particles that change cells: blocks become one item and two from
+# halos around 1528 and particles that change cells: blocks become one item and two from
 # substep to substep; with moves past the skin in every pass (the corrections of particles
 # at random places, nothing carries) and, the corrections not applied, without
 @pytest.mark.parametrize("small", [0, 64])
 @pytest.mark.parametrize("speed", [0.05, 0.6])
 @pytest.mark.parametrize("applied", [1, 0])
 def test_gpu_blocks_split_and_join_between_substeps(F, small, speed, applied):
-    p, x, v = _scene(F, (8, 12, 12), (9, 9, 10), 0.98, seed=17)
+    p, x, v = _scene(F, (8, 12, 12), (10, 11, 11), 0.98, seed=17)
     rng = np.random.default_rng(5)
     v[:, :3] = rng.normal(0.0, speed, (len(x), 3))
     p.active_apply_delta_positions = applied

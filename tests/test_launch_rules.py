@@ -66,7 +66,7 @@ def test_a_shape_read_and_set_again_launches_the_same_step(ask, n, small, tiles)
 def test_split_blocks_do_not_decide_the_grid(ask, blocks, n, capped):
     is_capped, grid = ask("grid", blocks, n)
     assert is_capped == capped
-    # every block, and as many halves more as there can be: a halo of more than 1352
+    # every block, and as many halves more as there can be: a halo of more than 1528
     # particles, each particle in at most 8 halos
-    items = min(blocks, n) + min(blocks, n // 169)
+    items = min(blocks, n) + min(blocks, n // 191)
     assert grid >= items and grid % 32 == 0 and grid < items + 64
