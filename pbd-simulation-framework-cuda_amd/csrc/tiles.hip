@@ -415,7 +415,7 @@ __device__ __forceinline__ uint32_t tile_class(uint32_t b, uint32_t nflags, cons
 // lane's cells in flight at once.
 constexpr uint32_t kHaloLanes = 16;
 // Flags of a wave.  Where the blocks fill few waves, four blocks a wave are one chain of two
-// loads (6 to 9 us up to 1M particles in a box that they fill); with more flags the chain
+// loads (7 us at 32K particles, 17 at 1M); with more flags the chain
 // repeats, but the waves that only sweep empty blocks, of a box far larger than its fluid,
 // are fewer.  us a step at 4 / 16 / 64 flags: 2K 167 / 173 / 173, 211K splash (45K flags) 472
 // / 485 / 509, 1M column (41K) 949 / 951 / 988, 16M column (0.3M) 13557 / 13370 / 13368, 1.2M
@@ -1498,7 +1498,8 @@ struct WideLds {
   float4 q[TileCap<5>::value + kScanUnroll];
   uint16_t list[kWideParticles][kNlMax];  // 16-byte chunks, as the global lists'
 };
-static_assert(2 * sizeof(WideLds) <= kLdsBytes, "two workgroups per CU");
+// (the registers, 93 to 99, admit one workgroup of 16 waves a CU)
+static_assert(2 * sizeof(WideLds) <= kLdsBytes, "LDS of two workgroups");
 static_assert(sizeof(TileShared<5>) % 16 == 0 || alignof(WideLds) >= 16, "alignment of the halo");
 
 // The value that lane p of the quad holds.
