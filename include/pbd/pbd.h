@@ -383,10 +383,9 @@ typedef struct pbd_launch_shape {
   uint32_t tile_bits;         /* neighbour-pass tiles of 2^tile_bits cells: 5 or 6 (0 = per particle) */
   uint32_t sort_items;        /* onesweep tile of 256 x sort_items keys: 4, 8, 16 (0 = by particle count) */
   uint32_t small_tile_max;    /* blocks of at most this many particles take one wave each: 0 .. 64
-                                 (32 and more: of up to 64); a block of more than 8 whose halo does
-                                 not fit a wave's tile takes a workgroup all the same.  Until a
-                                 shape is set, by particle count: 0 up to 2^16, 32 below 2^21,
-                                 else 64 */
+                                 (32 and more: of up to 64); a block whose halo does not fit a
+                                 wave's tile takes a workgroup all the same (up to 2^16 particles:
+                                 one of more than 8).  Until a shape is set, by particle count: 0 up to 2^16, 32 below 2^21, else 64 */
   uint32_t stride_grid;       /* workgroups of the capped tile grid (batches): a multiple of 32 */
   uint32_t list_skin_pct;     /* tile neighbour lists: skin in percent of the list radius, 0 .. 50
                                  (0: every lambda and omega pass rebuilds its lists) */

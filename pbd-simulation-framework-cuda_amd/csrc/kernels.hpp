@@ -71,7 +71,13 @@ struct TileList {
 };
 
 constexpr uint32_t kTileSmall = 64;           // particles of a small tile (one wave)
-constexpr uint32_t kTileSmallSure = 8;        // up to here small whatever its halo holds
+// Blocks of up to this many particles are small whatever their halo.  None, by the times: ms
+// for 200 steps of a dam break with blocks of up to 8 left small / none: 110K 91.2 / 86.8, 262K
+// 122.1 / 116.6, 512K 193.0 / 183.8, 1M 375.2 / 373.8; and 64K with a threshold of 64 set 85.0
+// / 80.1.  Up to 2^16 particles, where small tiles are only made for a shape that asks for
+// them, 8 stays all the same: those blocks have no lists, and the comparison of the reverse
+// mode's lists from the forward with built ones needs blocks without.
+__host__ __device__ inline uint32_t small_sure(uint32_t n) { return n <= (1u << 16) ? 8u : 0u; }
 constexpr uint32_t kTileCrowded = 1u << 31;   // a block that is large for its halo
 constexpr uint32_t kTileSplit = 1u << 30;     // a block that is two items for its halo
 // Blocks that are two items: a halo of more than 1528 particles; a particle is in at most 8 (1528 / 8 = 191).
@@ -133,8 +139,8 @@ inline uint32_t direct_grid(uint32_t ntiles, uint32_t n) {
 // particle count end[b] - (start[b] - 1) (small: at most small_max <= kTileSmall),
 // both ascending; count[0..1] = their lengths.  bcount holds
 // ceil(nflags / kTileCompactChunk) packed block counts.
-// A block of more than kTileSmallSure particles is small only if its halo fits a small
-// tile, and one whose halo exceeds a tile is two items.  bcount starts at zero.
+// A block of more than small_sure(n) particles is small only if its halo fits a small tile,
+// and one whose halo exceeds a tile is two items.  bcount starts at zero.
 hipError_t launch_tile_compact(hipStream_t st, int bits, const DevParams& P, const StepBuffers& B, uint32_t nflags,
                                uint32_t* start, const uint32_t* end, uint32_t small_max, uint32_t* bcount, uint32_t* large, uint32_t* small,
                                uint32_t* count);

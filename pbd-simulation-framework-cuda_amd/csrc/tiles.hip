@@ -369,7 +369,7 @@ __device__ __forceinline__ int tile_pick(const TileList& T, const TileItems& it,
 template <int BITS>
 struct TileCap;
 // The capacity decides how many workgroups a CU holds: with 1528 slots (and small tiles'
-// 272) a lambda pass has 26 KB and 6 of them, as many as its 73 to 79 VGPRs allow, an omega
+// 312) a lambda pass has 26 KB and 6 of them, as many as its 73 to 79 VGPRs allow, an omega
 // pass (a slot's global index beside it) 32 KB and 5, at 1920 slots 5 and 4.  us a step at
 // 1920 / 1352 slots, when it was lowered: 1M column 1060 / 964, 1M splash 1438 / 1285, 16M
 // column 14700 / 13650, 64 uneven scenes 7360 / 7110; at 1352 / 1528 / 1560: 1M column 912 /
@@ -382,7 +382,8 @@ struct TileCap;
 template <>
 struct TileCap<5> {
   static constexpr int value = 1528;  // 2x4x4 blocks: 144 halo cells, ~1150 particles at rest density
-  static constexpr int small = 272;   // a small tile's halo (one wave, a quarter of the LDS)
+  // a small tile's halo (one wave, a quarter of the LDS; 64 uneven scenes 6390 us at 272, 6350)
+  static constexpr int small = 312;
   static constexpr int adjoint = 1920;  // of the reverse passes' list builders
 };
 template <>
@@ -408,9 +409,11 @@ __device__ __forceinline__ uint32_t tile_class(uint32_t b, uint32_t nflags, cons
 // Marks the occupied blocks by their halos and counts the items of every 4096 flags: a
 // block of at most small_max particles whose halo is more than a small tile holds is
 // large (kTileCrowded; as a small one every pass took it particle by particle from global
-// memory: 1M splash with small tiles of up to 64, 1862 us, with the marks 1438), and a
-// large one whose halo is more than a tile holds is two items (kTileSplit).  Blocks of at
-// most kTileSmallSure particles stay small.  A wave takes F flags, a lane each, and counts
+// memory: 1M splash with small tiles of up to 64, 1862 us, with the marks 1438; also one of a
+// few particles beside a crowd, whose 27 cells of each one lane would walk: with blocks of up
+// to 8 left small, steps 11 to 20 of a 262K dam break took 663 us each, with none 521; see
+// small_sure), and a
+// large one whose halo is more than a tile holds is two items (kTileSplit).  A wave takes F flags, a lane each, and counts
 // the halos of those that need it four at a time, kHaloLanes lanes a block, all of a
 // lane's cells in flight at once.
 constexpr uint32_t kHaloLanes = 16;
@@ -435,7 +438,7 @@ __global__ __launch_bounds__(256) void k_tile_classify(DevParams P, uint32_t nfl
   const uint32_t s = lane < F && base + lane < nflags ? start[base + lane] : 0u;
   const uint32_t own = s ? end[base + lane] - tile_begin(s) : 0u;
   uint32_t mark = 0u;
-  for (uint64_t todo = __ballot(own > min(kTileSmallSure, small_max)); todo;) {
+  for (uint64_t todo = __ballot(own > min(small_sure(P.n), small_max)); todo;) {
     // the next four blocks, one for each group of lanes
     uint32_t k = 64u;
 #pragma unroll

@@ -1,6 +1,6 @@
 """Split blocks (halos of more than 1528 particles) beyond the plain step: with solids and
 friction against the oracle, and on the capped grid of boxes with more than 2^20 blocks
-against the direct one."""
+against the direct one; and the edges of whole, split and small tiles."""
 import numpy as np
 import pytest
 
@@ -102,13 +102,40 @@ def test_gpu_layered_blocks_stay_on_tiles(F, O, small):
     assert _match(F, O, p, x, small, "layers") == 0
 
 
+
+# a small tile's 312 slots
+@pytest.mark.parametrize("own,halo", [(12, 312), (12, 313), (64, 312), (64, 313), (9, 1400)])
+def test_gpu_small_blocks_at_their_capacity_stay_on_tiles(F, O, own, halo):
+    p, x = _block_scene(F, 5, own, halo)
+    p.solver_iterations = 2
+    p.active_apply_delta_positions = 0
+    assert _match(F, O, p, x, 64, f"own {own}, halo {halo}") == 0
+
+
+def test_gpu_few_particles_beside_a_crowd_stay_on_tiles(F, O):
+    """A column of 9 particles a cell with spray beside it, one or two particles in a block
+    whose halo holds 300 and more: no particle is walked from global memory."""
+    p, _, _ = _scene(F, (32, 32, 32), (1,), 0.98)
+    c = np.indices((32, 32, 32)).reshape(3, -1).T
+    rng = np.random.default_rng(12)
+    spray = (c[:, 0] >= 16) & (rng.uniform(size=len(c)) < 0.04)
+    c = np.repeat(c, np.where(c[:, 0] < 16, 9, spray.astype(int)), 0)
+    x = np.ones((len(c), 4), np.float32)
+    x[:, :3] = (c + rng.uniform(0.02, 0.98, c.shape)) * 0.1
+    assert len(x) > 1 << 16  # where small tiles are on by default
+    p.solver_iterations = 2
+    p.active_apply_delta_positions = 0
+    assert _match(F, O, p, x, None, "spray") == 0
+
+
 def _match(F, O, p, x, small, label):
     """One step against the oracle by the parity tests' bounds; the particles without a list
     for their block's halo."""
     print(f"tile capacity: {label}, n {len(x)}, small {small}", flush=True)
     ctx = F.Context(p, len(x))
     ctx.add_particles(x)
-    ctx.set_launch_shape(small_tile_max=small)
+    if small is not None:
+        ctx.set_launch_shape(small_tile_max=small)
     ctx.compute()
     got = {k: ctx.download(k) for k in ("cell_ids", "particle_ids", "neighbour_counters", "densities", "lambdas",
                                         "delta_positions")}
